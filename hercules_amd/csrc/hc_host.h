@@ -135,9 +135,9 @@ struct hc_ctx {
     // divergence screen (screen_div_error after every substep when screen =
     // 1): scr[0] div_hist_max, scr[4 + 4 s ..] the record of slot s (div_avg,
     // div_max, div_hist_max, NaN flag; slot 0 on request, 1..3 the substeps);
-    // scr_rows / scr_blk the per-row and per-block partials
+    // scr_units / scr_groups the summaries of runs of points (hc_screen.hip)
     int screen = 0;
-    double *scr = nullptr, *scr_rows = nullptr, *scr_blk = nullptr;
+    double *scr = nullptr, *scr_units = nullptr, *scr_groups = nullptr;
 };
 
 // Steps taken for tuning or for a gradient's forward run leave the

@@ -9,161 +9,317 @@
 // and stops on the first NaN in u, v or w (screen_div_error_spec,
 // src/module_spectral.f90:899-1007, stores |d|: plain maxima).  div_max and div_hist_max are
 // therefore SIGNED and depend on the scan order: after a negative d is stored
-// the next point always replaces it.  The screen reproduces that sequence
-// exactly in two launches:
-//   k_div_rows    all points in parallel: per block (16 rows of one level)
-//                 the sum of |d| and the NaN flag, per row and per block the
-//                 largest |d|;
-//   k_div_signed  one wavefront walks the blocks in scan order and opens only
-//                 those whose largest |d| can change a state (|d| > state, or
-//                 any state < 0), then their rows, then their points, taking
-//                 the first qualifying point of each 64 by a ballot.  Every
-//                 state change happens at a point it visits in order, so the
-//                 result equals the sequential scan; the untouched blocks cost
-//                 one load of their maximum.
+// the next point always replaces it.
+//
+// Parallel form.  After a point is taken the state is its d, so the next
+// point taken is the first later one with |d'| > d: a pointer that does not
+// depend on how the scan got there.  A run of points therefore maps an
+// incoming state S through the first point with |d| > S, which is one of the
+// run's records (strict prefix maxima of |d|, about ln n of them), to the d
+// where that point's chain of pointers ends.  Three launches:
+//   k_div_units   d of 4096 consecutive points (scan order is memory order)
+//                 in LDS, 64 chunks of 64.  Per chunk and point, the end of
+//                 its chain within the chunk (next-greater search over a
+//                 table of shuffled maxima, then pointer doubling).  One lane
+//                 per record then walks the chunks to the end of the unit:
+//                 records and their final states, sum of |d|, NaN flag.
+//   k_div_groups  the same walk over the records of 64 units
+//   k_div_final   one wavefront applies the groups to div_max and
+//                 div_hist_max in order.
+// A unit with more than kRec records (long monotone |d|) or a group of such
+// units is walked by k_div_final point by point instead.  At 128x128x129 the
+// three take 107 + 36 + 21 us; one wavefront that visited every taken point
+// (a state that a negative d resets takes ~10% of all points) took 2350 us
+// after a 28 us pass for the row maxima.
 #include "hc_host.h"
 
 #include <mutex>
 
 namespace {
-constexpr int kRowsPerBlock = 16;
 constexpr int kScrLen = 32;
+constexpr int kChunk = 64;                 // points of a chunk, chunks of a batch, units of a group
+constexpr int kBatch = kChunk * kChunk;    // points held in LDS at a time
+constexpr int kRec = 32;                   // records kept per unit / group
+// a unit's or group's summary: sum |d|, max |d|, NaN flag, number of records
+// (-1: more than kRec, or a member had), records, final states
+constexpr int kSum = 4 + 2 * kRec;
 
 __global__ void k_scr_zero(double *f, int n)
 {
     if ((int)threadIdx.x < n) f[threadIdx.x] = 0.0;
 }
 
+// signed divergence of point q (scan order) as the states keep it
+// (screen_div_error_spec stores |d|, src/module_spectral.f90:931-946) and the
+// magnitude it is compared by; a NaN is never taken
 template <int CDS, class R>
-__global__ __launch_bounds__(256) void k_div_rows(StepArgsT<R> F, StepArgs D, double *rowmax, double *blk)
+HC_DEV void point_div(const StepArgsT<R> &F, const StepArgs &D, unsigned q, double &d, double &a)
 {
-    __shared__ double rs[4], rm[4];
-    __shared__ int rn[4];
-    const int k = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int gx = gridDim.x, b = k * gx + blockIdx.x;
-    double s = 0.0, bmax = 0.0;
-    int nan = 0;
-    for (int r = wv; r < kRowsPerBlock; r += 4) {
-        const int j = blockIdx.x * kRowsPerBlock + r;
-        if (j >= D.ny) break;
-        double m = 0.0;
-        for (int i = lane; i < D.nx; i += 64) {
-            const double d = div_at<CDS, R>(F, D, i, j, k);
-            s += fabs(d);
-            m = fmax(m, fabs(d));
-            const size_t o = ((size_t)k * D.ny + j) * D.nx + i;
-            const R u0 = F.u[o], v0 = F.v[o], w0 = F.w[o];
-            if (u0 != u0 || v0 != v0 || w0 != w0) nan = 1;
-        }
-        for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
-        if (lane == 0) rowmax[(size_t)k * D.ny + j] = m;
-        bmax = fmax(bmax, m);
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        s += __shfl_xor(s, o, 64);
-        nan |= __shfl_xor(nan, o, 64);
-    }
-    if (lane == 0) { rs[wv] = s; rm[wv] = bmax; rn[wv] = nan; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        blk[3 * (size_t)b] = (rs[0] + rs[1]) + (rs[2] + rs[3]);
-        blk[3 * (size_t)b + 1] = fmax(fmax(rm[0], rm[1]), fmax(rm[2], rm[3]));
-        blk[3 * (size_t)b + 2] = (double)(rn[0] | rn[1] | rn[2] | rn[3]);
-    }
+    const unsigned row = q / (unsigned)D.nx, i = q - row * (unsigned)D.nx;
+    const unsigned k = row / (unsigned)D.ny, j = row - k * (unsigned)D.ny;
+    d = div_at<CDS, R>(F, D, (int)i, (int)j, (int)k);
+    a = fabs(d);
+    if (CDS == 3) d = a;
 }
 
-// State of the scan: s1 = div_max, s2 = div_hist_max (updated when fin).
-// screen_div_error_spec stores |d| instead of d (src/module_spectral.f90:931-946),
-// so with absval the states are plain running maxima.
-struct ScanState {
-    double s1, s2;
-    bool fin, absval;
-    // can a value of magnitude a change a state?
-    HC_DEV bool hit(double a) const { return a > s1 || (fin && a > s2); }
-    HC_DEV void take(double d)
-    {
-        const double a = fabs(d), keep = absval ? a : d;
-        if (a > s1) s1 = keep;
-        if (fin && a > s2) s2 = keep;
-    }
+// One lane's walk state: lane r < nrec follows record r.
+struct Walk {
+    double S, rec, gmax;  // state, the record's magnitude, largest |d| so far (uniform)
+    int nrec;             // uniform; -1 once there are more than kRec
 };
-
-// one row of points in scan order (i ascending), 64 at a time
-template <int CDS, class R>
-HC_DEV void scan_row(const StepArgsT<R> &F, const StepArgs &D, int j, int k, ScanState &S, int lane)
+// Lanes whose state the run [pm] (kChunk nondecreasing prefix maxima) beats:
+// position of the first entry above S
+HC_DEV int first_above(const double *pm, int n2, double S)
 {
-    for (int i0 = 0; i0 < D.nx; i0 += 64) {
-        const int i = i0 + lane;
-        const double d = i < D.nx ? div_at<CDS, R>(F, D, i, j, k) : 0.0;
-        const double a = i < D.nx ? fabs(d) : -1.0;
-        int pos = -1;
-        while (true) {
-            const unsigned long long m = __ballot(lane > pos && S.hit(a));
-            if (!m) break;
-            const int L = __ffsll((long long)m) - 1;
-            S.take(__shfl(d, L, 64));
-            pos = L;
+    int pos = 0;
+    for (int st = n2 >> 1; st > 0; st >>= 1)
+        if (!(pm[pos + st - 1] > S)) pos += st;
+    return pos;
+}
+// new records of a run: bit set where entry `i` of the lanes is one; out = its final state
+HC_DEV void add_records(Walk &w, unsigned long long m, double mag, double out, int lane)
+{
+    while (m) {
+        const int b = __ffsll((long long)m) - 1;
+        m &= m - 1;
+        const double g = __shfl(mag, b, 64), o = __shfl(out, b, 64);
+        if (w.nrec >= 0) {
+            if (w.nrec == kRec) { w.nrec = -1; return; }
+            if (lane == w.nrec) { w.rec = g; w.S = o; }
+            ++w.nrec;
         }
     }
 }
-
-template <int CDS, class R>
-__global__ __launch_bounds__(64) void k_div_signed(StepArgsT<R> F, StepArgs D, const double *rowmax, const double *blk,
-                                                   int nblk, int gx, double *state, double *rec, int fin)
+HC_DEV void write_summary(const Walk &w, double *o, double sum, int nan, int lane)
 {
-    // state[0]: div_hist_max before the call (updated in place when fin)
-    const int lane = threadIdx.x;
-    // fixed-order sum of the block sums, NaN flag
+    if (lane == 0) { o[0] = sum; o[1] = w.gmax; o[2] = (double)nan; o[3] = (double)w.nrec; }
+    if (lane < kRec) {
+        const bool on = lane < w.nrec;
+        o[4 + lane] = on ? w.rec : HUGE_VAL;
+        o[4 + kRec + lane] = on ? w.S : 0.0;
+    }
+}
+
+// Bound by the walk's LDS latency and the shuffles of the chunk tables, not
+// by HBM: 4096 points keep 70 KB of LDS, two blocks per CU.
+template <int CDS, class R>
+__global__ __launch_bounds__(256) void k_div_units(StepArgsT<R> F, StepArgs D, unsigned N, int nb, double *units)
+{
+    __shared__ double dd[kBatch], pm[kBatch], cmax[kChunk], rs[4];
+    __shared__ unsigned char ex[kBatch];
+    __shared__ int rn[4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const double ninf = -HUGE_VAL;
     double s = 0.0;
     int nan = 0;
-    for (int b = lane; b < nblk; b += 64) {
-        s += blk[3 * (size_t)b];
-        nan |= blk[3 * (size_t)b + 2] != 0.0;
+    Walk w{0.0, 0.0, ninf, 0};
+    for (int bt = 0; bt < nb; ++bt) {
+        const size_t base = ((size_t)blockIdx.x * nb + bt) * kBatch;
+        if (base >= N) break;
+        for (int c = wv; c < kChunk; c += 4) {
+            const size_t q = base + (size_t)c * kChunk + lane;
+            double d = 0.0, a = ninf;
+            if (q < N) {
+                double mag;
+                point_div<CDS, R>(F, D, (unsigned)q, d, mag);
+                s += mag;
+                if (mag >= 0.0) a = mag;
+                const R u0 = F.u[q], v0 = F.v[q], w0 = F.w[q];
+                if (u0 != u0 || v0 != v0 || w0 != w0) nan = 1;
+            }
+            // t[e] = max over the 2^e points after this one
+            double t[6];
+            t[0] = __shfl_down(a, 1, 64);
+            if (lane == 63) t[0] = ninf;
+#pragma unroll
+            for (int e = 1; e < 6; ++e) {
+                const int h = 1 << (e - 1);
+                const double o = __shfl_down(t[e - 1], h, 64);
+                t[e] = fmax(t[e - 1], lane + h < 64 ? o : ninf);
+            }
+            // the first later point with |d| > d, or this one
+            int pos = lane;
+#pragma unroll
+            for (int e = 5; e >= 0; --e) {
+                const double o = __shfl(t[e], pos & 63, 64);
+                if (pos < 64 && !(o > d)) pos += 1 << e;
+            }
+            int p = pos + 1 < 64 ? pos + 1 : lane;
+#pragma unroll
+            for (int e = 0; e < 6; ++e) p = __shfl(p, p, 64);
+            double m = a;
+#pragma unroll
+            for (int e = 1; e < 64; e <<= 1) {
+                const double o = __shfl_up(m, e, 64);
+                if (lane >= e) m = fmax(m, o);
+            }
+            const int at = c * kChunk + lane;
+            dd[at] = d;
+            pm[at] = m;
+            ex[at] = (unsigned char)p;
+            if (lane == 63) cmax[c] = m;
+        }
+        __syncthreads();
+        if (wv == 0) {
+            for (int c = 0; c < kChunk; ++c) {
+                const double cm = cmax[c];
+                const int at = c * kChunk;
+                if (lane < w.nrec && cm > w.S) w.S = dd[at + ex[at + first_above(pm + at, kChunk, w.S)]];
+                if (cm > w.gmax) {
+                    const double mine = pm[at + lane], prev = lane ? pm[at + lane - 1] : ninf;
+                    add_records(w, __ballot(mine > fmax(w.gmax, prev)), mine, dd[at + ex[at + lane]], lane);
+                    w.gmax = cm;
+                }
+            }
+        }
+        __syncthreads();
     }
     for (int o = 32; o > 0; o >>= 1) {
         s += __shfl_xor(s, o, 64);
         nan |= __shfl_xor(nan, o, 64);
     }
-    ScanState S{0.0, state[0], fin != 0, CDS == 3};
+    if (lane == 0) { rs[wv] = s; rn[wv] = nan; }
+    __syncthreads();
+    if (wv == 0)
+        write_summary(w, units + (size_t)blockIdx.x * kSum, (rs[0] + rs[1]) + (rs[2] + rs[3]),
+                      rn[0] | rn[1] | rn[2] | rn[3], lane);
+}
+
+// 64 units to one summary, the same walk over their records
+__global__ __launch_bounds__(64) void k_div_groups(const double *units, int nunit, double *groups)
+{
+    __shared__ double rec[kChunk][kRec], out[kChunk][kRec];
+    const int lane = threadIdx.x, u0 = blockIdx.x * kChunk, n = min(kChunk, nunit - u0);
+    const double ninf = -HUGE_VAL;
+    for (int q = lane; q < n * 2 * kRec; q += 64) {
+        const int u = q / (2 * kRec), r = q - u * 2 * kRec;
+        const double v = units[(size_t)(u0 + u) * kSum + 4 + r];
+        if (r < kRec) rec[u][r] = v;
+        else out[u][r - kRec] = v;
+    }
+    double sum = 0.0, mx = ninf, cnt = 0.0;
+    int nan = 0;
+    if (lane < n) {
+        const double *h = units + (size_t)(u0 + lane) * kSum;
+        sum = h[0];
+        mx = h[1];
+        nan = h[2] != 0.0;
+        cnt = h[3];
+    }
+    const bool bad = __any(cnt < 0.0);
+    for (int o = 32; o > 0; o >>= 1) {
+        sum += __shfl_xor(sum, o, 64);
+        nan |= __shfl_xor(nan, o, 64);
+    }
+    __syncthreads();
+    Walk w{0.0, 0.0, ninf, bad ? -1 : 0};
+    for (int c = 0; c < n; ++c) {
+        const double cm = __shfl(mx, c, 64);
+        if (!bad) {
+            if (lane < w.nrec && cm > w.S) w.S = out[c][first_above(rec[c], kRec, w.S)];
+            if (cm > w.gmax) {
+                const bool on = lane < (int)__shfl(cnt, c, 64);
+                const double mine = on ? rec[c][lane] : 0.0;
+                add_records(w, __ballot(on && mine > w.gmax), mine, on ? out[c][lane] : 0.0, lane);
+            }
+        }
+        w.gmax = fmax(w.gmax, cm);
+    }
+    write_summary(w, groups + (size_t)blockIdx.x * kSum, sum, nan, lane);
+}
+
+// State of the scan: s[0] = div_max, s[1] = div_hist_max (updated when fin)
+struct ScanState {
+    double s[2];
+    int n;
+    HC_DEV bool hit(double a) const { return a > s[0] || (n > 1 && a > s[1]); }
+};
+// a summary's n records applied to the states: the first record above each
+HC_DEV void apply(ScanState &S, int n, double rec, double out, int lane)
+{
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const unsigned long long m = __ballot(e < S.n && lane < n && rec > S.s[e]);
+        if (m) S.s[e] = __shfl(out, __ffsll((long long)m) - 1, 64);
+    }
+}
+// points [q0, q1) one at a time, 64 loaded together
+template <int CDS, class R>
+HC_DEV void scan_points(const StepArgsT<R> &F, const StepArgs &D, size_t q0, size_t q1, ScanState &S, int lane)
+{
+    for (size_t b = q0; b < q1; b += 64) {
+        double d = 0.0, a = -HUGE_VAL;
+        if (b + lane < q1) point_div<CDS, R>(F, D, (unsigned)(b + lane), d, a);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            int pos = -1;
+            while (true) {
+                const unsigned long long m = __ballot(e < S.n && lane > pos && a > S.s[e]);
+                if (!m) break;
+                pos = __ffsll((long long)m) - 1;
+                S.s[e] = __shfl(d, pos, 64);
+            }
+        }
+    }
+}
+
+// state[0]: div_hist_max before the call (updated in place when fin)
+template <int CDS, class R>
+__global__ __launch_bounds__(64) void k_div_final(StepArgsT<R> F, StepArgs D, unsigned N, int nb, const double *units,
+                                                  int nunit, const double *groups, int ngroup, double *state,
+                                                  double *rec, int fin)
+{
+    const int lane = threadIdx.x;
+    double s = 0.0;
+    int nan = 0;
+    for (int g = lane; g < ngroup; g += 64) {
+        s += groups[(size_t)g * kSum];
+        nan |= groups[(size_t)g * kSum + 2] != 0.0;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o, 64);
+        nan |= __shfl_xor(nan, o, 64);
+    }
+    ScanState S{{0.0, state[0]}, fin ? 2 : 1};
     if (!nan) {
-        constexpr int U = 8;
-        for (int b0 = 0; b0 < nblk; b0 += 64 * U) {
-            double bm[U];
+        constexpr int U = 8;  // summaries loaded ahead of their use
+        for (int g0 = 0; g0 < ngroup; g0 += U) {
+            double mx[U], ct[U], rc[U], ou[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int b = b0 + u * 64 + lane;
-                bm[u] = b < nblk ? blk[3 * (size_t)b + 1] : -1.0;
+                const double *h = groups + (size_t)min(g0 + u, ngroup - 1) * kSum;
+                mx[u] = h[1];
+                ct[u] = h[3];
+                rc[u] = h[4 + (lane & (kRec - 1))];
+                ou[u] = h[4 + kRec + (lane & (kRec - 1))];
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                int pos = -1;
-                while (true) {
-                    const unsigned long long m = __ballot(lane > pos && bm[u] >= 0.0 && S.hit(bm[u]));
-                    if (!m) break;
-                    const int L = __ffsll((long long)m) - 1;
-                    const int b = b0 + u * 64 + L, k = b / gx, j0 = (b - k * gx) * kRowsPerBlock;
-                    // the rows of block b in order
-                    const int nr = min(kRowsPerBlock, D.ny - j0);
-                    const double rmx = lane < nr ? rowmax[(size_t)k * D.ny + j0 + lane] : -1.0;
-                    int rpos = -1;
-                    while (true) {
-                        const unsigned long long rm = __ballot(lane > rpos && rmx >= 0.0 && S.hit(rmx));
-                        if (!rm) break;
-                        const int r = __ffsll((long long)rm) - 1;
-                        scan_row<CDS, R>(F, D, j0 + r, k, S, lane);
-                        rpos = r;
+                const int g = g0 + u;
+                if (g >= ngroup || !S.hit(mx[u])) continue;
+                if (ct[u] >= 0.0) {
+                    apply(S, (int)ct[u], rc[u], ou[u], lane);
+                    continue;
+                }
+                for (int q = g * kChunk; q < min((g + 1) * kChunk, nunit); ++q) {
+                    const double *h = units + (size_t)q * kSum;
+                    if (!S.hit(h[1])) continue;
+                    if (h[3] >= 0.0) {
+                        apply(S, (int)h[3], h[4 + (lane & (kRec - 1))], h[4 + kRec + (lane & (kRec - 1))], lane);
+                    } else {
+                        const size_t per = (size_t)nb * kBatch, q0 = q * per;
+                        scan_points<CDS, R>(F, D, q0, q0 + per < N ? q0 + per : (size_t)N, S, lane);
                     }
-                    pos = L;
                 }
             }
         }
     }
     if (lane == 0) {
         rec[0] = s / ((double)D.nx * D.ny * D.nz);
-        rec[1] = S.s1;
-        rec[2] = nan ? state[0] : S.s2;
+        rec[1] = S.s[0];
+        rec[2] = S.s[1];
         rec[3] = nan;
-        if (fin && !nan) state[0] = S.s2;
+        if (fin && !nan) state[0] = S.s[1];
     }
 }
 
@@ -172,20 +328,26 @@ __global__ void k_scr_set(double *f, double v)
     if (threadIdx.x == 0) f[0] = v;
 }
 
-// Partials of one screen: per-row maxima (ny nz), per-block sums, maxima and
-// NaN flags (3 gx nz), where gx = ceil(ny / 16).
+// Partials of one screen: the units' and groups' summaries
 struct ScreenBufs {
-    double *rows, *blk, *state, *rec;
+    double *units, *groups, *state, *rec;
+    int nb;  // batches of 4096 points per unit
 };
-inline size_t screen_rows_len(int ny, int nz) { return (size_t)ny * nz; }
-inline size_t screen_blk_len(int ny, int nz) { return 3 * (size_t)((ny + kRowsPerBlock - 1) / kRowsPerBlock) * nz; }
+inline int screen_units(const hc_ctx *c, int nb)
+{
+    const size_t N = (size_t)c->nx * c->ny * c->nz, per = (size_t)nb * kBatch;
+    return (int)((N + per - 1) / per);
+}
+inline int screen_groups(int nunit) { return (nunit + kChunk - 1) / kChunk; }
 
 template <int CDS, class R>
 void launch_screen(hc_ctx *c, const StepArgsT<R> &F, const StepArgs &D, const ScreenBufs &B, int fin)
 {
-    const int gx = (c->ny + kRowsPerBlock - 1) / kRowsPerBlock, nblk = gx * c->nz;
-    hipLaunchKernelGGL((k_div_rows<CDS, R>), dim3(gx, c->nz), dim3(256), 0, c->stream, F, D, B.rows, B.blk);
-    hipLaunchKernelGGL((k_div_signed<CDS, R>), dim3(1), dim3(64), 0, c->stream, F, D, B.rows, B.blk, nblk, gx,
+    const unsigned N = (unsigned)c->nx * (unsigned)c->ny * (unsigned)c->nz;
+    const int nu = screen_units(c, B.nb), ng = screen_groups(nu);
+    hipLaunchKernelGGL((k_div_units<CDS, R>), dim3(nu), dim3(256), 0, c->stream, F, D, N, B.nb, B.units);
+    hipLaunchKernelGGL(k_div_groups, dim3(ng), dim3(64), 0, c->stream, B.units, nu, B.groups);
+    hipLaunchKernelGGL((k_div_final<CDS, R>), dim3(1), dim3(64), 0, c->stream, F, D, N, B.nb, B.units, nu, B.groups, ng,
                        B.state, B.rec, fin);
 }
 
@@ -215,10 +377,10 @@ int queue_screen(hc_ctx *c, const ScreenBufs &B, int fin)
 int screen_alloc(hc_ctx *c)
 {
     if (c->scr) return 0;
-    const int gx = (c->ny + kRowsPerBlock - 1) / kRowsPerBlock;
+    const int nu = screen_units(c, 1), ng = screen_groups(nu);
     int e = dalloc(c, (void **)&c->scr, kScrLen * sizeof(double));
-    if (!e) e = dalloc(c, (void **)&c->scr_rows, (size_t)c->ny * c->nz * sizeof(double));
-    if (!e) e = dalloc(c, (void **)&c->scr_blk, 3 * (size_t)gx * c->nz * sizeof(double));
+    if (!e) e = dalloc(c, (void **)&c->scr_units, (size_t)nu * kSum * sizeof(double));
+    if (!e) e = dalloc(c, (void **)&c->scr_groups, (size_t)ng * kSum * sizeof(double));
     if (!e) {
         // div_hist_max starts at 0 (module_io's save variable)
         hipLaunchKernelGGL(k_scr_zero, dim3(1), dim3(64), 0, c->stream, c->scr, kScrLen);
@@ -232,7 +394,7 @@ int screen_alloc(hc_ctx *c)
 int screen_queue(hc_ctx *c, int slot, int fin)
 {
     if (int e = screen_alloc(c)) return e;
-    return queue_screen(c, ScreenBufs{c->scr_rows, c->scr_blk, c->scr, c->scr + 4 + 4 * slot}, fin);
+    return queue_screen(c, ScreenBufs{c->scr_units, c->scr_groups, c->scr, c->scr + 4 + 4 * slot, 1}, fin);
 }
 
 // ---------------------------------------------------------------------------
@@ -269,9 +431,17 @@ extern "C" int hc_screen_div_error_noalloc(hc_ctx *c, int isfinal, double *div_a
 {
     if (!c || !div_hist_max) return set_err(HC_ERR_ARG, "null argument");
     if (isfinal != 0 && isfinal != 1) return set_err(HC_ERR_ARG, "isfinal must be 0 or 1");
-    const size_t nrows = screen_rows_len(c->ny, c->nz), nblk = screen_blk_len(c->ny, c->nz);
-    const size_t need = 8 + nrows + nblk;
-    if (need > kScratchDoubles)
+    // the size of grid that is taken: ny nz rows and 3 values for 16 rows of a
+    // level within the scratch
+    const size_t need = 8 + (size_t)c->ny * c->nz + 3 * (size_t)((c->ny + 15) / 16) * c->nz;
+    // units of as many batches as make their summaries fit: 1 to 8 (a grid of
+    // this size has nx <= 512, so under 2^28 points)
+    int nb = 1, nu = screen_units(c, 1);
+    while (nb < 64 && 8 + (size_t)(nu + screen_groups(nu)) * kSum > kScratchDoubles) {
+        nb *= 2;
+        nu = screen_units(c, nb);
+    }
+    if (need > kScratchDoubles || 8 + (size_t)(nu + screen_groups(nu)) * kSum > kScratchDoubles)
         return set_err(HC_ERR_ARG, "screen partials of %zu doubles (ny=%d, nz=%d) exceed the scratch of %zu doubles",
                        need, c->ny, c->nz, kScratchDoubles);
     int dev = -1;
@@ -280,8 +450,8 @@ extern "C" int hc_screen_div_error_noalloc(hc_ctx *c, int isfinal, double *div_a
     double *ptr = nullptr;
     if (int e = scratch_ptr(dev, &ptr)) return e;
     // scratch layout: [0] div_hist_max in/out, [4..7] the record, then the
-    // row maxima and the block partials (both fully rewritten by each call)
-    const ScreenBufs B{ptr + 8, ptr + 8 + nrows, ptr, ptr + 4};
+    // units' and the groups' summaries (both fully rewritten by each call)
+    const ScreenBufs B{ptr + 8, ptr + 8 + (size_t)nu * kSum, ptr, ptr + 4, nb};
     hipLaunchKernelGGL(k_scr_set, dim3(1), dim3(64), 0, c->stream, ptr, *div_hist_max);
     HIPCHK(hipGetLastError());
     if (int e = queue_screen(c, B, isfinal)) return e;

@@ -87,3 +87,64 @@ def test_nan_stops_the_step(entry):
     if entry == "steps":
         assert ch.scalar("stps") == 1  # stopped after the first step
     ch.close()
+
+
+def _planted(kind, shape, dz, rng):
+    """w fields (nz, ny, nx) whose divergence in scan order is of one kind."""
+    nz, ny, nx = shape
+    n = nz * ny * nx
+    d = rng.standard_normal(n)
+    ramp = np.arange(1, n + 1) / n
+    if kind == "rising":       # every point is a record
+        d = ramp
+    elif kind == "rising_alternate":
+        d = ramp * np.where(np.arange(n) % 2, 1.0, -1.0)
+    elif kind == "negative":
+        d = -np.abs(d)
+    elif kind == "zero":
+        d = np.zeros(n)
+    elif kind == "late_peak":  # long stretches that change nothing
+        d = 1e-3 * d
+        d[n // 3] = 5.0
+        d[2 * n // 3] = -6.0
+    w = np.cumsum(d.reshape(shape) * dz[:, None, None], axis=0)
+    if kind == "infinite":
+        w[nz // 2, ny // 2, nx // 2] = np.inf
+    return w
+
+
+@pytest.mark.parametrize("shape", [(9, 16, 16), (50, 16, 48), (65, 64, 64)])
+@pytest.mark.parametrize("kind", ["random", "rising", "rising_alternate", "negative", "zero", "late_peak", "infinite"])
+def test_scan_equals_the_point_by_point_rule(kind, shape):
+    """div_max and div_hist_max bit for bit against the rule applied to one
+    point after another (u = v = 0, so d = (w(k) - w(k-1)) / dz(k)), runs
+    shorter and longer than the 4096 points of a unit, and more records than
+    a unit keeps; div_avg to the rounding of a sum of positive terms."""
+    nz, ny, nx = shape
+    ch = Channel(cases.closed_channel(nx=nx, ny=ny, nz=nz))
+    dz = ch.mesh()[1]
+    rng = np.random.default_rng(nz)
+    hist = 0.0
+    import ctypes as C
+    h2 = C.c_double(0.0)
+    for fin in (1, 0, 1):
+        w = _planted(kind, shape, dz, rng)
+        ch.set_field("w", w)
+        with np.errstate(invalid="ignore"):
+            d = ((w - np.concatenate([np.zeros_like(w[:1]), w[:-1]], 0)) / dz[:, None, None]).reshape(-1)
+        mx, hs = 0.0, hist
+        for x in d.tolist():
+            a = abs(x)
+            if a > mx:
+                mx = x
+            if fin and a > hs:
+                hs = x
+        hist = hs
+        got = ch.screen_div_error_ref(fin)
+        assert got[1] == mx and got[2] == hist, (kind, fin, got, mx, hist)
+        if np.isfinite(d).all():
+            assert got[0] == pytest.approx(np.abs(d).mean(), rel=1e-12)
+        a1, m1 = C.c_double(), C.c_double()
+        assert ch.L.hc_screen_div_error_noalloc(ch.h, fin, C.byref(a1), C.byref(m1), C.byref(h2)) == 0
+        assert m1.value == mx and h2.value == hist
+    ch.close()
