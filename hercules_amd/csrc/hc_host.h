@@ -69,7 +69,7 @@ struct hc_ctx {
         int ytile = 0;      // y transform columns per block (0: 8 for FP64, 16 for FP32)
         int c2r_pts = 1024; // inverse-x points per field per block
         int col_remap = 0;  // XCD-contiguous column block order
-        int rhs_xt = 0;     // FD momentum right-hand side: 0 whole rows with the x R2C fused, 1-4 x-y tiles
+        int rhs_xt = 0;     // FD momentum right-hand side: 0 chosen by size (march_shape), 1-4 marching x-y tiles
                             // (32x8, 64x8, 32x16, 64x4) and a separate in-place R2C
     } tune;
     int lo_l = 0, lo_m = 0;
@@ -186,7 +186,7 @@ inline bool fft_len_ok(int n)
     return n == 16 || n == 32 || n == 48 || n == 64 || n == 96 || n == 128 || n == 192 || n == 256 || n == 384 ||
            n == 512;
 }
-// rows of a right-hand-side tile for nx (rhs2_ty for nx <= 256, rhs_ty above):
+// rows of a right-hand-side tile for nx (rhs2_ty for nx <= 256):
 // ny must be a multiple of it
 inline int rhs_tile_rows(int nx)
 {

@@ -1,77 +1,11 @@
 // Momentum right-hand side of the FD substep (get_momentum_cnvdiff,
 // src/module_cnvdiff.f90:35-374) fused with the x-direction R2C of qu, qv,
-// qw: the two-phase LDS tile (nx <= 256), the staged-row kernel (nx = 512),
-// the global-memory kernel of damped substeps and of the 6th-order z
-// operators, and the Rayleigh damping means.
+// qw: marching tiles (hc_march.h), whole rows fused with the x transform
+// (short rows and FP32), the sponge's tiles and edge points, the
+// global-memory kernel of the 6th-order z operators, and the Rayleigh damping
+// means.
 #include "hc_host.h"
-
-// Momentum RHS + x R2C of qu,qv,qw.  Block: full rows j0..j0+TY-1 of level
-// k, one point per thread; every row the stencils reach is staged in LDS
-// once (coalesced), then the same LDS holds the q rows for the FFT.
-template <int NX>
-constexpr int rhs_ty()
-{
-    return NX == 16 ? 16 : NX == 32 ? 32 : NX == 64 ? 16 : NX == 128 ? 8 : NX == 192 ? 4 : NX == 256 ? 4 : 1;
-}
-
-template <int NX>
-constexpr int rhs_threads() { return NX * rhs_ty<NX>() <= 512 ? NX * rhs_ty<NX>() : NX * rhs_ty<NX>() / 2; }
-
-template <int CDS, int NX, class R>
-__global__ __launch_bounds__(rhs_threads<NX>()) void k_rhs_mom(StepArgsT<R> A)
-{
-    using C = cplx<R>;
-    constexpr int TY = rhs_ty<NX>();
-    constexpr int T = rhs_threads<NX>(), PP = NX * TY / T, NL = NX / 2;
-    using Tl = RhsTile<NX, TY>;
-    static_assert(Tl::NROWS * NX >= 3 * TY * NX, "FFT rows must fit in the staging area");
-    __shared__ __align__(16) R sm[Tl::NROWS * NX];
-    const int tid = threadIdx.x;
-    const int nty = A.ny / TY;
-    const int logical = xcd_remap(blockIdx.x, nty * A.nlev);
-    const int jt = logical % nty, k = A.klo + logical / nty, j0 = jt * TY;
-    for (int q = tid; q < Tl::NROWS * NX; q += T) {
-        int r = q / NX, i = q - r * NX;
-        sm[q] = rhs_stage_value<NX, TY>(A, r, i, j0, k);
-    }
-    const R dpx = A.dp_opt == 2 ? R(A.scal[0]) : A.dpx;
-    PointVals<R> pv[PP];
-#pragma unroll
-    for (int pp = 0; pp < PP; ++pp) {
-        const int pt = tid + pp * T;
-        pv[pp].load(A, pt % NX, j0 + pt / NX, k);
-    }
-    __syncthreads();
-    R qs[PP][3];
-#pragma unroll
-    for (int pp = 0; pp < PP; ++pp) {
-        const int pt = tid + pp * T, i = pt % NX, jj = pt / NX, j = j0 + jj;
-        Ld<NX, TY, R> q(A, sm, i, jj, j, k, pv[pp]);
-        R f, g, h;
-        momentum_point<CDS>(q, dpx, f, g, h, qs[pp][0], qs[pp][1], qs[pp][2]);
-        const size_t c = ((size_t)k * A.ny + j) * NX + i;
-        A.ff[c] = f;
-        A.gg[c] = g;
-        A.hh[c] = h;
-    }
-    __syncthreads();  // staging no longer read: reuse it for the q rows
-#pragma unroll
-    for (int pp = 0; pp < PP; ++pp) {
-        const int pt = tid + pp * T, i = pt % NX, jj = pt / NX;
-        sm[(0 * TY + jj) * NX + i] = qs[pp][0];
-        sm[(1 * TY + jj) * NX + i] = qs[pp][1];
-        sm[(2 * TY + jj) * NX + i] = qs[pp][2];
-    }
-    __syncthreads();
-    C *sq_ = reinterpret_cast<C *>(sm);
-    lds_fft<NL, 3 * TY, NL, 1, T, -1>(sq_, A.tw_nl, tid);
-    C *outs[3] = {A.s0, A.s1, A.s2};
-    for (int p = tid; p < 3 * TY * NL; p += T) {
-        int row = p / NL, l = p - row * NL, fi = row / TY, r = row - fi * TY;
-        outs[fi][((size_t)k * A.ny + j0 + r) * NL + l] = r2c_post<NL>(sq_ + row * NL, l, A.tw_nx, A.norm);
-    }
-}
-
+#include "hc_march.h"
 
 template <int CDS, int NX, class R>
 __global__ __launch_bounds__(rhs2_threads<NX>(), (rhs2_waves<NX, R>())) void k_rhs_mom2(StepArgsT<R> A)
@@ -196,25 +130,22 @@ __global__ __launch_bounds__(rhs2_threads<NX>(), (rhs2_waves<NX, R>())) void k_r
     }
 }
 
-// Momentum right-hand side on a TX x TY tile of level k (x tiles fastest,
-// then y tiles, then levels, in XCD-contiguous order), without the x
-// transform: the same phases, terms and wall rules as k_rhs_mom2 on LDS rows
-// of S = TX + 6 points (columns i0-3 .. i0+TX+2; a derived row holds the
-// columns that phase 2 reads).  ff, gg, hh are stored; qu, qv, qw go as
-// physical rows into the storage of their spectra (a row of nx values takes
-// the bytes of its nx/2 modes), which launch_r2c_n then transforms in place.
-// The small LDS tile lets several blocks share a CU, so that one block's
-// loads overlap another's stencils.
-// DAMP (levels that read the sponge of a damped substep, FP64): every value
-// is read as rayleigh_damping leaves it (src/module_tools.f90:705-749): a
-// level k >= kdamp0 damped at the domain's interior (i, j), undamped at a
-// wrapped x / y position (the stale halo) and in a z ghost.  That equals the
-// reference for the points two or more columns and rows from the domain's
-// x / y edges, whose interpolants all sit at interior centres;
-// k_rhs_mom_edge then recomputes the points nearer the edges.
-template <int CDS, int TX, int TY, class R, bool DAMP = false>
-__global__ __launch_bounds__(TX * TY, 4) void k_rhs_mom_xt(StepArgsT<R> A)
+// Momentum right-hand side of the levels that read the sponge of a damped
+// substep, on a TX x TY tile of level k (x tiles fastest, then y tiles, then
+// levels, in XCD-contiguous order), without the x transform: the phases,
+// terms and wall rules of k_rhs_mom2 on LDS rows of S = TX + 6 points
+// (columns i0-3 .. i0+TX+2; a derived row holds the columns that phase 2
+// reads).  Outputs as k_rhs_mom_march's.  Every value is read as
+// rayleigh_damping leaves it (src/module_tools.f90:705-749): a level k >=
+// kdamp0 damped at the domain's interior (i, j), undamped at a wrapped x / y
+// position (the stale halo) and in a z ghost.  That equals the reference for
+// the points two or more columns and rows from the domain's x / y edges,
+// whose interpolants all sit at interior centres; k_rhs_mom_edge then
+// recomputes the points nearer the edges.
+template <int CDS, int TX, int TY>
+__global__ __launch_bounds__(TX * TY, 4) void k_rhs_mom_sponge(StepArgs A)
 {
+    using R = double;
     constexpr int T = TX * TY, S = TX + 6, HX = 3;
     using Tl = Tile2<S, TY>;
     constexpr int NST = (Tl::NRAW * S + T - 1) / T;
@@ -239,11 +170,9 @@ __global__ __launch_bounds__(TX * TY, 4) void k_rhs_mom_xt(StepArgsT<R> A)
     auto gx = [&](int x) -> unsigned { return (unsigned)wrapi(i0 - HX + x, nx); };
     // field fid of level kk as the damped substep reads it (interior point)
     auto dmp = [&](int fid, int kk, R v) __attribute__((always_inline)) {
-        if constexpr (DAMP) {
-            if (kk >= A.kdamp0 && ((A.dmask >> fid) & 1)) {
-                const R s = A.dmp_s[kk], m = A.dmp_m[fid * A.nz + kk];
-                v = v - s * (v - m);
-            }
+        if (kk >= A.kdamp0 && ((A.dmask >> fid) & 1)) {
+            const R s = A.dmp_s[kk], m = A.dmp_m[fid * A.nz + kk];
+            v = v - s * (v - m);
         }
         return v;
     };
@@ -283,7 +212,7 @@ __global__ __launch_bounds__(TX * TY, 4) void k_rhs_mom_xt(StepArgsT<R> A)
                          (unsigned)(i0 + x)];
         }
     }
-    if constexpr (DAMP) {
+    {
         // the staged rows: damped at the domain's interior positions only
 #pragma unroll
         for (int m = 0; m < NST; ++m) {
@@ -388,7 +317,7 @@ __global__ __launch_bounds__(TX * TY, 4) void k_rhs_mom_xt(StepArgsT<R> A)
 // of the domain's x / y edges (x in 0,1,nx-2,nx-1 or y in 0,1,ny-2,ny-1):
 // their stencils read stale halos and interpolants evaluated at wrapped
 // centres, which the accessor PtD reproduces.  Writes ff, gg, hh and the
-// physical qu, qv, qw over the values k_rhs_mom_xt<..., DAMP> left there.
+// physical qu, qv, qw over the values k_rhs_mom_sponge left there.
 template <int CDS>
 __global__ __launch_bounds__(256) void k_rhs_mom_edge(StepArgs A)
 {
@@ -419,13 +348,38 @@ __global__ __launch_bounds__(256) void k_rhs_mom_edge(StepArgs A)
     reinterpret_cast<double *>(A.s2)[c] = qw;
 }
 
-// Tile shapes of k_rhs_mom_xt (launch-shape knob rhs_xt; 0 is the fused
-// whole-row kernel)
+// Tile shapes of k_rhs_mom_march and k_rhs_mom_sponge (launch-shape knob
+// rhs_xt; 0 leaves the choice to march_shape)
 constexpr int kRhsXtTX[5] = {0, 32, 64, 32, 64};
 constexpr int kRhsXtTY[5] = {0, 8, 8, 16, 4};
 bool rhs_xt_fits(int shape, int nx, int ny)
 {
     return shape >= 1 && shape <= 4 && nx % kRhsXtTX[shape] == 0 && ny % kRhsXtTY[shape] == 0;
+}
+
+// Tile shape of the marching kernel, 0 for whole rows fused with the x
+// transform.  Without a choice by the caller: FP64 rows of 96 and more march
+// (whole rows hold one block of 1024 threads and 158 KB per CU), as do rows
+// beyond 256, which do not fit a block.  Shorter rows stay fused (64x64x65:
+// 23.0 us against 23.4 in two launches), and so do FP32 rows up to 256: two
+// blocks per CU and no rows through HBM, 0.312 ms at 256x256x257 against
+// 0.342 for the best tile.  Every length from 96 on is a multiple of 32 and
+// ny of 16, so 32x8 divides the grid.
+template <class R>
+static int march_shape(const hc_ctx *c)
+{
+    if (rhs_xt_fits(c->tune.rhs_xt, c->nx, c->ny)) return c->tune.rhs_xt;
+    return c->nx > 256 || (sizeof(R) == 8 && c->nx >= 96) ? 1 : 0;
+}
+// Levels of one block's run.  A run costs two levels' loads more than it
+// forms, so about 12 levels and more; but at least three blocks per CU (what
+// the registers hold), and up to eight (or runs of 48 levels) so that the
+// last blocks leave no CU idle for long.
+static int march_levels(int ntile, int nlev, int ncu)
+{
+    const int lo = 3 * ncu / ntile, hi = std::max(8 * ncu / ntile, nlev / 48);
+    const int nrun = std::max(1, std::min(nlev, std::min(std::max(nlev / 12, lo), std::max(hi, lo))));
+    return (nlev + nrun - 1) / nrun;
 }
 
 // Momentum RHS + x R2C of qu,qv,qw through a global-memory accessor: PtD in
@@ -539,8 +493,8 @@ int rhs_momentum(hc_ctx *c, const StepArgs &A, StepArgsT<R> &B)
             if (rhs_xt_fits(sh, c->nx, c->ny) && c->nx >= 4 && c->ny >= 4) {
                 const dim3 g((unsigned)(c->nx / kRhsXtTX[sh] * (c->ny / kRhsXtTY[sh]) * B.nlev));
 #define HC_XTD(TX_, TY_)                                                                                                 \
-    if (P.cds == 1) hipLaunchKernelGGL((k_rhs_mom_xt<1, TX_, TY_, R, true>), g, dim3(TX_ * TY_), 0, c->stream, B);       \
-    else hipLaunchKernelGGL((k_rhs_mom_xt<2, TX_, TY_, R, true>), g, dim3(TX_ * TY_), 0, c->stream, B);
+    if (P.cds == 1) hipLaunchKernelGGL((k_rhs_mom_sponge<1, TX_, TY_>), g, dim3(TX_ * TY_), 0, c->stream, B);       \
+    else hipLaunchKernelGGL((k_rhs_mom_sponge<2, TX_, TY_>), g, dim3(TX_ * TY_), 0, c->stream, B);
                 switch (sh) {
                 case 1: HC_XTD(32, 8) break;
                 case 2: HC_XTD(64, 8) break;
@@ -580,12 +534,13 @@ int rhs_momentum(hc_ctx *c, const StepArgs &A, StepArgsT<R> &B)
     if (!z6 && ksplit > 0) {
         B.klo = 0;
         B.nlev = ksplit;
-        if (rhs_xt_fits(c->tune.rhs_xt, c->nx, c->ny)) {
-            const int sh = c->tune.rhs_xt;
-            const dim3 g((unsigned)(c->nx / kRhsXtTX[sh] * (c->ny / kRhsXtTY[sh]) * ksplit));
+        if (const int sh = march_shape<R>(c)) {
+            const int ntile = c->nx / kRhsXtTX[sh] * (c->ny / kRhsXtTY[sh]);
+            B.kchunk = march_levels(ntile, ksplit, c->ncu);
+            const dim3 g((unsigned)(ntile * ((ksplit + B.kchunk - 1) / B.kchunk)));
 #define HC_XT(TX_, TY_)                                                                                      \
-    if (P.cds == 1) hipLaunchKernelGGL((k_rhs_mom_xt<1, TX_, TY_, R>), g, dim3(TX_ * TY_), 0, c->stream, B); \
-    else hipLaunchKernelGGL((k_rhs_mom_xt<2, TX_, TY_, R>), g, dim3(TX_ * TY_), 0, c->stream, B);
+    if (P.cds == 1) hipLaunchKernelGGL((k_rhs_mom_march<1, TX_, TY_, R>), g, dim3(TX_ * TY_), 0, c->stream, B); \
+    else hipLaunchKernelGGL((k_rhs_mom_march<2, TX_, TY_, R>), g, dim3(TX_ * TY_), 0, c->stream, B);
             switch (sh) {
             case 1: HC_XT(32, 8) break;
             case 2: HC_XT(64, 8) break;
@@ -605,12 +560,6 @@ int rhs_momentum(hc_ctx *c, const StepArgs &A, StepArgsT<R> &B)
         constexpr int T_ = rhs2_threads<NX_>();                                                          \
         if (P.cds == 1) hipLaunchKernelGGL((k_rhs_mom2<1, NX_, R>), g1, dim3(T_), 0, c->stream, B);      \
         else hipLaunchKernelGGL((k_rhs_mom2<2, NX_, R>), g1, dim3(T_), 0, c->stream, B);                 \
-    } else {                                                                                             \
-        constexpr int TY_ = rhs_ty<NX_>();                                                               \
-        dim3 g1((unsigned)(c->ny / TY_ * ksplit));                                                       \
-        constexpr int T_ = rhs_threads<NX_>();                                                           \
-        if (P.cds == 1) hipLaunchKernelGGL((k_rhs_mom<1, NX_, R>), g1, dim3(T_), 0, c->stream, B);       \
-        else hipLaunchKernelGGL((k_rhs_mom<2, NX_, R>), g1, dim3(T_), 0, c->stream, B);                  \
     }
             HC_DISPATCH_N(c->nx, HC_RHS)
 #undef HC_RHS

@@ -222,3 +222,30 @@ def test_temperature_solve_with_top_gradient_matches_oracle(wall_rows):
     err = rel_l2(got, ref)
     print(f"t solve, top gradient, wall_rows {wall_rows}: rel L2 {err:.3e}")
     assert err < 1e-13
+
+
+@pytest.mark.parametrize("shape,tile,kw", [
+    ((96, 16, 3), 0, {}),                  # the fewest levels: a run's first level, interior and top
+    ((32, 32, 13), 1, {"cds": 1}),         # one tile wide, forced on short rows
+    ((128, 32, 50), 0, {"u_mrf": 0.3}),    # runs of unequal length, moving frame
+    ((192, 48, 37), 4, {"dp_opt": 3, "fc": 0.5, "ug": 1.0, "vg": 0.2}),
+    ((384, 16, 20), 0, {"cds": 1}),        # rows beyond 256
+    ((512, 32, 26), 0, {"dp_opt": 2}),
+    ((64, 64, 33), 3, {}),
+])
+def test_marching_tiles_match_oracle(shape, tile, kw):
+    """k_rhs_mom_march at the edges of its tiles and runs of levels: 1e-10 as
+    for every step here (agreement is round-off times the pressure solve's
+    condition)."""
+    nx, ny, nz = shape
+    prm, st = small_case("closed", nx=nx, ny=ny, nz=nz, **{"dt": 5e-4, "wall_rows": 1, **kw})
+    o = make_oracle(prm, st)
+    ch = _channel(prm, st)
+    ch.set_tuning(rhs_xt=tile)
+    o.steps(2)
+    ch.steps(2)
+    for n in ["u", "v", "w", "p"]:
+        err = rel_l2(ch.get_field(n), o.get(n))
+        print(f"{shape} {tile} {kw} {n}: rel L2 {err:.3e}")
+        assert err < 1e-10, (n, err)
+    ch.close()
