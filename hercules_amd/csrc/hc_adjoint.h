@@ -70,7 +70,7 @@ HC_DEV double2 lvl_up(const ColMap &m, const double2 (&v)[L], int r, double2 nex
 #pragma unroll
     for (int q = 0; q < L; ++q)
         if (q == r + 1) cand = v[q];
-    return r + 1 < m.cnt ? cand : next;
+    return r < L - 1 ? cand : next;
 }
 template <int L>
 HC_DEV double2 lvl_dn(const double2 (&v)[L], int r, double2 prev)
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(64 * kColWaves) void k_adj_column(StepArgs A)
     extern __shared__ double2 tile_raw[];
     double2 *tile = tile_raw;
     const int l = blockIdx.x * kColWaves + (threadIdx.x >> 6), jm = blockIdx.y;
-    const ColMap m = col_map(A.nz);
+    const ColMap m = col_map<L>(A.nz);
     const int nz = A.nz, nl = A.nl, ny = A.ny;
     const bool is00 = (l == 0 && jm == 0);
     const size_t plane = (size_t)ny * nl, col0 = (size_t)jm * nl + (size_t)blockIdx.x * kColWaves;
@@ -108,8 +108,8 @@ __global__ __launch_bounds__(64 * kColWaves) void k_adj_column(StepArgs A)
     auto lev = [&](int t, int k) { return A.lev[t * nz + k]; };
     // 1. adjoint of phi: projection u** = u* - cdt G phi and the increment
     //    P_inc = phi - cnu (slap + Lz) phi (Neumann ghosts)
-    const double2 pprev = shfl_up_c(last_of<L>(pb, m.cnt), 1), pnext = shfl_dn_c(pb[0], 1);
-    const double2 wprev = shfl_up_c(last_of<L>(wb[0], m.cnt), 1);
+    const double2 pprev = part_prev(pb[L - 1]), pnext = part_next(pb[0]);
+    const double2 wprev = part_prev(wb[0][L - 1]);
     double2 ph[1][L];
 #pragma unroll
     for (int r = 0; r < L; ++r) {
@@ -136,10 +136,10 @@ __global__ __launch_bounds__(64 * kColWaves) void k_adj_column(StepArgs A)
     //    solve, then the delnull zeroing of level 0 of the (0,0) source
     double a[L], b[L], c[L];
     assemble_T<L>(A, 2, l, jm, is00, m, a, b, c);
-    wave_tridiag_refined<L, 1>(m.cnt, a, b, c, ph);
+    wave_tridiag_refined<L, 1>(a, b, c, ph);
     if (is00 && m.lane == 0) ph[0][0] = czero();
     // 3. adjoint of u*, v*, w*: add the transposed divergence / dt
-    const double2 snext = shfl_dn_c(ph[0][0], 1);
+    const double2 snext = part_next(ph[0][0]);
 #pragma unroll
     for (int r = 0; r < L; ++r) {
         if (r >= m.cnt) continue;
@@ -154,9 +154,9 @@ __global__ __launch_bounds__(64 * kColWaves) void k_adj_column(StepArgs A)
     // 4. transposed Helmholtz solves; the w source's top level is discarded
     //    by the forward solve, so its adjoint is zero
     assemble_T<L>(A, 0, l, jm, is00, m, a, b, c);
-    wave_tridiag<L, 2>(m.cnt, a, b, c, ub);
+    wave_tridiag<L, 2>(a, b, c, ub);
     assemble_T<L>(A, 1, l, jm, is00, m, a, b, c);
-    wave_tridiag<L, 1>(m.cnt, a, b, c, wb);
+    wave_tridiag<L, 1>(a, b, c, wb);
 #pragma unroll
     for (int r = 0; r < L; ++r)
         if (r < m.cnt && m.k0 + r == nz - 1) wb[0][r] = czero();

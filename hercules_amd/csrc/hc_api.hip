@@ -573,7 +573,7 @@ StepArgs base_args(hc_ctx *c)
     const hc_params &P = c->prm;
     A.u = c->u; A.v = c->v; A.w = c->w; A.p = c->p; A.t = c->t;
     A.s0 = c->s[0]; A.s1 = c->s[1]; A.s2 = c->s[2]; A.s3 = c->s[3];
-    A.lev = c->lev; A.symx = c->symx; A.symy = c->symy;
+    A.lev = c->lev; A.levp = c->levp; A.symx = c->symx; A.symy = c->symy;
     A.tw_nl = c->tw_nl; A.tw_nx = c->tw_nx; A.tw_ny = c->tw_ny;
     A.scal = c->scal;
     A.nx = c->nx; A.ny = c->ny; A.nz = c->nz; A.nl = c->nl;
@@ -744,7 +744,7 @@ extern "C" int hc_create(const hc_params *prm, hc_ctx **out)
         const int ty = rhs_tile_rows(P.nx);
         if (P.ny % ty != 0) return set_err(HC_ERR_UNSUPPORTED, "ny=%d must be a multiple of %d for nx=%d", P.ny, ty, P.nx);
     }
-    int L = col_levels(P.nz);
+    int L = col_levels(P.nz, P.precision == HC_MIXED);
     if (L < 0) return set_err(HC_ERR_UNSUPPORTED, "nz=%d too large", P.nz);
     hc_ctx *c = new hc_ctx();
     c->prm = P;
@@ -777,6 +777,15 @@ extern "C" int hc_create(const hc_params *prm, hc_ctx **out)
     build_symbols(P, c->ny, c->ny, c->dy, P.ly, sy);
     auto tnl = twiddles(c->nl), tnx = twiddles(c->nx), tny = twiddles(c->ny);
     if (!e) e = dalloc(c, (void **)&c->lev, c->h_lev.size() * sizeof(double));
+    // the level tables as the column kernels read them: lane 16 (s mod 4) + s / 4
+    // holds levels s L .. s L + L - 1 (hc_device.h)
+    std::vector<double> hp((size_t)LV_COUNT * L * 64, 0.0);
+    for (int tab = 0; tab < LV_COUNT; ++tab)
+        for (int k = 0; k < P.nz; ++k) {
+            const int s = k / L, lane = 16 * (s % 4) + s / 4;
+            hp[((size_t)tab * L + k % L) * 64 + lane] = c->h_lev[(size_t)tab * P.nz + k];
+        }
+    if (!e) e = dalloc(c, (void **)&c->levp, hp.size() * sizeof(double));
     if (!e) e = dalloc(c, (void **)&c->symx, sx.size() * sizeof(double));
     if (!e) e = dalloc(c, (void **)&c->symy, sy.size() * sizeof(double));
     if (!e) e = dalloc(c, (void **)&c->tw_nl, tnl.size() * sizeof(double2));
@@ -842,6 +851,7 @@ extern "C" int hc_create(const hc_params *prm, hc_ctx **out)
     }
     double scal0[8] = {P.dp_opt == 1 ? 1.0 : 0.0, 0, 0, 0, 0, 0, 0, 0};
     hipError_t r = hipMemcpyAsync(c->lev, c->h_lev.data(), c->h_lev.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
+    if (r == hipSuccess) r = hipMemcpyAsync(c->levp, hp.data(), hp.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
     if (r == hipSuccess) r = hipMemcpyAsync(c->symx, sx.data(), sx.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
     if (r == hipSuccess) r = hipMemcpyAsync(c->symy, sy.data(), sy.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
     if (r == hipSuccess) r = hipMemcpyAsync(c->tw_nl, tnl.data(), tnl.size() * sizeof(double2), hipMemcpyHostToDevice, c->stream);

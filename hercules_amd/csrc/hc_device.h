@@ -2,7 +2,7 @@
 //   * batched in-place Stockham FFTs over LDS (radix 4/2/3),
 //   * a wave64 partitioned tridiagonal solver (one system per wavefront,
 //     levels split across lanes, interface system by parallel cyclic
-//     reduction over lane shuffles).
+//     reduction).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -175,22 +175,171 @@ HC_DEV void lds_fft(C *lds, const C *__restrict__ tw, int tid)
 // Wave64 partitioned tridiagonal solver.
 //
 // One system a_k x_{k-1} + b_k x_k + c_k x_{k+1} = d_k of n levels per
-// wavefront.  Lane s owns `cnt` consecutive levels (cnt <= L) held in
-// registers; lanes are filled in order, so lanes with cnt == 0 come last.
-// The first level of each lane is its interface unknown X_s; the remaining
-// levels are eliminated locally (Thomas, pivots never shared) in terms of
-// X_s and X_{s+1}, giving a tridiagonal system in X over the lanes that is
-// solved by parallel cyclic reduction through lane shuffles, after which the
-// interior is recovered.  Requires a_0 = 0 and c_{n-1} = 0.  NR complex
-// right-hand sides share the matrix; d is overwritten by the solution.
-// Re (double or float) is the arithmetic of the whole solve.
+// wavefront.  Part s = 0..63 owns the L consecutive levels s L .. s L + L-1
+// in registers; levels past n are rows of the identity (a = c = d = 0, b =
+// 1), so that no step depends on how many levels a part holds.  The first
+// level of each part is its interface unknown X_s; the others are eliminated
+// locally (Thomas, pivots never shared) in terms of X_s and X_{s+1}, giving a
+// tridiagonal system in X over the parts that is solved by parallel cyclic
+// reduction, after which the interior is recovered.  Requires a_0 = 0 and
+// c_{n-1} = 0.  NR complex right-hand sides share the matrix; d is
+// overwritten by the solution.
+//
+// Part s sits in lane 16 (s mod 4) + s / 4: the reduction's strides of 4, 8,
+// 16 and 32 parts are then shifts by 1, 2, 4 and 8 within a row of 16 lanes,
+// which are DPP moves, and only strides 1 and 2 go through the LDS crossbar.
+// A neighbour beyond the ends may read anything finite: the coefficient that
+// multiplies it is exactly zero at every stage.
+// (256x256x257 FP64, k_column_mom, five levels per lane in lane order with
+// levels spread evenly, every operation selected by the part's count and
+// every shift a ds_bpermute: 3647 VALU instructions and 588 bpermutes.)
+template <class Re> HC_DEV Re lane_of(Re v, int lane) { return __shfl(v, lane, 64); }
+template <class C> HC_DEV C lane_of_c(C v, int lane) { return mk2<C>(__shfl(v.x, lane, 64), __shfl(v.y, lane, 64)); }
+HC_DEV int part_of_lane() { const int lane = threadIdx.x & 63; return ((lane & 15) << 2) | (lane >> 4); }
+HC_DEV int lane_of_part(int s) { return ((s & 3) << 4) | ((s & 63) >> 2); }
+// a value of the part before / after this one (of the other end beyond the ends)
+template <class C> HC_DEV C part_prev(C v) { return lane_of_c(v, lane_of_part(part_of_lane() - 1)); }
+template <class C> HC_DEV C part_next(C v) { return lane_of_c(v, lane_of_part(part_of_lane() + 1)); }
+
+// lane i of a row of 16 receives lane i - N (UP) or i + N, zero beyond the row
+template <int N, bool UP> HC_DEV int row_shift(int v)
+{
+    return __builtin_amdgcn_mov_dpp(v, (UP ? 0x110 : 0x100) + N, 0xf, 0xf, true);
+}
+template <int N, bool UP> HC_DEV float row_shift(float v)
+{
+    return __int_as_float(row_shift<N, UP>(__float_as_int(v)));
+}
+template <int N, bool UP> HC_DEV double row_shift(double v)
+{
+    return __hiloint2double(row_shift<N, UP>(__double2hiint(v)), row_shift<N, UP>(__double2loint(v)));
+}
+// the value ST parts below (UP) or above; lane: that part's lane, for strides under 4
+template <int ST, bool UP, class Re> HC_DEV Re part_shift(Re v, int lane)
+{
+    if constexpr (ST < 4) return lane_of(v, lane);
+    else return row_shift<ST / 4, UP>(v);
+}
+template <int ST, int NR, class Re>
+HC_DEV void pcr_stages(Re &al, Re &be, Re &ga, cplx<Re> (&de)[NR], int s)
+{
+    if constexpr (ST < 64) {
+        using C = cplx<Re>;
+        const int lo = lane_of_part(s - ST), hi = lane_of_part(s + ST);
+        const Re ib = rcpr(be);
+        const Re k1 = al * part_shift<ST, true>(ib, lo), k2 = ga * part_shift<ST, false>(ib, hi);
+        const Re al_lo = part_shift<ST, true>(al, lo), ga_lo = part_shift<ST, true>(ga, lo);
+        const Re al_hi = part_shift<ST, false>(al, hi), ga_hi = part_shift<ST, false>(ga, hi);
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            const C l = mk2<C>(part_shift<ST, true>(de[q].x, lo), part_shift<ST, true>(de[q].y, lo));
+            const C h = mk2<C>(part_shift<ST, false>(de[q].x, hi), part_shift<ST, false>(de[q].y, hi));
+            de[q] = caxpy_neg(caxpy_neg(de[q], k1, l), k2, h);
+        }
+        be = be - ga_lo * k1 - al_hi * k2;
+        al = -al_lo * k1;
+        ga = -ga_hi * k2;
+        pcr_stages<ST * 2, NR, Re>(al, be, ga, de, s);
+    }
+}
+
+template <int L, int NR, class Re>
+HC_DEV void wave_tridiag(const Re (&a)[L], const Re (&b)[L], const Re (&c)[L], cplx<Re> (&d)[NR][L])
+{
+    using C = cplx<Re>;
+    static_assert(L >= 2, "a part holds its interface level and at least one more");
+    const int s = part_of_lane();
+    // interior levels 1..L-1 in terms of the part's X and the next part's:
+    // x_r = d_r + g_r X + h_r X'
+    Re cp[L], g[L], h[L];
+#pragma unroll
+    for (int r = 1; r < L; ++r) {
+        const Re iv = rcpr(r > 1 ? b[r] - a[r] * cp[r - 1] : b[r]);
+        cp[r] = c[r] * iv;
+        g[r] = (r == 1 ? -a[1] : -a[r] * g[r - 1]) * iv;
+        h[r] = r == L - 1 ? -c[r] * iv : Re(0);
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            const C y = r > 1 ? caxpy_neg(d[q][r], a[r], d[q][r - 1]) : d[q][r];
+            d[q][r] = cscale(y, iv);
+        }
+    }
+#pragma unroll
+    for (int r = L - 2; r >= 1; --r) {
+        g[r] -= cp[r] * g[r + 1];
+        h[r] = -cp[r] * h[r + 1];
+#pragma unroll
+        for (int q = 0; q < NR; ++q) d[q][r] = caxpy_neg(d[q][r], cp[r], d[q][r + 1]);
+    }
+    // interface rows: the level before X_s is the last of part s-1
+    const int before = lane_of_part(s - 1), after = lane_of_part(s + 1);
+    Re al = a[0] * lane_of(g[L - 1], before);
+    Re be = b[0] + a[0] * lane_of(h[L - 1], before) + c[0] * g[1];
+    Re ga = c[0] * h[1];
+    C de[NR];
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+        de[q] = caxpy_neg(caxpy_neg(d[q][0], a[0], lane_of_c(d[q][L - 1], before)), c[0], d[q][1]);
+    pcr_stages<1, NR, Re>(al, be, ga, de, s);
+    const Re ib = rcpr(be);
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+        const C X = cscale(de[q], ib), Xn = lane_of_c(X, after);
+#pragma unroll
+        for (int r = 1; r < L; ++r) {
+            d[q][r].x += g[r] * X.x + h[r] * Xn.x;
+            d[q][r].y += g[r] * X.y + h[r] * Xn.y;
+        }
+        d[q][0] = X;
+    }
+}
+
+// The same solve followed by one step of fixed-precision iterative
+// refinement: r = d - T x is formed with the neighbouring parts' values and
+// solved again.  PCR's residual on the stiff stretched-grid Neumann systems
+// is 1e3-1e4 times that of a sequential Thomas sweep (its forward error is
+// comparable); one refinement step brings the residual back to the Thomas
+// level, which is what the divergence of the projected velocity measures.
+template <int L, int NR, class Re>
+HC_DEV void wave_tridiag_refined(const Re (&a)[L], const Re (&b)[L], const Re (&c)[L], cplx<Re> (&d)[NR][L])
+{
+    using C = cplx<Re>;
+    C res[NR][L];
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+#pragma unroll
+        for (int r = 0; r < L; ++r) res[q][r] = d[q][r];
+    wave_tridiag<L, NR>(a, b, c, d);
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+        const C xprev = part_prev(d[q][L - 1]), xnext = part_next(d[q][0]);
+#pragma unroll
+        for (int r = 0; r < L; ++r) {
+            const C xm = r == 0 ? xprev : d[q][r > 0 ? r - 1 : 0];
+            const C xp = r == L - 1 ? xnext : d[q][r < L - 1 ? r + 1 : r];
+            const C x0 = d[q][r];
+            res[q][r].x -= a[r] * xm.x + b[r] * x0.x + c[r] * xp.x;
+            res[q][r].y -= a[r] * xm.y + b[r] * x0.y + c[r] * xp.y;
+        }
+    }
+    wave_tridiag<L, NR>(a, b, c, res);
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+#pragma unroll
+        for (int r = 0; r < L; ++r) d[q][r] = cadd(d[q][r], res[q][r]);
+}
+
+// ---- Systems of the mixed variant (FP32 spectra): the levels spread evenly
+// over the lanes in order (cnt <= L each; lanes with none come last).  Its
+// Poisson solution moves by more than FP32 rounding when operations are
+// rounded in another order, so these solves keep theirs.
 template <class Re> HC_DEV Re shfl_up1(Re v, int d) { return __shfl_up(v, d, 64); }
 template <class Re> HC_DEV Re shfl_dn1(Re v, int d) { return __shfl_down(v, d, 64); }
 template <class C> HC_DEV C shfl_up_c(C v, int d) { return mk2<C>(__shfl_up(v.x, d, 64), __shfl_up(v.y, d, 64)); }
 template <class C> HC_DEV C shfl_dn_c(C v, int d) { return mk2<C>(__shfl_down(v.x, d, 64), __shfl_down(v.y, d, 64)); }
 
 template <int L, int NR, class Re>
-HC_DEV void wave_tridiag(int cnt, const Re (&a)[L], const Re (&b)[L], const Re (&c)[L], cplx<Re> (&d)[NR][L])
+HC_DEV void lane_tridiag(int cnt, const Re (&a)[L], const Re (&b)[L], const Re (&c)[L], cplx<Re> (&d)[NR][L])
 {
     using C = cplx<Re>;
     const Re zero = Re(0), one = Re(1);
@@ -326,14 +475,9 @@ HC_DEV void wave_tridiag(int cnt, const Re (&a)[L], const Re (&b)[L], const Re (
     for (int q = 0; q < NR; ++q) d[q][0] = X[q];
 }
 
-// The same solve followed by one step of fixed-precision iterative
-// refinement: r = d - T x is formed with the neighbouring lanes' values and
-// solved again.  PCR's residual on the stiff stretched-grid Neumann systems
-// is 1e3-1e4 times that of a sequential Thomas sweep (its forward error is
-// comparable); one refinement step brings the residual back to the Thomas
-// level, which is what the divergence of the projected velocity measures.
+// and refined as below
 template <int L, int NR, class Re>
-HC_DEV void wave_tridiag_refined(int cnt, const Re (&a)[L], const Re (&b)[L], const Re (&c)[L], cplx<Re> (&d)[NR][L])
+HC_DEV void lane_tridiag_refined(int cnt, const Re (&a)[L], const Re (&b)[L], const Re (&c)[L], cplx<Re> (&d)[NR][L])
 {
     using C = cplx<Re>;
     const int lane = threadIdx.x & 63;
@@ -342,7 +486,7 @@ HC_DEV void wave_tridiag_refined(int cnt, const Re (&a)[L], const Re (&b)[L], co
     for (int q = 0; q < NR; ++q)
 #pragma unroll
         for (int r = 0; r < L; ++r) d0[q][r] = d[q][r];
-    wave_tridiag<L, NR>(cnt, a, b, c, d);
+    lane_tridiag<L, NR>(cnt, a, b, c, d);
     C res[NR][L];
 #pragma unroll
     for (int q = 0; q < NR; ++q) {
@@ -369,7 +513,7 @@ HC_DEV void wave_tridiag_refined(int cnt, const Re (&a)[L], const Re (&b)[L], co
             }
         }
     }
-    wave_tridiag<L, NR>(cnt, a, b, c, res);
+    lane_tridiag<L, NR>(cnt, a, b, c, res);
 #pragma unroll
     for (int q = 0; q < NR; ++q)
 #pragma unroll

@@ -84,6 +84,7 @@ struct hc_ctx {
     int fcur, scur;
     double2 *s[4];
     double *lev, *symx, *symy, *scal, *part, *stage;
+    double *levp = nullptr;  // lev in the order the column kernels read it: [table][r][lane] for level r of a lane's Lcol
     // 6th-order z operators (zorder = 6): stencil starts and weights, and
     // the interpolants the right-hand-side kernels read (k_zinterp6)
     int *zst = nullptr;
@@ -193,13 +194,15 @@ inline int rhs_tile_rows(int nx)
     return nx == 16 ? 16 : nx == 32 ? 32 : nx == 48 ? 16 : nx == 64 ? 16 : nx == 96 ? 8 : nx == 128 ? 8 : nx <= 256 ? 4 : 1;
 }
 
-inline int col_levels(int nz)
+// levels per lane of the column kernels (7 for FP64 spectra only)
+inline int col_levels(int nz, bool mixed)
 {
     int L = (nz + 63) / 64;
     if (L <= 2) return 2;
     if (L <= 3) return 3;
     if (L <= 4) return 4;
     if (L <= 5) return 5;
+    if (L <= 7 && !mixed) return 7;
     if (L <= 8) return 8;
     if (L <= 16) return 16;
     return -1;
@@ -293,6 +296,7 @@ inline StepArgsT<double> rows_args<double>(const StepArgs &A, const View<double>
     case 3: MACRO(3); break;                                                              \
     case 4: MACRO(4); break;                                                              \
     case 5: MACRO(5); break;                                                              \
+    case 7: MACRO(7); break;                                                              \
     case 8: MACRO(8); break;                                                              \
     case 16: MACRO(16); break;                                                            \
     default: return set_err(HC_ERR_UNSUPPORTED, "unsupported nz");                       \
@@ -363,6 +367,7 @@ hipError_t spec_set_lds(int L, int bytes);
 // launch_spec_columns) over spectra stored as R
 template <class RIO> struct SpecIO;  // hc_spectral.h
 template <class R> void zinterp6(hc_ctx *c, StepArgsT<R> &B);
+template <class R> void z6_terms(hc_ctx *c, const StepArgsT<R> &B, int e0);
 template <class R> void launch_col6(int kind, hipStream_t st, const StepArgs &A, const ColIO<R> &io, int eq);
 template <class R> void launch_spec_col6(int kind, hipStream_t st, const StepArgs &A, const SpecIO<R> &io);
 hipError_t z6_set_lds(int L, int bytes);

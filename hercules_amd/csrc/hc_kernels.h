@@ -89,6 +89,7 @@ struct StepArgsT {
     Cx *s0, *s1, *s2, *s3;
     // tables
     const R *lev, *symx, *symy;
+    const double *levp;  // lev in the column kernels' order (hc_ctx::levp)
     const Cx *tw_nl, *tw_nx, *tw_ny;
     const double *scal;  // device scalars: [0] dpx_drive, [1] ubar
     int nx, ny, nz, nl;

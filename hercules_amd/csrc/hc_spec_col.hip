@@ -69,6 +69,7 @@ hipError_t spec_set_lds(int L, int bytes)
     case 3: HC_A(3) break;
     case 4: HC_A(4) break;
     case 5: HC_A(5) break;
+    case 7: HC_A(7) break;
     case 8: HC_A(8) break;
     case 16: HC_A(16) break;
     default: return hipErrorInvalidValue;

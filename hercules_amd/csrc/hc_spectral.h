@@ -293,33 +293,22 @@ HC_DEV C zghost(const StepArgs &A, int kind, bool bottom, C c, bool is00)
     }
 }
 
-// value of level r+1 of this lane (runtime r), or the next lane's first
-template <int L, class C>
-HC_DEV C col_up(const ColMap &m, const C (&c)[L], int r, C next)
-{
-    C cand = czero_t<C>();
-#pragma unroll
-    for (int q = 0; q < L; ++q)
-        if (q == r + 1) cand = c[q];
-    return r + 1 < m.cnt ? cand : next;
-}
-
 // q += coef * ((c(k+1)-c(k))/dz_t - (c(k)-c(k-1))/dz_b)/dz
-template <int L, class C>
-HC_DEV void add_dzz(const StepArgs &A, const ColMap &m, int kind, bool is00, const C (&c)[L], real_of<C> coef,
+template <int L, class C, class M>
+HC_DEV void add_dzz(const StepArgs &A, const M &m, int kind, bool is00, const C (&c)[L], real_of<C> coef,
                     C (&q)[L])
 {
     using Re = real_of<C>;
     const int nz = A.nz;
-    const C prev = shfl_up_c(last_of<L>(c, m.cnt), 1);
-    const C next = shfl_dn_c(c[0], 1);
+    const C prev = col_before<L>(m, c);
+    const C next = col_after<L>(m, c);
 #pragma unroll
     for (int r = 0; r < L; ++r) {
         if (r >= m.cnt) continue;
         const int k = m.k0 + r;
         const C cm = k == 0 ? zghost(A, kind, true, c[r], is00) : (r == 0 ? prev : c[r > 0 ? r - 1 : 0]);
         const C cp = k == nz - 1 ? zghost(A, kind, false, c[r], is00) : col_up<L>(m, c, r, next);
-        const Re idzt = Re(A.lev[LV_IDZT * nz + k]), idzb = Re(A.lev[LV_IDZB * nz + k]), idz = Re(A.lev[LV_IDZ * nz + k]);
+        const Re idzt = Re(col_lev<L>(A, m, LV_IDZT, r)), idzb = Re(col_lev<L>(A, m, LV_IDZB, r)), idz = Re(col_lev<L>(A, m, LV_IDZ, r));
         const Re zx = ((cp.x - c[r].x) * idzt - (c[r].x - cm.x) * idzb) * idz;
         const Re zy = ((cp.y - c[r].y) * idzt - (c[r].y - cm.y) * idzb) * idz;
         q[r].x += coef * zx;
@@ -329,13 +318,13 @@ HC_DEV void add_dzz(const StepArgs &A, const ColMap &m, int kind, bool is00, con
 
 // w levels k < kend3: q += coef * ((w(k+1)-w(k))/dz(k+1) - (w(k)-w(k-1))/dz(k))/dz_t(k),
 // w(k0-1) = 0 and w(kend3) = 0 (src/module_spectral.f90:357-370)
-template <int L, class C>
-HC_DEV void add_dzz_w(const StepArgs &A, const ColMap &m, const C (&c)[L], real_of<C> coef, C (&q)[L])
+template <int L, class C, class M>
+HC_DEV void add_dzz_w(const StepArgs &A, const M &m, const C (&c)[L], real_of<C> coef, C (&q)[L])
 {
     using Re = real_of<C>;
     const int nz = A.nz;
-    const C prev = shfl_up_c(last_of<L>(c, m.cnt), 1);
-    const C next = shfl_dn_c(c[0], 1);
+    const C prev = col_before<L>(m, c);
+    const C next = col_after<L>(m, c);
 #pragma unroll
     for (int r = 0; r < L; ++r) {
         if (r >= m.cnt) continue;
@@ -373,8 +362,8 @@ HC_DEV ColPos spec_pos(const SpecIO<RIO> &io, int ny)
 // only the spectra; its z diffusion (src/module_spectral.f90:83, 225, 367,
 // 547) and w pressure gradient (:382) are formed from the physical fields,
 // which keep the undamped values.  No-op without damping.
-template <int L, class CC>
-HC_DEV void spec_undamped(const StepArgs &A, const ColMap &m, size_t plane, size_t col, int fid, CC (&x)[L])
+template <int L, class CC, class M>
+HC_DEV void spec_undamped(const StepArgs &A, const M &m, size_t plane, size_t col, int fid, CC (&x)[L])
 {
     if (!A.spund) return;
     const cplx<double> *u = A.spund + (size_t)fid * (A.nz - A.kdamp0) * plane;
@@ -392,8 +381,8 @@ HC_DEV void spec_undamped(const StepArgs &A, const ColMap &m, size_t plane, size
 // with X, Y, R the transformed products of k_spec_mom.  f_new replaces f_old.
 // With four LDS sub-tiles (A.ntile >= 4) the component moves in three
 // global phases: {c, X, Y, R} in, {f_old} in, {f_new} out.
-template <int L, class CI, class CC>
-HC_DEV void spec_assemble(const StepArgs &A, const SpecIO<real_of<CI>> &io, CI *tile, const ColMap &m, size_t plane,
+template <int L, class CI, class CC, class M>
+HC_DEV void spec_assemble(const StepArgs &A, const SpecIO<real_of<CI>> &io, CI *tile, const M &m, size_t plane,
                           size_t col0, int e, bool is00, real_of<CC> kx, real_of<CC> ky, real_of<CC> hxy,
                           const CC (&cp)[L], CC (&q)[L])
 {
@@ -409,7 +398,7 @@ HC_DEV void spec_assemble(const StepArgs &A, const SpecIO<real_of<CI>> &io, CI *
     CC x[L], f[L];
     if (batch) {
         const CI *srcs[4] = {cs, io.sp[ix], io.sp[iy], io.sp[ir]};
-        col_fill_n<L, 4>(srcs, tile, nz, plane, col0);
+        col_fill_n<L, 4, M::parts>(srcs, tile, nz, plane, col0);
         __syncthreads();
         col_take<L>(tile, m, x);
     } else {
@@ -443,7 +432,7 @@ HC_DEV void spec_assemble(const StepArgs &A, const SpecIO<real_of<CI>> &io, CI *
 #pragma unroll
         for (int r = 0; r < L; ++r) q[r] = csub(q[r], times_i(cp[r], cdt * kk));
     } else {
-        const CC next = shfl_dn_c(cp[0], 1);
+        const CC next = col_after<L>(m, cp);
 #pragma unroll
         for (int r = 0; r < L; ++r) {
             const int k = m.k0 + r;
@@ -455,7 +444,7 @@ HC_DEV void spec_assemble(const StepArgs &A, const SpecIO<real_of<CI>> &io, CI *
     }
     if (batch) {
         __syncthreads();
-        col_fill(fo, tile, nz, plane, col0);
+        col_fill<L, M::parts>(fo, tile, nz, plane, col0);
         __syncthreads();
         col_take<L>(tile, m, x);
     } else {
@@ -470,7 +459,7 @@ HC_DEV void spec_assemble(const StepArgs &A, const SpecIO<real_of<CI>> &io, CI *
     if (batch) {
         col_put<L>(tile + sub, m, f);
         __syncthreads();
-        col_drain(fo, tile + sub, nz, plane, col0);
+        col_drain<L, M::parts>(fo, tile + sub, nz, plane, col0);
         __syncthreads();
     } else {
         col_store<L>(fo, tile, nz, plane, col0, m, f);
@@ -493,7 +482,8 @@ __global__ __launch_bounds__(64 * kColWaves) void k_column_spec(StepArgs A, Spec
     const ColPos pos = spec_pos(io, A.ny);
     if (pos.skip) return;  // block-uniform, before any barrier
     const int l = pos.bx * kColWaves + (threadIdx.x >> 6), jm = pos.jm;
-    const ColMap m = col_map(A.nz);
+    constexpr bool PARTS = sizeof(RIO) == 8;
+    const auto m = col_map<L, PARTS>(A.nz);
     const int nz = A.nz, nl = A.nl, ny = A.ny;
     const bool is00 = (l == 0 && jm == 0);
     const int mw = jm < ny / 2 ? jm : jm - ny;
@@ -524,16 +514,19 @@ __global__ __launch_bounds__(64 * kColWaves) void k_column_spec(StepArgs A, Spec
         RC a[L], b[L], c[L];
         assemble<L>(A, 0, l, jm, is00, m, a, b, c);
         if (is00) fixups<L>(A, 0, m, duv[0]);
-        wave_tridiag<L, 2>(m.cnt, a, b, c, duv);
+        if constexpr (decltype(m)::parts) wave_tridiag<L, 2>(a, b, c, duv);
+        else lane_tridiag<L, 2>(m.cnt, a, b, c, duv);
 #pragma unroll
         for (int r = 0; r < L; ++r)
             if (r < m.cnt && m.k0 + r == nz - 1) dw[0][r] = czero_t<CC>();
         assemble<L>(A, 1, l, jm, is00, m, a, b, c);
-        wave_tridiag<L, 1>(m.cnt, a, b, c, dw);
+        if constexpr (decltype(m)::parts) wave_tridiag<L, 1>(a, b, c, dw);
+        else lane_tridiag<L, 1>(m.cnt, a, b, c, dw);
         col_divergence<L>(A, m, l, jm, duv[0], duv[1], dw[0], RC(A.idt), dp[0]);
         assemble<L>(A, 2, l, jm, is00, m, a, b, c);
         if (is00) fixups<L>(A, 2, m, dp[0]);
-        wave_tridiag_refined<L, 1>(m.cnt, a, b, c, dp);
+        if constexpr (decltype(m)::parts) wave_tridiag_refined<L, 1>(a, b, c, dp);
+        else lane_tridiag_refined<L, 1>(m.cnt, a, b, c, dp);
         const RC cdt = RC(A.rc * A.dt);
         // new pressure first (:461), then the projection (:464)
         const RC slap = RC(A.symx[SY_L * nl + l] + A.symy[SY_L * ny + jm]);
@@ -563,10 +556,10 @@ __global__ __launch_bounds__(64 * kColWaves) void k_column_spec(StepArgs A, Spec
         col_put<L>(tile + 2 * sub, m, dw[0]);
         col_put<L>(tile + 3 * sub, m, cpr);
         __syncthreads();
-        col_drain(io.cu, tile, nz, plane, col0);
-        col_drain(io.cv, tile + sub, nz, plane, col0);
-        col_drain(io.cw, tile + 2 * sub, nz, plane, col0);
-        col_drain(io.cp, tile + 3 * sub, nz, plane, col0);
+        col_drain<L, PARTS>(io.cu, tile, nz, plane, col0);
+        col_drain<L, PARTS>(io.cv, tile + sub, nz, plane, col0);
+        col_drain<L, PARTS>(io.cw, tile + 2 * sub, nz, plane, col0);
+        col_drain<L, PARTS>(io.cp, tile + 3 * sub, nz, plane, col0);
     } else {
         col_store<L>(io.cu, tile, nz, plane, col0, m, duv[0]);
         col_store<L>(io.cv, tile, nz, plane, col0, m, duv[1]);
@@ -588,7 +581,8 @@ __global__ __launch_bounds__(64 * kColWaves) void k_column_spec_t(StepArgs A, Sp
     const ColPos pos = spec_pos(io, A.ny);
     if (pos.skip) return;
     const int l = pos.bx * kColWaves + (threadIdx.x >> 6), jm = pos.jm;
-    const ColMap m = col_map(A.nz);
+    constexpr bool PARTS = sizeof(RIO) == 8;
+    const auto m = col_map<L, PARTS>(A.nz);
     const int nz = A.nz, nl = A.nl, ny = A.ny;
     const bool is00 = (l == 0 && jm == 0);
     const int mw = jm < ny / 2 ? jm : jm - ny;
@@ -632,7 +626,8 @@ __global__ __launch_bounds__(64 * kColWaves) void k_column_spec_t(StepArgs A, Sp
         RC a[L], b[L], c[L];
         assemble<L>(A, 3, l, jm, is00, m, a, b, c);
         if (is00) fixups<L>(A, 3, m, d[0]);
-        wave_tridiag<L, 1>(m.cnt, a, b, c, d);
+        if constexpr (decltype(m)::parts) wave_tridiag<L, 1>(a, b, c, d);
+        else lane_tridiag<L, 1>(m.cnt, a, b, c, d);
     } else {
 #pragma unroll
         for (int r = 0; r < L; ++r) d[0][r] = czero_t<CC>();

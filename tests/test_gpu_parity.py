@@ -249,3 +249,25 @@ def test_marching_tiles_match_oracle(shape, tile, kw):
         print(f"{shape} {tile} {kw} {n}: rel L2 {err:.3e}")
         assert err < 1e-10, (n, err)
     ch.close()
+
+
+@pytest.mark.parametrize("nz,kw", [
+    (3, {}), (64, {}), (65, {}), (127, {"isscalar": 1, "got": 0.05}), (129, {"cds": 1}), (320, {}), (321, {}),
+    (448, {"dp_opt": 2}), (449, {}), (512, {}), (513, {}), (1024, {}),
+])
+def test_column_levels_match_oracle(nz, kw):
+    """Column kernels at the ends of every number of levels per lane (2 to 16),
+    of the block shapes (beyond 512 levels two columns) and of three and four
+    LDS tiles.  u, v, w, t as for every step; p to round-off times the
+    condition of the (0,0) Neumann system, 4/dz_min^2 over (pi/lz)^2."""
+    prm, st = small_case("closed", nx=16, ny=16, nz=nz, wall_rows=1, dt=2e-4, **kw)
+    o = make_oracle(prm, st)
+    ch = _channel(prm, st)
+    o.steps(1)
+    ch.steps(1)
+    kappa = 4.0 / ch.mesh()[1].min() ** 2 / (np.pi / prm.lz) ** 2
+    for n in ["u", "v", "w", "p"] + (["t"] if prm.isscalar else []):
+        err = rel_l2(ch.get_field(n), o.get(n))
+        print(f"nz {nz} {kw} {n}: rel L2 {err:.3e}")
+        assert err < max(1e-10, 10 * 2.3e-16 * kappa if n == "p" else 0.0), (n, err)
+    ch.close()
