@@ -839,7 +839,10 @@ HC_DEV void temperature_point(const Q &q, typename Q::Real &s, typename Q::Real 
         tyy = (-q.T(0, 2, 0) + Re(16.0) * q.T(0, 1, 0) - Re(30.0) * q.T(0, 0, 0) + Re(16.0) * q.T(0, -1, 0) - q.T(0, -2, 0)) * A.c12y2;
     }
     Re t0 = q.T(0, 0, 0), twz, tzz;
-    if constexpr (ZO == 6) {
+    if constexpr (ZO == 6 && sizeof(Re) == 8) {  // k_z6_terms' values, left where s and qt go
+        twz = A.ss[q.center()];
+        tzz = reinterpret_cast<const Re *>(A.s0)[q.center()];
+    } else if constexpr (ZO == 6) {
         twz = q.twz6();
         tzz = q.tzz6();
     } else {
@@ -876,12 +879,118 @@ HC_DEV C c2r_pre(C xl, C xt, C twl)
     return mk2<C>(a.x - e.y, a.y + e.x);  // A + i e
 }
 
+// ---------------------------------------------------------------------------
+// LDS tile of the momentum right-hand side: full x rows j0..j0+TY-1 of
+// level k and the halo rows each stencil reaches, staged once per block.
+template <int NX, int TY>
+struct RhsTile {
+    static constexpr int RU = TY + 6;   // u, v, w at k:   rows j0-3 .. j0+TY+2
+    static constexpr int RP = TY + 3;   // p at k:         rows j0-1 .. j0+TY+1
+    static constexpr int RWM = TY + 3;  // w at k-1:       rows j0-1 .. j0+TY+1
+    static constexpr int RVP = TY + 3;  // v at k+1:       rows j0-2 .. j0+TY
+    static constexpr int RUP = TY;      // u at k+1:       rows j0   .. j0+TY-1
+    static constexpr int OU = 0, OV = RU, OW = 2 * RU, OP = 3 * RU, OWM = OP + RP, OVP = OWM + RWM,
+                         OUP = OVP + RVP, NROWS = OUP + RUP;
+};
+
 template <int NX>
 HC_DEV int wrapx(int i)
 {
     if constexpr ((NX & (NX - 1)) == 0) return i & (NX - 1);
     else return i < 0 ? i + NX : (i >= NX ? i - NX : i);
 }
+
+// Value of staged row r (of RhsTile) at column i, with the wall rules of
+// update_boundary_uvw / _p (src/module_boundary.f90:33-162) for the ghost
+// levels k-1 = -1 and k+1 = nz.
+template <int NX, int TY, class R>
+HC_DEV R rhs_stage_value(const StepArgsT<R> &A, int r, int i, int j0, int k)
+{
+    using Tl = RhsTile<NX, TY>;
+    const int ny = A.ny, nz = A.nz;
+    auto at = [&](int jj, int kk) -> size_t { return ((size_t)kk * ny + wrapi(jj, ny)) * NX + i; };
+    if (r < Tl::OV) return A.u[at(j0 - 3 + r, k)];
+    if (r < Tl::OW) return A.v[at(j0 - 3 + (r - Tl::OV), k)];
+    if (r < Tl::OP) return A.w[at(j0 - 3 + (r - Tl::OW), k)];
+    if (r < Tl::OWM) return A.p[at(j0 - 1 + (r - Tl::OP), k)];
+    if (r < Tl::OVP) return k == 0 ? R(0.0) : A.w[at(j0 - 1 + (r - Tl::OWM), k - 1)];
+    if (r < Tl::OUP) {
+        int jj = j0 - 2 + (r - Tl::OVP);
+        if (k + 1 < nz) return A.v[at(jj, k + 1)];
+        R top = A.v[at(jj, nz - 1)];
+        return A.ochannel == 0 ? -top : top;
+    }
+    int jj = j0 + (r - Tl::OUP);
+    if (k + 1 < nz) return A.u[at(jj, k + 1)];
+    R top = A.u[at(jj, nz - 1)];
+    return A.ochannel == 0 ? -top - R(2.0) * A.u_mrf : top;
+}
+
+// LDS accessor: the offsets momentum_point uses, read from the staged rows;
+// the single-point values at k-1 / k+1 come from registers.
+// Single-point values of one RHS point at levels k-1 / k+1 and the previous
+// substep's right-hand sides, loaded ahead of the LDS staging barrier.
+template <class R>
+struct PointVals {
+    R u_km, v_km, w_kp, p_kp, t_k, t_kp, f0, g0, h0;
+    HC_DEV void load(const StepArgsT<R> &a, int i, int j, int k)
+    {
+        PtT<R> g(a, i, j, k);
+        u_km = g.U(0, 0, -1);
+        v_km = g.V(0, 0, -1);
+        const bool in = k + 1 < a.nz;
+        w_kp = in ? g.W(0, 0, 1) : R(0.0);
+        p_kp = g.P(0, 0, 1);
+        t_k = a.isscalar ? g.T(0, 0, 0) : R(0.0);
+        t_kp = (a.isscalar && in) ? g.T(0, 0, 1) : R(0.0);
+        f0 = g.f0();
+        g0 = g.g0();
+        h0 = g.h0();
+    }
+};
+
+template <int NX, int TY, class R>
+struct Ld : Interp<Ld<NX, TY, R>> {
+    using Real = R;
+    using Tl = RhsTile<NX, TY>;
+    const StepArgsT<R> &A;
+    const R *sm;
+    int i, jj, j, k;
+    R u_km, v_km, w_kp, p_kp, t_k, t_kp, f0_, g0_, h0_;
+    HC_DEV Ld(const StepArgsT<R> &a, const R *s, int i_, int jj_, int j_, int k_, const PointVals<R> &pv)
+        : A(a), sm(s), i(i_), jj(jj_), j(j_), k(k_), u_km(pv.u_km), v_km(pv.v_km), w_kp(pv.w_kp),
+          p_kp(pv.p_kp), t_k(pv.t_k), t_kp(pv.t_kp), f0_(pv.f0), g0_(pv.g0), h0_(pv.h0) {}
+    HC_DEV R f0() const { return f0_; }
+    HC_DEV R g0() const { return g0_; }
+    HC_DEV R h0() const { return h0_; }
+    HC_DEV R row(int base, int r, int di) const { return sm[(base + r) * NX + wrapx<NX>(i + di)]; }
+    HC_DEV R U(int di, int dj, int dk) const
+    {
+        if (dk == 0) return row(Tl::OU, jj + 3 + dj, di);
+        if (dk > 0) return row(Tl::OUP, jj + dj, di);
+        return u_km;
+    }
+    HC_DEV R V(int di, int dj, int dk) const
+    {
+        if (dk == 0) return row(Tl::OV, jj + 3 + dj, di);
+        if (dk > 0) return row(Tl::OVP, jj + 2 + dj, di);
+        return v_km;
+    }
+    HC_DEV R W(int di, int dj, int dk) const
+    {
+        if (dk == 0) return row(Tl::OW, jj + 3 + dj, di);
+        if (dk < 0) return row(Tl::OWM, jj + 1 + dj, di);
+        return w_kp;
+    }
+    HC_DEV R P(int di, int dj, int dk) const
+    {
+        if (dk == 0) return row(Tl::OP, jj + 1 + dj, di);
+        return p_kp;
+    }
+    HC_DEV R T(int, int, int dk) const { return dk == 0 ? t_k : t_kp; }
+    HC_DEV R lev(int tab, int kk) const { return A.lev[tab * A.nz + kk]; }
+    HC_DEV size_t center() const { return ((size_t)k * A.ny + j) * NX + i; }
+};
 
 // Block id remap so that each of the 8 XCDs (which receive hardware block
 // ids round-robin) works through one contiguous range of logical tiles and

@@ -54,6 +54,9 @@ struct MarchTile {
 // read anyway.  f, g, h are stored; qu, qv, qw go as physical rows into the
 // storage of their spectra (a row of nx values takes the bytes of its nx/2
 // modes), which launch_r2c_n then transforms in place.
+// ZO = 6 (6th- and 4th-order z): the z terms at a point are k_z6_terms', left
+// where the outputs go, and the rows of level k+1 give way to those of u and v
+// at the faces of level k (zfu, zfv).
 // A level costs a thread 270 FP64 and 76 other VALU instructions and 56 LDS
 // reads; HBM and the latency of its two barriers at three waves per SIMD
 // bound it (held to 128 VGPRs for four waves, the loads in flight spill and
@@ -62,13 +65,14 @@ struct MarchTile {
 // 256x256x257 (64x4 0.64, 64x8 and 32x16, of 512 threads, 0.68), where the
 // same tiles restaged level by level took 0.66 and whole rows fused with the
 // transform 0.83; 3.9 ms at 512x512x385 (one row per block: 16.0).
-template <int CDS, int TX, int TY, class R>
+template <int CDS, int TX, int TY, class R, int ZO = 2>
 __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_march(StepArgsT<R> A)
 {
     using Tl = MarchTile<TX, TY>;
     constexpr int D0 = CDS == 1 ? 1 : 0, D1 = CDS == 1 ? 3 : 4;  // faces at -2 .. 1 of a point (cds 1: -1, 0)
     constexpr int T = TX * TY, S = Tl::S, NV = Tl::NRAW * S, NU = Tl::RU * S, NPV = Tl::RP * S;
-    constexpr int LEFT = NU % T, REST = 3 * LEFT <= T ? LEFT : 0, NM = NU / T + (LEFT > REST ? 1 : 0);
+    constexpr int NF = ZO == 6 ? 5 : 3;
+    constexpr int LEFT = NU % T, REST = NF * LEFT <= T ? LEFT : 0, NM = NU / T + (LEFT > REST ? 1 : 0);
     constexpr int NP = (NPV + T - 1) / T;
     __shared__ R raw[2][NV];
     __shared__ R fuv[Tl::RF * S];
@@ -101,20 +105,26 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
         op[m] = src_off(j0 - 1 + r, q - r * S);
     }
     if constexpr (REST > 0) {
-        if (tid < 3 * REST) {
+        if (tid < NF * REST) {
             const int fd = tid / REST, q = NM * T + tid - fd * REST, r = q / S;
-            rest = (fd == 0 ? A.u : fd == 1 ? A.v : A.w) + src_off(j0 - 3 + r, q - r * S);
-            rest_at = fd * NU + q;
+            rest = (fd == 0 ? A.u : fd == 1 ? A.v : fd == 2 ? A.w : fd == 3 ? A.zfu : A.zfv) +
+                   src_off(j0 - 3 + r, q - r * S);
+            rest_at = fd < 3 ? fd * NU + q : NV + (fd - 3) * NU + q;
         }
     }
     struct Level {
-        R f[3][NM], p[NP], x;
+        R f[NF][NM], p[NP], x;
     };
     auto fetch = [&](Level &v, int k) __attribute__((always_inline)) {
         const size_t lo = (size_t)k * plane;
         const R *ub = A.u + lo, *vb = A.v + lo, *wb = A.w + lo, *pb = A.p + lo;
 #pragma unroll
         for (int m = 0; m < NM; ++m) { v.f[0][m] = ub[ouv[m]]; v.f[1][m] = vb[ouv[m]]; v.f[2][m] = wb[ouv[m]]; }
+        if constexpr (ZO == 6) {
+            const R *fu = A.zfu + lo, *fv = A.zfv + lo;
+#pragma unroll
+            for (int m = 0; m < NM; ++m) { v.f[3][m] = fu[ouv[m]]; v.f[4][m] = fv[ouv[m]]; }
+        }
 #pragma unroll
         for (int m = 0; m < NP; ++m) v.p[m] = pb[op[m]];
         if constexpr (REST > 0) v.x = rest_at >= 0 ? rest[lo] : R(0);
@@ -124,7 +134,7 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
         for (int m = 0; m < NM; ++m)
             if (m < NM - 1 || NU >= NM * T || tid + m * T < NU) {
 #pragma unroll
-                for (int fd = 0; fd < 3; ++fd) dst[fd * NU + tid + m * T] = v.f[fd][m];
+                for (int fd = 0; fd < NF; ++fd) dst[(fd < 3 ? fd * NU : NV + (fd - 3) * NU) + tid + m * T] = v.f[fd][m];
             }
 #pragma unroll
         for (int m = 0; m < NP; ++m)
@@ -132,7 +142,7 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
         if constexpr (REST > 0)
             if (rest_at >= 0) dst[rest_at] = v.x;
     };
-    const bool two = k0 + 1 < nz;
+    const bool two = ZO == 2 && k0 + 1 < nz;
     {
         Level a;
         fetch(a, k0);
@@ -149,7 +159,7 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
     R ukm = R(0), vkm = R(0), wkm = R(0), fuw_km = R(0), fwv_km = R(0);
     R wx[4], wy[3];
     const bool bot = k0 == 0;
-    if (!bot) {
+    if (ZO == 2 && !bot) {
         const size_t lo = (size_t)(k0 - 1) * plane;
         ukm = A.u[lo + cp];
         vkm = A.v[lo + cp];
@@ -164,7 +174,7 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
     R tk = A.isscalar ? A.t[c] : R(0);
     const R dpx = A.dp_opt == 2 ? R(A.scal[0]) : A.dpx;
     __syncthreads();
-    {
+    if constexpr (ZO == 2) {
         const R u0 = raw[0][(Tl::OU + jj + 3) * S + xl], v0 = raw[0][(Tl::OV + jj + 3) * S + xl];
         if (bot) {
             ukm = -u0 - R(2.0) * um;
@@ -176,13 +186,20 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
         }
     }
     for (int k = k0, b = 0; k < k1; ++k, b ^= 1) {
-        const R *cur = raw[b], *nxt = raw[b ^ 1];
-        const bool top = k == nz - 1, more = k + 1 < k1, ahead = more && k + 2 < nz;
+        const R *cur = raw[ZO == 6 ? 0 : b], *nxt = raw[ZO == 6 ? 1 : b ^ 1];
+        const bool top = k == nz - 1, more = k + 1 < k1, ahead = more && (ZO == 6 || k + 2 < nz);
         Level pre;
-        if (ahead) fetch(pre, k + 2);
+        if (ahead) fetch(pre, ZO == 6 ? k + 1 : k + 2);
         R o0 = R(0), o1 = R(0), o2 = R(0), tkp = R(0);
         if (A.use_f0) { o0 = A.ff0[c]; o1 = A.gg0[c]; o2 = A.hh0[c]; }
-        if (A.isscalar && !top) tkp = A.t[c + plane];
+        if (ZO == 2 && A.isscalar && !top) tkp = A.t[c + plane];
+        R z[6];  // ZO = 6: k_z6_terms' values at the point
+        if constexpr (ZO == 6) {
+            z[0] = A.ff[c]; z[1] = A.gg[c]; z[2] = A.hh[c];
+            z[3] = reinterpret_cast<const R *>(A.s0)[c];
+            z[4] = reinterpret_cast<const R *>(A.s1)[c];
+            z[5] = reinterpret_cast<const R *>(A.s2)[c];
+        }
         // uhy*vhx, which the points of two rows and columns on either side read
         for (int e = tid; e < Tl::RF * (TX + 3); e += T) {
             const int r = e / (TX + 3), x = 1 + e - r * (TX + 3);
@@ -209,7 +226,7 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
 #pragma unroll
                 for (int d = D0; d < D1; ++d) {
                     m[d] = mid4<CDS>(r[d], r[d + 1], r[d + 2], r[d + 3]);
-                    x[d] = zface(qu_[d - 2], pu[d - 2], lt) * m[d];
+                    x[d] = (ZO == 6 ? qu_[d - 2] : zface(qu_[d - 2], pu[d - 2], lt)) * m[d];
                 }
                 fuw = x[2];
                 con = dif4<CDS>(x[0], x[1], x[2], x[3]) * (CDS == 1 ? A.idx : A.c24x);
@@ -224,19 +241,25 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
                 for (int d = 0; d < 7; ++d) r[d] = pw[(d - 3) * S];
 #pragma unroll
                 for (int d = D0; d < D1; ++d)
-                    x[d] = zface(qv_[(d - 2) * S], pv[(d - 2) * S], lt) * mid4<CDS>(r[d], r[d + 1], r[d + 2], r[d + 3]);
+                    x[d] = (ZO == 6 ? qv_[(d - 2) * S] : zface(qv_[(d - 2) * S], pv[(d - 2) * S], lt)) *
+                           mid4<CDS>(r[d], r[d + 1], r[d + 2], r[d + 3]);
                 fwv = x[2];
                 con += dif4<CDS>(x[0], x[1], x[2], x[3]) * (CDS == 1 ? A.idy : A.c24y);
                 lap += CDS == 1 ? (r[4] - R(2.0) * w0 + r[2]) * A.idy2
                                 : (-r[5] + R(16.0) * r[4] - R(30.0) * w0 + R(16.0) * r[2] - r[1]) * A.c12y2;
             }
-            const R wkp = k + 1 == nz - 1 ? R(0) : nxt[(Tl::OW + jj + 3) * S + xl];
-            const R pkp = nxt[(Tl::OP + jj + 1) * S + xl];
-            const R wwz = (sq(R(0.5) * (w0 + wkp)) - sq(R(0.5) * (w0 + wkm))) * idzt;
-            const R wzz = ((wkp - w0) * A.lev[LV_IDZ * nz + k + 1] - (w0 - wkm) * idz) * idzt;
-            h = -con - wwz - um * wx_;
-            if (A.isscalar) h += A.got * (zface(tkp, tk, lt) - A.t_ref);
-            qw = w0 + A.dt * (A.ra * h + A.rb * o2) + cn * (lap + wzz) - cdt * ((pkp - pp[0]) * idzt);
+            if constexpr (ZO == 6) {
+                h = -con - z[2] - um * wx_;
+                qw = w0 + A.dt * (A.ra * h + A.rb * o2) + cn * lap + A.rc * z[5];
+            } else {
+                const R wkp = k + 1 == nz - 1 ? R(0) : nxt[(Tl::OW + jj + 3) * S + xl];
+                const R pkp = nxt[(Tl::OP + jj + 1) * S + xl];
+                const R wwz = (sq(R(0.5) * (w0 + wkp)) - sq(R(0.5) * (w0 + wkm))) * idzt;
+                const R wzz = ((wkp - w0) * A.lev[LV_IDZ * nz + k + 1] - (w0 - wkm) * idz) * idzt;
+                h = -con - wwz - um * wx_;
+                if (A.isscalar) h += A.got * (zface(tkp, tk, lt) - A.t_ref);
+                qw = w0 + A.dt * (A.ra * h + A.rb * o2) + cn * (lap + wzz) - cdt * ((pkp - pp[0]) * idzt);
+            }
         }
         A.hh[c] = h;
         reinterpret_cast<R *>(A.s2)[c] = qw;
@@ -270,9 +293,9 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
                 con += dif4<2>(F[-2 * S], F[-S], F[0], F[S]) * A.c24y;
                 lap += (-pu[2 * S] + R(16.0) * pu[S] - R(30.0) * u0 + R(16.0) * pu[-S] - pu[-2 * S]) * A.c12y2;
             }
-            const R uwz = (fuw - fuw_km) * idz;
             const R ukp = top ? (A.ochannel == 0 ? -u0 - R(2.0) * um : u0) : qu_[0];
-            const R uzz = ((ukp - u0) * idzt - (u0 - ukm) * idzb) * idz;
+            const R uwz = ZO == 6 ? z[0] : (fuw - fuw_km) * idz;
+            const R uzz = ZO == 6 ? z[3] : ((ukp - u0) * idzt - (u0 - ukm) * idzb) * idz;
             if (A.dp_opt == 3) {
                 const R x0 = mid4<CDS>(pv[-1], v0, pv[1], pv[2]), x1 = mid4<CDS>(pv[-S - 1], pv[-S], pv[-S + 1], pv[-S + 2]);
                 f = -con - uwz - um * ux + A.fc * (R(0.5) * (x0 + x1) - A.vg);
@@ -307,9 +330,9 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
             }
             lap += CDS == 1 ? (pv[1] - R(2.0) * v0 + pv[-1]) * A.idx2
                             : (-pv[2] + R(16.0) * pv[1] - R(30.0) * v0 + R(16.0) * pv[-1] - pv[-2]) * A.c12x2;
-            const R vwz = (fwv - fwv_km) * idz;
             const R vkp = top ? (A.ochannel == 0 ? -v0 : v0) : qv_[0];
-            const R vzz = ((vkp - v0) * idzt - (v0 - vkm) * idzb) * idz;
+            const R vwz = ZO == 6 ? z[1] : (fwv - fwv_km) * idz;
+            const R vzz = ZO == 6 ? z[4] : ((vkp - v0) * idzt - (v0 - vkm) * idzb) * idz;
             g = -con - vwz - um * vx;
             if (A.dp_opt == 3) {
                 const R a0 = mid4<CDS>(pu[-S], u0, pu[S], pu[2 * S]), a1 = mid4<CDS>(pu[-S - 1], pu[-1], pu[S - 1], pu[2 * S - 1]);
@@ -325,6 +348,7 @@ __global__ __launch_bounds__(TX * TY, sizeof(R) == 8 ? 3 : 4) void k_rhs_mom_mar
         tk = tkp;
         if (!more) break;
         __syncthreads();
-        if (ahead) put(raw[b], pre);
+        if (ahead) put(raw[ZO == 6 ? 0 : b], pre);
+        if (ZO == 6) __syncthreads();
     }
 }

@@ -1,11 +1,81 @@
 // Momentum right-hand side of the FD substep (get_momentum_cnvdiff,
 // src/module_cnvdiff.f90:35-374) fused with the x-direction R2C of qu, qv,
 // qw: marching tiles (hc_march.h), whole rows fused with the x transform
-// (short rows and FP32), the sponge's tiles and edge points, the
-// global-memory kernel of the 6th-order z operators, and the Rayleigh damping
-// means.
+// (short rows and FP32), the sponge's tiles and edge points, the FP32 kernels
+// of rows beyond 256 and of the 6th-order z operators, and the Rayleigh
+// damping means.
 #include "hc_host.h"
 #include "hc_march.h"
+
+// Momentum RHS + x R2C of qu,qv,qw.  Block: full rows j0..j0+TY-1 of level
+// k, one point per thread; every row the stencils reach is staged in LDS
+// once (coalesced), then the same LDS holds the q rows for the FFT.  FP32 rows
+// beyond 256 only: p of the mixed variant, solved from FP32 sources, moves by
+// 1e-4 when a source is rounded differently, so its arithmetic stays.
+template <int NX>
+constexpr int rhs_ty()
+{
+    return NX == 16 ? 16 : NX == 32 ? 32 : NX == 64 ? 16 : NX == 128 ? 8 : NX == 192 ? 4 : NX == 256 ? 4 : 1;
+}
+
+template <int NX>
+constexpr int rhs_threads() { return NX * rhs_ty<NX>() <= 512 ? NX * rhs_ty<NX>() : NX * rhs_ty<NX>() / 2; }
+
+template <int CDS, int NX, class R>
+__global__ __launch_bounds__(rhs_threads<NX>()) void k_rhs_mom(StepArgsT<R> A)
+{
+    using C = cplx<R>;
+    constexpr int TY = rhs_ty<NX>();
+    constexpr int T = rhs_threads<NX>(), PP = NX * TY / T, NL = NX / 2;
+    using Tl = RhsTile<NX, TY>;
+    static_assert(Tl::NROWS * NX >= 3 * TY * NX, "FFT rows must fit in the staging area");
+    __shared__ __align__(16) R sm[Tl::NROWS * NX];
+    const int tid = threadIdx.x;
+    const int nty = A.ny / TY;
+    const int logical = xcd_remap(blockIdx.x, nty * A.nlev);
+    const int jt = logical % nty, k = A.klo + logical / nty, j0 = jt * TY;
+    for (int q = tid; q < Tl::NROWS * NX; q += T) {
+        int r = q / NX, i = q - r * NX;
+        sm[q] = rhs_stage_value<NX, TY>(A, r, i, j0, k);
+    }
+    const R dpx = A.dp_opt == 2 ? R(A.scal[0]) : A.dpx;
+    PointVals<R> pv[PP];
+#pragma unroll
+    for (int pp = 0; pp < PP; ++pp) {
+        const int pt = tid + pp * T;
+        pv[pp].load(A, pt % NX, j0 + pt / NX, k);
+    }
+    __syncthreads();
+    R qs[PP][3];
+#pragma unroll
+    for (int pp = 0; pp < PP; ++pp) {
+        const int pt = tid + pp * T, i = pt % NX, jj = pt / NX, j = j0 + jj;
+        Ld<NX, TY, R> q(A, sm, i, jj, j, k, pv[pp]);
+        R f, g, h;
+        momentum_point<CDS>(q, dpx, f, g, h, qs[pp][0], qs[pp][1], qs[pp][2]);
+        const size_t c = ((size_t)k * A.ny + j) * NX + i;
+        A.ff[c] = f;
+        A.gg[c] = g;
+        A.hh[c] = h;
+    }
+    __syncthreads();  // staging no longer read: reuse it for the q rows
+#pragma unroll
+    for (int pp = 0; pp < PP; ++pp) {
+        const int pt = tid + pp * T, i = pt % NX, jj = pt / NX;
+        sm[(0 * TY + jj) * NX + i] = qs[pp][0];
+        sm[(1 * TY + jj) * NX + i] = qs[pp][1];
+        sm[(2 * TY + jj) * NX + i] = qs[pp][2];
+    }
+    __syncthreads();
+    C *sq_ = reinterpret_cast<C *>(sm);
+    lds_fft<NL, 3 * TY, NL, 1, T, -1>(sq_, A.tw_nl, tid);
+    C *outs[3] = {A.s0, A.s1, A.s2};
+    for (int p = tid; p < 3 * TY * NL; p += T) {
+        int row = p / NL, l = p - row * NL, fi = row / TY, r = row - fi * TY;
+        outs[fi][((size_t)k * A.ny + j0 + r) * NL + l] = r2c_post<NL>(sq_ + row * NL, l, A.tw_nx, A.norm);
+    }
+}
+
 
 template <int CDS, int NX, class R>
 __global__ __launch_bounds__(rhs2_threads<NX>(), (rhs2_waves<NX, R>())) void k_rhs_mom2(StepArgsT<R> A)
@@ -338,7 +408,7 @@ __global__ __launch_bounds__(256) void k_rhs_mom_edge(StepArgs A)
     PtD q(A, i, j, k);
     double f, g, h, qu, qv, qw;
     const double dpx = A.dp_opt == 2 ? A.scal[0] : A.dpx;
-    momentum_point<CDS, 2>(q, dpx, f, g, h, qu, qv, qw);
+    momentum_point<CDS>(q, dpx, f, g, h, qu, qv, qw);
     const size_t c = ((size_t)k * ny + j) * nx + i;
     A.ff[c] = f;
     A.gg[c] = g;
@@ -359,17 +429,18 @@ bool rhs_xt_fits(int shape, int nx, int ny)
 
 // Tile shape of the marching kernel, 0 for whole rows fused with the x
 // transform.  Without a choice by the caller: FP64 rows of 96 and more march
-// (whole rows hold one block of 1024 threads and 158 KB per CU), as do rows
-// beyond 256, which do not fit a block.  Shorter rows stay fused (64x64x65:
-// 23.0 us against 23.4 in two launches), and so do FP32 rows up to 256: two
-// blocks per CU and no rows through HBM, 0.312 ms at 256x256x257 against
-// 0.342 for the best tile.  Every length from 96 on is a multiple of 32 and
-// ny of 16, so 32x8 divides the grid.
+// (whole rows hold one block of 1024 threads and 158 KB per CU, and rows
+// beyond 256 do not fit a block).  Shorter rows stay fused (64x64x65: 23.0 us
+// against 23.4 in two launches).  FP32 rows keep their kernels: up to 256 two
+// blocks share a CU and no rows go through HBM, 0.312 ms at 256x256x257
+// against 0.342 for the best tile; beyond, the tiles would change p by more
+// than FP32 rounding explains (see k_rhs_mom).  Every length from 96 on is a
+// multiple of 32 and ny of 16, so 32x8 divides the grid.
 template <class R>
 static int march_shape(const hc_ctx *c)
 {
     if (rhs_xt_fits(c->tune.rhs_xt, c->nx, c->ny)) return c->tune.rhs_xt;
-    return c->nx > 256 || (sizeof(R) == 8 && c->nx >= 96) ? 1 : 0;
+    return sizeof(R) == 8 && c->nx >= 96 ? 1 : 0;
 }
 // Levels of one block's run.  A run costs two levels' loads more than it
 // forms, so about 12 levels and more; but at least three blocks per CU (what
@@ -383,7 +454,8 @@ static int march_levels(int ntile, int nlev, int ncu)
 }
 
 // Momentum RHS + x R2C of qu,qv,qw through a global-memory accessor: PtD in
-// a damped substep, Pt with the 6th-order z operators (ZO = 6).  Block:
+// a damped substep (sponge levels of grids that no tile divides), PtT<float>
+// with the 6th-order z operators (ZO = 6) in the mixed variant.  Block:
 // rows_per_block full rows of level k.
 template <int CDS, int NX, class Acc = PtD, int ZO = 2>
 __global__ __launch_bounds__(kRhsThreads) void k_rhs_mom_damped(StepArgsT<typename Acc::Real> A)
@@ -520,15 +592,34 @@ int rhs_momentum(hc_ctx *c, const StepArgs &A, StepArgsT<R> &B)
             }
         }
     }
-    if (z6 && !damp) {  // 6th/4th-order z operators: the global-memory point kernel
-        B.dmask = 0;
+    if (z6) {  // 6th/4th-order z operators (no damping): z terms per column, then the tiles
         zinterp6<R>(c, B);
-        const dim3 grow((c->ny + rows - 1) / rows, c->nz);
+        if constexpr (sizeof(R) == 4) {
+            // mixed: the point kernel, whose rounding p depends on
+            B.dmask = 0;
+            const dim3 grow((c->ny + rows - 1) / rows, c->nz);
 #define HC_RHSZ(NX_)                                                                                                   \
     if (P.cds == 1) hipLaunchKernelGGL((k_rhs_mom_damped<1, NX_, PtT<R>, 6>), grow, dim3(kRhsThreads), 0, c->stream, B); \
     else hipLaunchKernelGGL((k_rhs_mom_damped<2, NX_, PtT<R>, 6>), grow, dim3(kRhsThreads), 0, c->stream, B);
-        HC_DISPATCH_N(c->nx, HC_RHSZ)
+            HC_DISPATCH_N(c->nx, HC_RHSZ)
 #undef HC_RHSZ
+            return 0;
+        } else {
+        z6_terms<R>(c, B, 0);
+        // 32x8 tiles, 16x16 for the lengths that 32 does not divide
+        const bool wide = c->nx % 32 == 0;
+        const int ntile = c->nx * c->ny / 256;
+        B.kchunk = march_levels(ntile, c->nz, c->ncu);
+        const dim3 g((unsigned)(ntile * ((c->nz + B.kchunk - 1) / B.kchunk)));
+#define HC_Z6(CDS_, TX_, TY_) hipLaunchKernelGGL((k_rhs_mom_march<CDS_, TX_, TY_, R, 6>), g, dim3(256), 0, c->stream, B);
+        if (P.cds == 1) { if (wide) { HC_Z6(1, 32, 8) } else { HC_Z6(1, 16, 16) } }
+        else { if (wide) { HC_Z6(2, 32, 8) } else { HC_Z6(2, 16, 16) } }
+#undef HC_Z6
+        const R *src[3] = {reinterpret_cast<const R *>(B.s0), reinterpret_cast<const R *>(B.s1),
+                           reinterpret_cast<const R *>(B.s2)};
+        cplx<R> *dst[3] = {B.s0, B.s1, B.s2};
+        if (int e = launch_r2c_n<R>(c, 3, src, dst)) return e;
+        }
     }
     int err = 0;
     if (!z6 && ksplit > 0) {
@@ -560,6 +651,12 @@ int rhs_momentum(hc_ctx *c, const StepArgs &A, StepArgsT<R> &B)
         constexpr int T_ = rhs2_threads<NX_>();                                                          \
         if (P.cds == 1) hipLaunchKernelGGL((k_rhs_mom2<1, NX_, R>), g1, dim3(T_), 0, c->stream, B);      \
         else hipLaunchKernelGGL((k_rhs_mom2<2, NX_, R>), g1, dim3(T_), 0, c->stream, B);                 \
+    } else if constexpr (sizeof(R) == 4) {                                                               \
+        constexpr int TY_ = rhs_ty<NX_>();                                                               \
+        dim3 g1((unsigned)(c->ny / TY_ * ksplit));                                                       \
+        constexpr int T_ = rhs_threads<NX_>();                                                           \
+        if (P.cds == 1) hipLaunchKernelGGL((k_rhs_mom<1, NX_, R>), g1, dim3(T_), 0, c->stream, B);       \
+        else hipLaunchKernelGGL((k_rhs_mom<2, NX_, R>), g1, dim3(T_), 0, c->stream, B);                  \
     }
             HC_DISPATCH_N(c->nx, HC_RHS)
 #undef HC_RHS

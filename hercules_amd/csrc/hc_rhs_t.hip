@@ -37,7 +37,7 @@ __global__ __launch_bounds__(kRhsThreads) void k_rhs_t(StepArgsT<typename Acc::R
 // j0..j0+TY-1 of level k; the t, u, v rows the stencils reach are staged in
 // LDS once (all loads issued before the first use), then the same LDS holds
 // the qt rows for the FFT.  Undamped substeps, nx <= 256.
-template <int CDS, int NX, class R>
+template <int CDS, int NX, class R, int ZO = 2>
 __global__ __launch_bounds__(rhs2_threads<NX>(), (rhs2_waves<NX, R>())) void k_rhs_t2(StepArgsT<R> A)
 {
     using C = cplx<R>;
@@ -86,7 +86,7 @@ __global__ __launch_bounds__(rhs2_threads<NX>(), (rhs2_waves<NX, R>())) void k_r
         q.w_k = wk;
         q.w_km = wkm;
         R s;
-        temperature_point<CDS>(q, s, qt, s0);
+        temperature_point<CDS, ZO>(q, s, qt, s0);
         A.ss[ck] = s;
     }
     __syncthreads();  // staging no longer read: reuse it for the qt rows
@@ -133,10 +133,18 @@ int rhs_temperature(hc_ctx *c, StepArgsT<R> &B)
     B.dmask = 16;  // t read damped, the updated velocities as they are
     if (z6) {
         B.dmask = 0;
+        if constexpr (sizeof(R) == 8) z6_terms<R>(c, B, 3);
         const dim3 grow((c->ny + rows - 1) / rows, c->nz);
-#define HC_RTZ(NX_)                                                                                                  \
-    if (P.cds == 1) hipLaunchKernelGGL((k_rhs_t<1, NX_, PtT<R>, 6>), grow, dim3(kRhsThreads), 0, c->stream, B);       \
-    else hipLaunchKernelGGL((k_rhs_t<2, NX_, PtT<R>, 6>), grow, dim3(kRhsThreads), 0, c->stream, B);
+#define HC_RTZ(NX_)                                                                                                   \
+    if constexpr (NX_ <= 256 && sizeof(R) == 8) {                                                                     \
+        dim3 g1((unsigned)(c->ny / rhs2_ty<NX_>() * c->nz));                                                          \
+        constexpr int T_ = rhs2_threads<NX_>();                                                                       \
+        if (P.cds == 1) hipLaunchKernelGGL((k_rhs_t2<1, NX_, R, 6>), g1, dim3(T_), 0, c->stream, B);                  \
+        else hipLaunchKernelGGL((k_rhs_t2<2, NX_, R, 6>), g1, dim3(T_), 0, c->stream, B);                             \
+    } else {                                                                                                          \
+        if (P.cds == 1) hipLaunchKernelGGL((k_rhs_t<1, NX_, PtT<R>, 6>), grow, dim3(kRhsThreads), 0, c->stream, B);   \
+        else hipLaunchKernelGGL((k_rhs_t<2, NX_, PtT<R>, 6>), grow, dim3(kRhsThreads), 0, c->stream, B);              \
+    }
         HC_DISPATCH_N(c->nx, HC_RTZ)
 #undef HC_RTZ
         return 0;

@@ -21,6 +21,16 @@ void zinterp6(hc_ctx *c, StepArgsT<R> &B)
 template void zinterp6<double>(hc_ctx *, StepArgsT<double> &);
 template void zinterp6<float>(hc_ctx *, StepArgsT<float> &);
 
+// z terms of the momentum (e0 = 0) or temperature (e0 = 3) right-hand side
+template <class R>
+void z6_terms(hc_ctx *c, const StepArgsT<R> &B, int e0)
+{
+    const dim3 grid((unsigned)(((size_t)B.nx * B.ny + 255) / 256), e0 == 3 ? 1 : 3, (unsigned)stream_chunks(B.nz));
+    if (c->prm.cds == 1) hipLaunchKernelGGL((k_z6_terms<1, R>), grid, dim3(256), 0, c->stream, B, e0);
+    else hipLaunchKernelGGL((k_z6_terms<2, R>), grid, dim3(256), 0, c->stream, B, e0);
+}
+template void z6_terms<double>(hc_ctx *, const StepArgsT<double> &, int);
+
 namespace {
 // right-hand sides in0/in1 (null: in place), solutions f0/f1
 template <class CI>

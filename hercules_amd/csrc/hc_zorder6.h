@@ -96,3 +96,154 @@ __global__ __launch_bounds__(256) void k_zinterp6(StepArgsT<R> A, R *fu, R *fv, 
         }
     }
 }
+
+// ---------------------------------------------------------------------------
+// z terms of the FD right-hand sides (get_momentum_cnvdiff,
+// get_temperature_cnvdiff with the 6th-order operators), once per point for
+// the tiles that add the horizontal ones (k_rhs_mom_march with ZO = 6, k_rhs_t2):
+//   e = 0, 1: d(uw)/dz, d2u/dz2 (of v) into ff, qu (gg, qv)
+//   e = 2:    d(ww)/dz - got (t - t_ref), and nu dt/2 d2w/dz2 - dt dp/dz over
+//             rc into hh, qw (levels below the top)
+//   e = 3:    d(tw)/dz, d2t/dz2 into ss, qt
+// One thread per (i, j) column, equation (e0 + blockIdx.y) and z chunk streams
+// along z with windows of kWin levels, as the spectral path's column kernels.
+// The fluxes through a face are formed once, where the accessors formed six
+// per point; a wall face carries none.
+// The window of a face quantity holds face kw at level kw; the band rows ZB_D
+// and ZB_F2 leave out the wall faces, ZB_C2_* the wall data, whose terms
+// zwall adds.
+template <class R>
+HC_DEV R zwall(const StepArgsT<R> &A, int op, int k, R bot, R top, bool has_top)
+{
+    const size_t e = (size_t)op * A.nz + k;
+    const int s = A.zst[e], jt = A.nz + 1 - s;
+    const double *w = A.zwt + e * kZW;
+    R v = R(0);
+    if (s == 0) v += R(w[0]) * bot;
+    if (has_top && jt < A.zn2) v += R(w[jt]) * top;
+    return v;
+}
+// NR stored values per level (load) become NW window entries (make)
+template <int NR, int NW, class R, class Load, class Make, class Row>
+HC_DEV void zterm_stream(int nrows, Load &&load, Make &&make, Row &&row)
+{
+    constexpr int PF = 3;
+    const int csz = (nrows + (int)gridDim.z - 1) / (int)gridDim.z;
+    const int kb = (int)blockIdx.z * csz, ke = min(kb + csz, nrows), ib = kb - kBandMax;
+    R win[NW][kWin], ring[PF][NR];
+#pragma unroll
+    for (int f = 0; f < NW; ++f)
+#pragma unroll
+        for (int t = 0; t < kWin; ++t) win[f][t] = R(0);
+#pragma unroll
+    for (int u = 0; u < PF; ++u) load(ib + u, ring[u]);
+    for (int i0 = ib; i0 < ke + kBandMax; i0 += PF) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+            const int i = i0 + u;
+            R in[NW];
+            make(i, ring[u], in);
+#pragma unroll
+            for (int f = 0; f < NW; ++f) {
+#pragma unroll
+                for (int t = 0; t < kWin - 1; ++t) win[f][t] = win[f][t + 1];
+                win[f][kWin - 1] = in[f];
+            }
+            load(i + PF, ring[u]);
+            const int k = i - kBandMax;
+            if (k >= kb && k < ke) row(k, win);
+        }
+    }
+}
+template <class R>
+HC_DEV R zdot(const StepArgsT<R> &A, int band, int k, const R (&x)[kWin])
+{
+    const double *b = A.zband + ((size_t)band * A.nz + k) * kBandRow;
+    R acc = R(0);
+#pragma unroll
+    for (int t = 0; t < kWin; ++t) acc += R(b[t]) * x[t];
+    return acc;
+}
+
+template <int CDS, class R>
+__global__ __launch_bounds__(256) void k_z6_terms(StepArgsT<R> A, int e0)
+{
+    const int nx = A.nx, ny = A.ny, nz = A.nz, e = e0 + (int)blockIdx.y;
+    const size_t plane = (size_t)nx * ny, col = blockIdx.x * (size_t)256 + threadIdx.x;
+    if (col >= plane) return;
+    const int j = (int)(col / nx), i = (int)(col - (size_t)j * nx);
+    if (e < 2) {
+        // neighbours of w across x (u) or y (v): the face interpolant whx, why
+        const R *f = e == 0 ? A.u : A.v, *zf = e == 0 ? A.zfu : A.zfv;
+        R *conv = e == 0 ? A.ff : A.gg, *dif = reinterpret_cast<R *>(e == 0 ? A.s0 : A.s1);
+        size_t o[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+            o[d] = e == 0 ? (size_t)j * nx + wrapi(i + d - 1, nx) : (size_t)wrapi(j + d - 1, ny) * nx + i;
+        const R wall = e == 0 ? R(-A.u_mrf) : R(0);
+        const int op = A.ochannel ? ZO_C2_DN : ZO_C2_DD, band = A.ochannel ? ZB_C2_DN : ZB_C2_DD;
+        zterm_stream<6, 2, R>(nz,
+            [&](int li, R (&v)[6]) __attribute__((always_inline)) {
+                const int lc = min(max(li, 0), nz - 1);
+                const size_t b = (size_t)lc * plane;
+                v[0] = f[b + col];
+                v[1] = zf[b + col];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) v[2 + d] = A.w[b + o[d]];
+            },
+            [&](int li, const R (&v)[6], R (&in)[2]) __attribute__((always_inline)) {
+                in[0] = li >= 0 && li < nz ? v[0] : R(0);
+                const R wh = CDS == 1 ? R(0.5) * (v[4] + v[3])
+                                      : (-v[5] + R(9.0) * v[4] + R(9.0) * v[3] - v[2]) / R(16.0);
+                in[1] = li >= 0 && li < nz - 1 ? v[1] * wh : R(0);
+            },
+            [&](int k, const R (&win)[2][kWin]) __attribute__((always_inline)) {
+                const size_t c = (size_t)k * plane + col;
+                conv[c] = zdot(A, ZB_D, k, win[1]);
+                dif[c] = zdot(A, band, k, win[0]) + zwall<R>(A, op, k, wall, wall, A.ochannel == 0);
+            });
+    } else if (e == 2) {
+        R *qw = reinterpret_cast<R *>(A.s2);
+        const R cn = R(0.5) * A.dt * A.nu;
+        zterm_stream<3, 3, R>(nz - 1,
+            [&](int li, R (&v)[3]) __attribute__((always_inline)) {
+                const size_t b = (size_t)min(max(li, 0), nz - 1) * plane + col;
+                v[0] = A.w[b];
+                v[1] = A.p[b];
+                v[2] = A.zcw[b];
+            },
+            [&](int li, const R (&v)[3], R (&in)[3]) __attribute__((always_inline)) {
+                const bool on = li >= 0 && li < nz;
+                in[0] = on && li < nz - 1 ? v[0] : R(0);
+                in[1] = on ? v[1] : R(0);
+                in[2] = on ? sq(v[2]) : R(0);
+            },
+            [&](int k, const R (&win)[3][kWin]) __attribute__((always_inline)) {
+                const size_t c = (size_t)k * plane + col;
+                R con = zdot(A, ZB_G, k, win[2]);
+                if (A.isscalar) con -= A.got * (A.zft[c] - A.t_ref);
+                A.hh[c] = con;
+                qw[c] = cn * zdot(A, ZB_F2, k, win[0]) - A.dt * zdot(A, ZB_G, k, win[1]);
+            });
+    } else {
+        R *qt = reinterpret_cast<R *>(A.s0);
+        const R top = A.tbc_top ? R(A.gdz_top * A.lev[LV_IDZT * nz + nz - 1]) : A.ttop;
+        const int op = A.tbc_top ? ZO_C2_DN : ZO_C2_DD, band = A.tbc_top ? ZB_C2_DN : ZB_C2_DD;
+        zterm_stream<3, 2, R>(nz,
+            [&](int li, R (&v)[3]) __attribute__((always_inline)) {
+                const size_t b = (size_t)min(max(li, 0), nz - 1) * plane + col;
+                v[0] = A.t[b];
+                v[1] = A.zft[b];
+                v[2] = A.w[b];
+            },
+            [&](int li, const R (&v)[3], R (&in)[2]) __attribute__((always_inline)) {
+                in[0] = li >= 0 && li < nz ? v[0] : R(0);
+                in[1] = li >= 0 && li < nz - 1 ? v[1] * v[2] : R(0);
+            },
+            [&](int k, const R (&win)[2][kWin]) __attribute__((always_inline)) {
+                const size_t c = (size_t)k * plane + col;
+                A.ss[c] = zdot(A, ZB_D, k, win[1]);
+                qt[c] = zdot(A, band, k, win[0]) + zwall<R>(A, op, k, A.tbot, top, true);
+            });
+    }
+}

@@ -220,3 +220,29 @@ def test_z6_other_flags_stay_divergence_free(kw):
     scale = np.abs(u).max() / (prm.lz / prm.nz)
     assert dmax < 1e-12 * scale, dmax
     ch.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz,kw", [
+    (32, 32, 16, {}),                        # one 32x8 tile wide, the fewest levels
+    (96, 16, 37, {"cds": 1}),                # runs of unequal length
+    (48, 16, 20, {"zorder": 4}),             # 16x16 tiles, three across
+    (384, 16, 17, {"tbc_top": 1, "dtdz_top": 0.5}),  # rows beyond 256: temperature through the accessor
+])
+def test_z6_tiles_match_torch_reference(nx, ny, nz, kw):
+    """Momentum and temperature right-hand sides of the 6th- and 4th-order z
+    operators on tiles wider than one, with the z terms of k_z6_terms;
+    tolerances as for the steps above."""
+    prm = cases.stratified_open_channel(nx=nx, ny=ny, nz=nz, **{"wall_rows": 1, "zorder": 6, "nu": 1.0 / 180.0,
+                                                                "dt": 5e-4, **kw})
+    st = cases.loglaw_noise(prm, seed=8)
+    ref = TorchChannel(prm).steps({k: torch.tensor(v) for k, v in st.items()}, 1)
+    ch = Channel(prm)
+    for k, v in st.items():
+        ch.set_field(k, v)
+    ch.init()
+    ch.steps(1)
+    for n in ["u", "v", "w", "p", "t"]:
+        err = rel_l2(ch.get_field(n), ref[n].numpy())
+        print(nx, ny, nz, kw, n, f"{err:.2e}")
+        assert err < (1e-9 if n == "p" else 1e-11), (n, err)
+    ch.close()
