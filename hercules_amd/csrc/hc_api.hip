@@ -481,8 +481,9 @@ static bool build_zops(hc_ctx *c)
     // (data index = w level + 1, nz - 1 unknowns), P on the levels.
     c->h_zband.assign((size_t)ZB_COUNT * nz * kBandRow, 0.0);
     const int bops[ZB_COUNT] = {ZO_C2_DD, ZO_C2_DN, ZO_F2, ZO_P, ZO_G, ZO_D, ZO_I_DD, ZO_I_DN, ZO_IFC};
-    // half bands the solver is instantiated for (5 and 7); the explicit G and D
-    // are applied over the full stored band, the interpolations over kIntHW
+    // half bands of the solver's first and last two rows (5 and 7; two less
+    // between); the explicit G and D are applied over the full stored band,
+    // the interpolations over kIntHW
     const int bhalf[ZB_COUNT] = {5, 5, 5, 7, kBandMax, kBandMax, kIntHW, kIntHW, kIntHW};
     for (int b = 0; b < ZB_COUNT; ++b) {
         const int op = bops[b];
@@ -501,7 +502,8 @@ static bool build_zops(hc_ctx *c)
                 const int lv = c->h_zst[e] + j - off;
                 if (w == 0.0 || lv < lo || lv > hi) continue;
                 const int d = lv - k;
-                if (d < -bhalf[b] || d > bhalf[b]) return false;
+                const int half = bhalf[b] - (b <= 3 && k >= 2 && k < nrow - 2 ? 2 : 0);
+                if (d < -half || d > half) return false;
                 c->h_zband[((size_t)b * nz + k) * kBandRow + kBandMax + d] += w;
             }
         }

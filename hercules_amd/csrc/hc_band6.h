@@ -6,20 +6,23 @@
 //   w:        (1 - rc hxy) I - rc kappa Z      Z = ZO_F2 on the interior faces
 //   p:        rc (hxy I + ZO_P)                ZO_P = ZO_D o ZO_G
 // and differs between columns only through the horizontal symbol hxy.  Z has
-// half band 5 (7-point stencils, shifted inwards at the walls) and ZO_P half
-// band 7.  Gaussian elimination without pivoting is stable for all of them
-// (growth factor below 1.7 on the channel grids), so each thread factors its
-// column's matrix row by row while eliminating the right-hand sides:
-//   forward  k = 0..n-1: row k of the matrix from the band table, eliminated
-//            against the previous PB rows of U kept in registers; U's row
-//            (PB entries right of the diagonal and 1/diagonal) goes to a
-//            scratch array, the eliminated right-hand side back in place;
-//   backward k = n-1..0: x(k) from U's row and the PB values of x above it.
+// half band 3 (7-point stencils) but for the first and last two rows, whose
+// stencils shift inwards at the walls and reach 5; ZO_P half band 5, and 7 in
+// those rows.  Gaussian elimination without pivoting is stable for all of
+// them (growth factor below 1.7 on the channel grids), so each thread factors
+// its column's matrix row by row while eliminating the right-hand sides.
+// U's rows (half band and 1/diagonal) and the eliminated right-hand sides of
+// a whole column are more bytes than the right-hand sides themselves, so they
+// are not kept: the levels are cut into the first PB, a remainder and segments
+// of kBandSeg,
+//   pass 1  eliminates from the bottom and keeps, at each segment's start,
+//           the rows that the next one depends on (scratch, scr),
+//   pass 2  takes the segments from the top: eliminates one again from its
+//           start, its rows of U into LDS, and back-substitutes through it.
 // Consecutive threads own consecutive l, so every load and store of a level
 // is one coalesced line across the wavefront.  The (0,0) mode adds the wall
 // data of u and t to the first right-hand side (the Crank-Nicolson implicit
-// half) and replaces the first pressure row by the delnull row, as the
-// iterative solves did.
+// half) and replaces the first pressure row by the delnull row.
 #pragma once
 
 
@@ -29,7 +32,7 @@ template <class CI>
 struct BandSys {
     const CI *in[2];  // right-hand sides (k, j, l)
     CI *f[2];         // solutions (may be in[]); hold the eliminated right-hand sides in between
-    double *scr;    // U rows: PB + 1 doubles per level and column, level-major
+    double *scr;    // segment starts: PI (PI + 1 + 2 nr) doubles per segment and column
     int nr;         // right-hand sides sharing the matrix: 1 or 2
     int eq;         // 0 u/v, 1 w, 2 p, 3 t
     int fix;        // apply the (0,0)-mode wall data / delnull row
@@ -68,14 +71,35 @@ HC_DEV double z6_wall_rhs(const StepArgs &A, int eq, int op, double ck, int k)
     return v;
 }
 
-template <int PB, class CI>
-__global__ __launch_bounds__(256) void k_z6_band(StepArgs A, BandArgs<CI> B)
+constexpr int kBandSeg = 12;  // levels of a segment
+// bytes of LDS of one block (one wavefront): the rows of a segment, the four
+// entries of the first two rows beyond the half band, the segment's band rows
+template <int PI>
+constexpr size_t band_lds(int nr)
 {
-    const BandSys<CI> S = B.s[blockIdx.y];
-    const int nl = A.nl, ny = A.ny, nz = A.nz;
+    return (size_t)((kBandSeg * (PI + 1 + 2 * nr) + 4) + (kBandSeg * (2 * PI + 1) + 63) / 64) * 64 * sizeof(double);
+}
+
+// PI: half band of all rows but the first and last two, whose band is PI + 2.
+// NR: right-hand sides.  A launch has about one wavefront per SIMD (33,024
+// columns at 256x256), so the loads in flight carry the rate: the elimination
+// of a segment is straight-line code that loads the next one's right-hand
+// sides and band rows as it goes, without a branch around a load, after which
+// a wait would be for all of them.  12 levels: U's rows of three blocks fill a
+// CU's LDS.  The solves of one step at 256x256x257 (three substeps, u, v, w,
+// t, p): 5.5 ms with U kept in memory, 4.9 ms with loads behind branches, 2.0
+// ms so (FP32 spectra 4.7 -> 1.6 ms).
+template <int PI, int NR, class CI>
+HC_DEV void band_solve(const StepArgs &A, const BandSys<CI> &S)
+{
+    constexpr int PB = PI + 2, SG = kBandSeg, NS = PI * (PI + 1 + 2 * NR), NL_ = PI + 1 + 2 * NR;
+    constexpr int W = 2 * PI + 1, TQ = (SG * W + 63) / 64;
+    static_assert(SG >= 9);  // the last two rows' stencils stay within the top segment
+    extern __shared__ double band_sm[];
+    const int lane = threadIdx.x, nl = A.nl, ny = A.ny, nz = A.nz;
     const int ncol = nl * ny;
-    const int col = blockIdx.x * 256 + threadIdx.x;
-    if (col >= ncol) return;
+    // lanes beyond the last column repeat it (same wavefront, same values)
+    const int col = min((int)blockIdx.x * 64 + lane, ncol - 1);
     const int l = col % nl, jm = col / nl;
     const size_t plane = (size_t)ncol;
     const bool face = S.eq == 1, pres = S.eq == 2;
@@ -111,154 +135,335 @@ __global__ __launch_bounds__(256) void k_z6_band(StepArgs A, BandArgs<CI> B)
     const double rc = A.rc, ck = rc * kap;
     const double cdiag = pres ? rc * hxy : 1.0 - rc * hxy, coff = pres ? rc : -ck;
     const bool is00 = S.fix && l == 0 && jm == 0;
+    const bool walls = is00 && (S.eq == 0 || S.eq == 3);
     const double *bt = A.zband + (size_t)band * nz * kBandRow + kBandMax;
-    const int nr = S.nr;
-    double U[PB][PB], dv[PB];
-    double2 y[2][PB];
+    // rows 0 .. PB-1, then nrem, then nfull segments.  n >= 15 (16 for p), so
+    // the top one, of SG or (nfull = 0) nrem rows, has PB + 2 and more.
+    const int nfull = (n - PB) / SG, nrem = n - PB - nfull * SG;
+    // LDS: row i of the segment, entry e (U's PI, 1/diagonal, the right-hand
+    // sides), and the two entries beyond PI of rows 0 and 1
+    auto row = [&](int i, int e) -> double & { return band_sm[(4 + i * NL_ + e) * 64 + lane]; };
+    auto wide = [&](int k, int e) -> double & { return band_sm[(2 * k + e) * 64 + lane]; };
+    double *tab = band_sm + (4 + SG * NL_) * 64;
+    // Every row is rounded as the elimination over the full band rounds it, so
+    // that segments of any position agree to the last bit: an entry is the
+    // product coff w (the diagonal fma(coff, w, cdiag)), rounded unless its
+    // first update is not zero, which takes the product unrounded.
+    auto prod = [](double x, double y) -> double {
+#pragma clang fp contract(off)
+        return x * y;
+    };
+    auto entry = [&](double w, int d) -> double { return d ? prod(coff, w) : fma(coff, w, cdiag); };
+    // band rows of the segment at k0: loaded a segment ahead, then through LDS
+    double tq[TQ];
+    auto tab_load = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < PB; ++t) {
-        dv[t] = 0.0;
-        y[0][t] = y[1][t] = make_double2(0.0, 0.0);
-#pragma unroll
-        for (int c = 0; c < PB; ++c) U[t][c] = 0.0;
-    }
-    // The right-hand sides (forward) and the U rows with the partial
-    // solutions (backward) of level k are loaded PF levels ahead into rings
-    // indexed by the unrolled loop position, in the stored type, so that a
-    // column's chain of levels waits less on its loads (a launch has about
-    // one wavefront per SIMD).  With FP64 spectra the kernel moves its bytes
-    // near the HBM rate already, and the one-level ring keeps its registers
-    // (two wavefronts per SIMD); FP32 spectra take four levels.
-    constexpr int PF = sizeof(CI) == 8 ? (PB >= 7 ? 2 : 4) : 1;
-    const CI zero = czero_t<CI>();
-    CI rq[PF][2];
-#pragma unroll
-    for (int u = 0; u < PF; ++u) {
-        const size_t o = (size_t)u * plane + col;
-        rq[u][0] = u < n ? S.in[0][o] : zero;
-        rq[u][1] = (u < n && nr > 1) ? S.in[1][o] : zero;
-    }
-    // ---- forward elimination
-    for (int k0 = 0; k0 < n; k0 += PF) {
-#pragma unroll
-      for (int u = 0; u < PF; ++u) {
-        const int k = k0 + u;
-        if (k >= n) break;
-        double a[2 * PB + 1];
-#pragma unroll
-        for (int d = -PB; d <= PB; ++d) a[d + PB] = coff * bt[(size_t)k * kBandRow + d];
-        a[PB] += cdiag;
-        const size_t o = (size_t)k * plane + col;
-        double2 r[2];
-        r[0] = ccast<double2>(rq[u][0]);
-        r[1] = ccast<double2>(rq[u][1]);
-        if (k + PF < n) {
-            const size_t on = (size_t)(k + PF) * plane + col;
-            rq[u][0] = S.in[0][on];
-            if (nr > 1) rq[u][1] = S.in[1][on];
+        for (int j = 0; j < TQ; ++j) {
+            const int e = lane + 64 * j;
+            tq[j] = bt[min(k0 + e / W, nz - 1) * kBandRow + e % W - PI];
         }
-        if (is00) {
-            if (pres) {
-                if (k == 0) {  // delnull: b0 phi(0) = 0 (src/module_poisson_solver.f90:558-564)
+    };
+    auto tab_put = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                    for (int d = 0; d <= 2 * PB; ++d) a[d] = 0.0;
-                    a[PB] = rc * (hxy + A.lev[LV_DP00 * nz]);
-                    r[0] = make_double2(0.0, 0.0);
-                }
-            } else if (S.eq == 0 || S.eq == 3) {
-                r[0].x += z6_wall_rhs(A, S.eq, op, ck, k);
+        for (int j = 0; j < TQ; ++j) tab[lane + 64 * j] = tq[j];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    // the PI rows before the current one, oldest first
+    struct Win {
+        double U[PI][PI], dv[PI];
+        double2 y[NR][PI];
+    };
+    Win w;
+    CI ring[SG][NR];
+    auto load_rhs = [&](int k, CI (&r)[NR]) __attribute__((always_inline)) {
+        const size_t o = (size_t)min(k, n - 1) * plane + col;
+#pragma unroll
+        for (int e = 0; e < NR; ++e) r[e] = S.in[e][o];
+    };
+    auto fill = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < SG; ++u) load_rhs(k0 + u, ring[u]);
+    };
+    auto keep = [&](int i, const double (&u)[PI], double dk, const double2 (&r)[NR]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < PI; ++c) row(i, c) = u[c];
+        row(i, PI) = dk;
+#pragma unroll
+        for (int e = 0; e < NR; ++e) { row(i, PI + 1 + 2 * e) = r[e].x; row(i, PI + 2 + 2 * e) = r[e].y; }
+    };
+    // rows 0 .. PB-1 from ring with the full band: rows 0 and 1 reach PB to the right
+    auto bottom = [&](bool store) __attribute__((always_inline)) {
+        double U[PB][PB], dv[PB];
+        double2 y[NR][PB];
+#pragma unroll
+        for (int t = 0; t < PB; ++t) {
+            dv[t] = 0.0;
+#pragma unroll
+            for (int e = 0; e < NR; ++e) y[e][t] = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int c = 0; c < PB; ++c) U[t][c] = 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < PB; ++k) {
+            double a[2 * PB + 1];
+#pragma unroll
+            for (int d = -PB; d <= PB; ++d) a[d + PB] = entry(bt[k * kBandRow + d], d);
+            double2 r[NR];
+#pragma unroll
+            for (int e = 0; e < NR; ++e) r[e] = ccast<double2>(ring[k][e]);
+            if (k < 3 && walls) r[0].x += z6_wall_rhs(A, S.eq, op, ck, k);
+            if (k == 0 && is00 && pres) {  // delnull: b0 phi(0) = 0 (src/module_poisson_solver.f90:558-564)
+#pragma unroll
+                for (int d = 0; d <= 2 * PB; ++d) a[d] = 0.0;
+                a[PB] = rc * (hxy + A.lev[LV_DP00 * nz]);
+                r[0] = make_double2(0.0, 0.0);
+            }
+#pragma unroll
+            for (int t = 0; t < PB; ++t) {
+                const double lt = a[t] * dv[t];
+#pragma unroll
+                for (int c = 1; c <= PB; ++c)
+                    if (c == PB && t > 0 && k > 0) a[t + PB] = fma(coff, bt[k * kBandRow + t], -prod(lt, U[t][PB - 1]));
+                    else a[t + c] -= lt * U[t][c - 1];
+#pragma unroll
+                for (int e = 0; e < NR; ++e) { r[e].x -= lt * y[e][t].x; r[e].y -= lt * y[e][t].y; }
+            }
+            const double dk = 1.0 / a[PB];
+#pragma unroll
+            for (int t = 0; t < PB - 1; ++t) {
+                dv[t] = dv[t + 1];
+#pragma unroll
+                for (int e = 0; e < NR; ++e) y[e][t] = y[e][t + 1];
+#pragma unroll
+                for (int c = 0; c < PB; ++c) U[t][c] = U[t + 1][c];
+            }
+            dv[PB - 1] = dk;
+#pragma unroll
+            for (int e = 0; e < NR; ++e) y[e][PB - 1] = r[e];
+#pragma unroll
+            for (int c = 0; c < PB; ++c) U[PB - 1][c] = a[PB + 1 + c];
+            if (store) {
+                double u[PI];
+#pragma unroll
+                for (int c = 0; c < PI; ++c) u[c] = a[PB + 1 + c];
+                keep(k, u, dk, r);
+                if (k < 2) { wide(k, 0) = a[PB + 1 + PI]; wide(k, 1) = a[PB + 2 + PI]; }
             }
         }
 #pragma unroll
-        for (int t = 0; t < PB; ++t) {
-            const double lt = a[t] * dv[t];
+        for (int t = 0; t < PI; ++t) {
+            w.dv[t] = dv[t + 2];
 #pragma unroll
-            for (int c = 1; c <= PB; ++c) a[t + c] -= lt * U[t][c - 1];
-            r[0].x -= lt * y[0][t].x;
-            r[0].y -= lt * y[0][t].y;
-            r[1].x -= lt * y[1][t].x;
-            r[1].y -= lt * y[1][t].y;
+            for (int e = 0; e < NR; ++e) w.y[e][t] = y[e][t + 2];
+#pragma unroll
+            for (int c = 0; c < PI; ++c) w.U[t][c] = U[t + 2][c];
         }
-        const double dk = 1.0 / a[PB];
-        double *srow = S.scr + (size_t)k * (PB + 1) * plane + col;
+    };
+    // row k, the i-th of its segment, from the right-hand sides q; into LDS if
+    // store; edge: one of the column's last three rows, tail: of its last two
+    auto step = [&](int k, int i, const CI (&q)[NR], bool store, bool edge, bool tail) __attribute__((always_inline)) {
+        double a[W];
 #pragma unroll
-        for (int c = 1; c <= PB; ++c) srow[(size_t)(c - 1) * plane] = a[PB + c];
-        srow[(size_t)PB * plane] = dk;
-        S.f[0][o] = ccast<CI>(r[0]);
-        if (nr > 1) S.f[1][o] = ccast<CI>(r[1]);
+        for (int d = -PI; d <= PI; ++d) a[d + PI] = entry(tab[i * W + d + PI], d);
+        double2 r[NR];
 #pragma unroll
-        for (int t = 0; t < PB - 1; ++t) {
-            dv[t] = dv[t + 1];
-            y[0][t] = y[0][t + 1];
-            y[1][t] = y[1][t + 1];
+        for (int e = 0; e < NR; ++e) r[e] = ccast<double2>(q[e]);
+        if (edge && walls) r[0].x += z6_wall_rhs(A, S.eq, op, ck, k);
+        if (tail) {  // these reach PB to the left: older rows of the segment from LDS
+            const double far = entry(bt[k * kBandRow - PB], -PB);
 #pragma unroll
-            for (int c = 0; c < PB; ++c) U[t][c] = U[t + 1][c];
+            for (int d = PB; d > PI; --d) {
+                double lt = far;
+                if (d == PB - 1) {
+                    const double lo = far * row(i - PB, PI);  // what the row before took from this entry
+                    lt = fma(coff, bt[k * kBandRow - d], -prod(lo, row(i - PB, 0)));
+                }
+                lt *= row(i - d, PI);
+#pragma unroll
+                for (int c = 1; c <= PI; ++c)
+                    if (c - d + PI >= 0) {
+                        if (d == PB) a[c - d + PI] = fma(coff, tab[i * W + c - d + PI], -prod(lt, row(i - d, c - 1)));
+                        else a[c - d + PI] -= lt * row(i - d, c - 1);
+                    }
+#pragma unroll
+                for (int e = 0; e < NR; ++e) {
+                    r[e].x -= lt * row(i - d, PI + 1 + 2 * e);
+                    r[e].y -= lt * row(i - d, PI + 2 + 2 * e);
+                }
+            }
         }
-        dv[PB - 1] = dk;
-        y[0][PB - 1] = r[0];
-        y[1][PB - 1] = r[1];
 #pragma unroll
-        for (int c = 0; c < PB; ++c) U[PB - 1][c] = a[PB + 1 + c];
-      }
+        for (int t = 0; t < PI; ++t) {
+            const double lt = a[t] * w.dv[t];
+#pragma unroll
+            for (int c = 1; c <= PI; ++c) a[t + c] -= lt * w.U[t][c - 1];
+#pragma unroll
+            for (int e = 0; e < NR; ++e) { r[e].x -= lt * w.y[e][t].x; r[e].y -= lt * w.y[e][t].y; }
+        }
+        const double dk = 1.0 / a[PI];
+        double u[PI];
+#pragma unroll
+        for (int c = 0; c < PI; ++c) u[c] = a[PI + 1 + c];
+        if (store) keep(i, u, dk, r);
+#pragma unroll
+        for (int t = 0; t < PI - 1; ++t) {
+            w.dv[t] = w.dv[t + 1];
+#pragma unroll
+            for (int e = 0; e < NR; ++e) w.y[e][t] = w.y[e][t + 1];
+#pragma unroll
+            for (int c = 0; c < PI; ++c) w.U[t][c] = w.U[t + 1][c];
+        }
+        w.dv[PI - 1] = dk;
+#pragma unroll
+        for (int e = 0; e < NR; ++e) w.y[e][PI - 1] = r[e];
+#pragma unroll
+        for (int c = 0; c < PI; ++c) w.U[PI - 1][c] = u[c];
+    };
+    // a segment of SG rows at k0; loads the right-hand sides of the one at next
+    auto segment = [&](int k0, int next, bool store, bool top) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < SG; ++u) {
+            step(k0 + u, u, ring[u], store, u >= SG - 3 && top, u >= SG - 2 && top);
+            load_rhs(next + u, ring[u]);
+        }
+    };
+    auto remainder = [&](bool store, bool top) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < SG - 1; ++u)
+            if (u < nrem) step(PB + u, u, ring[u], store, top && u >= nrem - 3, top && u >= nrem - 2);
+    };
+    // start of the remainder (slot 0) or of full segment slot - 1: PI rows of PI + 1 + 2 NR values
+    auto start = [&](int slot, bool put) __attribute__((always_inline)) {
+        double *p = S.scr + (size_t)slot * NS * plane + col;
+        auto move = [&](int e, double &v) __attribute__((always_inline)) {
+            if (put) p[(size_t)e * plane] = v;
+            else v = p[(size_t)e * plane];
+        };
+#pragma unroll
+        for (int t = 0; t < PI; ++t) {
+#pragma unroll
+            for (int c = 0; c < PI; ++c) move(t * NL_ + c, w.U[t][c]);
+            move(t * NL_ + PI, w.dv[t]);
+#pragma unroll
+            for (int e = 0; e < NR; ++e) {
+                move(t * NL_ + PI + 1 + 2 * e, w.y[e][t].x);
+                move(t * NL_ + PI + 2 + 2 * e, w.y[e][t].y);
+            }
+        }
+    };
+    // ---- pass 1
+    const int kf = PB + nrem;  // first row of the full segments
+    tab_load(PB);
+    fill(0);
+    bottom(false);
+    fill(PB);
+    if (nfull > 0 && nrem > 0) {
+        start(0, true);
+        tab_put();
+        remainder(false, false);
+        tab_load(kf);
+        fill(kf);
     }
-    // ---- back substitution
+    for (int g = 0; g < nfull - 1; ++g) {
+        const int k0 = kf + g * SG;
+        start(1 + g, true);
+        tab_put();
+        tab_load(k0 + SG);
+        segment(k0, k0 + SG, false, false);
+    }
+    // ---- pass 2; the top segment's start is the window as it stands
     const int mw = jm < ny / 2 ? jm : jm - ny;
     const bool zero_out = S.trunc && !(l < A.lc && mw < A.mc && mw > -A.mc);
-    double2 xs[2][PB];  // x at k+1 .. k+PB
+    const CI zero = czero_t<CI>();
+    double2 xs[NR][PI];  // x at k+1 .. k+PI
 #pragma unroll
-    for (int c = 0; c < PB; ++c) xs[0][c] = xs[1][c] = make_double2(0.0, 0.0);
-    if (face) {  // w at the top wall face
-        const size_t o = (size_t)(nz - 1) * plane + col;
-        S.f[0][o] = zero;
-        if (nr > 1) S.f[1][o] = zero;
-    }
-    double ub[PF][PB + 1];
-    CI fq[PF][2];
-    auto ld_back = [&](int k, double (&uu)[PB + 1], CI (&ff)[2]) __attribute__((always_inline)) {
+    for (int e = 0; e < NR; ++e)
+#pragma unroll
+        for (int c = 0; c < PI; ++c) xs[e][c] = make_double2(0.0, 0.0);
+    // x of row i of the segment, level k; x4 and x5 (rows 0 and 1): x at the
+    // levels PI + 1 and PI + 2 above
+    auto back = [&](int k, int i, const double2 (&x4)[NR], const double2 (&x5)[NR], int nwide) __attribute__((always_inline)) {
+        const double dk = row(i, PI);
+        double2 r[NR];
+#pragma unroll
+        for (int e = 0; e < NR; ++e)  // rounded to the stored type first: with FP32 spectra the last bits of u, v, w move p by 1e-4
+            r[e] = ccast<double2>(ccast<CI>(make_double2(row(i, PI + 1 + 2 * e), row(i, PI + 2 + 2 * e))));
+#pragma unroll
+        for (int c = 0; c < PI; ++c) {
+            const double u = row(i, c);
+#pragma unroll
+            for (int e = 0; e < NR; ++e) { r[e].x -= u * xs[e][c].x; r[e].y -= u * xs[e][c].y; }
+        }
+        if (nwide > 0) {
+            const double u4 = wide(i, 0);
+#pragma unroll
+            for (int e = 0; e < NR; ++e) { r[e].x -= u4 * x4[e].x; r[e].y -= u4 * x4[e].y; }
+        }
+        if (nwide > 1) {
+            const double u5 = wide(i, 1);
+#pragma unroll
+            for (int e = 0; e < NR; ++e) { r[e].x -= u5 * x5[e].x; r[e].y -= u5 * x5[e].y; }
+        }
         const size_t o = (size_t)k * plane + col;
-        const double *srow = S.scr + (size_t)k * (PB + 1) * plane + col;
 #pragma unroll
-        for (int c = 0; c <= PB; ++c) uu[c] = srow[(size_t)c * plane];
-        ff[0] = S.f[0][o];
-        ff[1] = nr > 1 ? S.f[1][o] : zero;
+        for (int e = 0; e < NR; ++e) {
+            r[e] = make_double2(r[e].x * dk, r[e].y * dk);
+#pragma unroll
+            for (int c = PI - 1; c > 0; --c) xs[e][c] = xs[e][c - 1];
+            xs[e][0] = r[e];
+            S.f[e][o] = zero_out ? zero : ccast<CI>(r[e]);
+        }
     };
+    const double2 none[NR] = {};
+    if (face) {  // w at the top wall face
 #pragma unroll
-    for (int u = 0; u < PF; ++u)
-        if (n - 1 - u >= 0) ld_back(n - 1 - u, ub[u], fq[u]);
-    for (int k0 = n - 1; k0 >= 0; k0 -= PF) {
-#pragma unroll
-      for (int q = 0; q < PF; ++q) {
-        const int k = k0 - q;
-        if (k < 0) break;
-        const size_t o = (size_t)k * plane + col;
-        double u[PB];
-#pragma unroll
-        for (int c = 0; c < PB; ++c) u[c] = ub[q][c];
-        const double dk = ub[q][PB];
-        double2 r[2];
-        r[0] = ccast<double2>(fq[q][0]);
-        r[1] = ccast<double2>(fq[q][1]);
-        if (k - PF >= 0) ld_back(k - PF, ub[q], fq[q]);
-#pragma unroll
-        for (int c = 0; c < PB; ++c) {
-            r[0].x -= u[c] * xs[0][c].x;
-            r[0].y -= u[c] * xs[0][c].y;
-            r[1].x -= u[c] * xs[1][c].x;
-            r[1].y -= u[c] * xs[1][c].y;
-        }
-        r[0] = make_double2(r[0].x * dk, r[0].y * dk);
-        r[1] = make_double2(r[1].x * dk, r[1].y * dk);
-#pragma unroll
-        for (int c = PB - 1; c > 0; --c) {
-            xs[0][c] = xs[0][c - 1];
-            xs[1][c] = xs[1][c - 1];
-        }
-        xs[0][0] = r[0];
-        xs[1][0] = r[1];
-        S.f[0][o] = zero_out ? zero : ccast<CI>(r[0]);
-        if (nr > 1) S.f[1][o] = zero_out ? zero : ccast<CI>(r[1]);
-      }
+        for (int e = 0; e < NR; ++e) S.f[e][(size_t)(nz - 1) * plane + col] = zero;
     }
+    for (int g = nfull - 1; g >= 0; --g) {
+        const int k0 = kf + g * SG, next = g > 0 ? k0 - SG : nrem > 0 ? PB : 0;
+        tab_put();
+        tab_load(next);
+        segment(k0, next, true, g == nfull - 1);
+        if (next > 0) start(g, false);  // while this one is back-substituted
+#pragma unroll
+        for (int u = SG - 1; u >= 0; --u) back(k0 + u, u, none, none, 0);
+    }
+    if (nrem > 0) {
+        tab_put();
+        remainder(true, nfull == 0);
+        fill(0);
+        for (int u = nrem - 1; u >= 0; --u) back(PB + u, u, none, none, 0);
+    }
+    bottom(true);
+    double2 xb[NR], xa[NR];  // x at levels PB and PB - 1
+#pragma unroll
+    for (int e = 0; e < NR; ++e) xb[e] = xs[e][0];
+#pragma unroll
+    for (int k = PB - 1; k >= 0; --k) {
+        if (k == 0) back(0, 0, xa, xb, 2);
+        else if (k == 1) back(1, 1, xb, none, 1);
+        else back(k, k, none, none, 0);
+        if (k == PB - 1) {
+#pragma unroll
+            for (int e = 0; e < NR; ++e) xa[e] = xs[e][0];
+        }
+    }
+}
+
+template <int PI, class CI>
+__global__ __launch_bounds__(64) void k_z6_band(StepArgs A, BandArgs<CI> B)
+{
+    const BandSys<CI> S = B.s[blockIdx.y];
+    if constexpr (PI == 3) {
+        if (S.nr > 1) {
+            band_solve<PI, 2, CI>(A, S);
+            return;
+        }
+    }
+    band_solve<PI, 1, CI>(A, S);
 }
 
 // ---------------------------------------------------------------------------

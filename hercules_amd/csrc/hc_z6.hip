@@ -49,15 +49,16 @@ BandSys<CI> band_sys(const CI *in0, const CI *in1, CI *f0, CI *f1, double *scr, 
     return b;
 }
 
-// Direct solves of nsys independent system groups, one thread per column;
-// the pressure (half band 7) runs alone.
+// Direct solves of nsys independent system groups, one thread per column
+// and one wavefront per block, which spreads the few wavefronts over all CUs;
+// the pressure (half band 5) runs alone.
 template <class CI>
 void band_launch(hipStream_t st, const StepArgs &A, const BandArgs<CI> &B, int nsys)
 {
     const int ncol = A.nl * A.ny;
-    const dim3 g((unsigned)((ncol + 255) / 256), (unsigned)nsys);
-    if (B.s[0].eq == 2) hipLaunchKernelGGL((k_z6_band<7, CI>), g, dim3(256), 0, st, A, B);
-    else hipLaunchKernelGGL((k_z6_band<5, CI>), g, dim3(256), 0, st, A, B);
+    const dim3 g((unsigned)((ncol + 63) / 64), (unsigned)nsys);
+    if (B.s[0].eq == 2) hipLaunchKernelGGL((k_z6_band<5, CI>), g, dim3(64), band_lds<5>(1), st, A, B);
+    else hipLaunchKernelGGL((k_z6_band<3, CI>), g, dim3(64), band_lds<3>(B.s[0].nr), st, A, B);
 }
 
 // the pressure correction phi: an FP64 half spectrum (A.zspc) in every
@@ -69,8 +70,8 @@ void pressure_solve(hipStream_t st, const StepArgs &A)
     band_launch(st, A, B, 1);
 }
 
-// U-row scratch of the second system group (the first starts at A.zscr):
-// 6 doubles per level and column for half band 5
+// scratch of the second system group (the first starts at A.zscr): 24
+// doubles per column for each segment of 12 levels and one more
 size_t band_off(const StepArgs &A) { return (size_t)6 * A.nz * A.nl * A.ny; }
 
 // one thread per (l, m) column and z chunk
@@ -149,5 +150,16 @@ template void launch_col6<float>(int, hipStream_t, const StepArgs &, const ColIO
 template void launch_spec_col6<double>(int, hipStream_t, const StepArgs &, const SpecIO<double> &);
 template void launch_spec_col6<float>(int, hipStream_t, const StepArgs &, const SpecIO<float> &);
 
-// the 6th-order column kernels use no dynamic LDS
-hipError_t z6_set_lds(int, int) { return hipSuccess; }
+hipError_t z6_set_lds(int, int)
+{
+    hipError_t e = hipSuccess;
+#define HC_A1(K_, B_)                                                                                               \
+    if (e == hipSuccess)                                                                                            \
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&K_), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(B_));
+    HC_A1((k_z6_band<3, double2>), band_lds<3>(2))
+    HC_A1((k_z6_band<3, float2>), band_lds<3>(2))
+    HC_A1((k_z6_band<5, double2>), band_lds<5>(1))
+    HC_A1((k_z6_band<5, float2>), band_lds<5>(1))
+#undef HC_A1
+    return e;
+}

@@ -246,3 +246,25 @@ def test_z6_tiles_match_torch_reference(nx, ny, nz, kw):
         print(nx, ny, nz, kw, n, f"{err:.2e}")
         assert err < (1e-9 if n == "p" else 1e-11), (n, err)
     ch.close()
+
+
+@pytest.mark.parametrize("order", [6, 4])
+@pytest.mark.parametrize("nz", [16, 17, 18, 19, 28, 29, 30, 41])
+def test_band_segments_match_torch_reference(nz, order):
+    """The band solves where a column's levels leave the segments of 12 a
+    remainder of no, one, few or eleven levels, and where the remainder is all
+    there is above the first rows; columns that do not fill a wavefront.
+    Tolerances as for the steps above."""
+    prm = cases.stratified_open_channel(nx=16, ny=16, nz=nz, wall_rows=1, zorder=order, nu=1.0 / 180.0, dt=5e-4)
+    st = cases.loglaw_noise(prm, seed=5)
+    ref = TorchChannel(prm).steps({k: torch.tensor(v) for k, v in st.items()}, 1)
+    ch = Channel(prm)
+    for k, v in st.items():
+        ch.set_field(k, v)
+    ch.init()
+    ch.steps(1)
+    for n in ["u", "v", "w", "p", "t"]:
+        err = rel_l2(ch.get_field(n), ref[n].numpy())
+        print(nz, order, n, f"{err:.2e}")
+        assert err < (1e-9 if n == "p" else 1e-11), (n, err)
+    ch.close()
