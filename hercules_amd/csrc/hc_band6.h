@@ -50,6 +50,7 @@ struct BandArgs {
 HC_DEV double z6_wall_rhs(const StepArgs &A, int eq, int op, double ck, int k)
 {
     const int nz = A.nz;
+    if (k >= 4 && k < nz - 4) return 0.0;  // no stencil of these reaches a wall
     double bot, top;
     bool has_top;
     if (eq == 0) {
@@ -470,78 +471,115 @@ __global__ __launch_bounds__(64) void k_z6_band(StepArgs A, BandArgs<CI> B)
 // Explicit column operations of the 6th-order step, one thread per (l, m)
 // column streaming along z.  A thread keeps a window of kWin levels of the
 // fields that an operator reaches (levels k-7 .. k+7 around the row k being
-// formed) and applies band rows (ZB_* tables, read as block-uniform values)
-// to it; the fields read at the row itself pass through a delay of kBandMax
-// levels.  Loads run kPF levels ahead of the window through a staging ring
-// indexed by the unrolled loop position, so the wavefront never waits on a
-// load issued less than kPF levels earlier.
+// formed) and applies band rows (ZB_* tables) to it.  Loads run PF levels
+// ahead through a ring indexed by the unrolled loop position.  The loop holds
+// no other load and no branch around one, which a wait would not tell from
+// those in flight: the band rows of the block's levels are staged in LDS,
+// levels out of range are loaded from the nearest one and dropped.  What bounds
+// these kernels then is HBM: at 256x256x257 w's right-hand side moves 8.8 fields
+// of 136 MB in 234 us (294 with the band rows read in the loop), the projection
+// 9.4 in 217 (267), the divergence 4.4 in 109 (130); with FP32 spectra t's
+// right-hand side 82 us (147), the divergence 62 (145).
 constexpr int kWin = 2 * kBandMax + 1;
 
-// A thread forms the rows kb .. ke-1 of its column's z chunk (blockIdx.z of
-// gridDim.z equal chunks), so that a launch has several wavefronts per SIMD.
-// Iterations i = kb - kBandMax, ...: window field w enters level i, point
-// fields enter level i - kBandMax, and row k = i - kBandMax (kb <= k < ke) is
-// formed by row(k, win, pts) with win[kBandMax + t] = level k + t (zero
-// outside 0 .. wlev[f] - 1; a chunk reads kBandMax levels beyond each end).
-// Fields are stored as CI (double2 or float2) and held in FP64.  A kernel
-// writes only its point fields' rows or fields it does not read.
+// A block forms the rows kb .. ke-1 of its columns (blockIdx.z of gridDim.z
+// equal chunks), so that a launch has several wavefronts per SIMD.
 constexpr int kStreamRowsPerChunk = 32;
 inline int stream_chunks(int nz) { return nz / kStreamRowsPerChunk < 1 ? 1 : (nz / kStreamRowsPerChunk > 8 ? 8 : nz / kStreamRowsPerChunk); }
+struct ZChunk {
+    int kb, ke, csz;
+};
+HC_DEV ZChunk z_chunk(int nrows)
+{
+    const int csz = (nrows + (int)gridDim.z - 1) / (int)gridDim.z, kb = (int)blockIdx.z * csz;
+    return {kb, min(kb + csz, nrows), csz};
+}
+// bytes of LDS that nb bands of a chunk take
+inline size_t stream_lds(int nz, int nb)
+{
+    const int nc = stream_chunks(nz);
+    return (size_t)nb * ((nz + nc - 1) / nc) * kBandRow * sizeof(double);
+}
+// rows kb .. ke-1 of band b of this launch's NB bands at sm + b csz kBandRow;
+// every thread of the block calls this (it ends in a barrier)
+template <int NB>
+HC_DEV void stage_bands(const double *zband, int nz, const ZChunk &z, const int (&band)[NB], double *sm)
+{
+    const int n = (z.ke - z.kb) * kBandRow;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+        for (int q = threadIdx.x; q < n; q += 256)
+            sm[b * z.csz * kBandRow + q] = zband[((size_t)band[b] * nz + z.kb) * kBandRow + q];
+    __syncthreads();
+}
+HC_DEV const double *band_row(const double *sm, const ZChunk &z, int b, int k)
+{
+    return sm + (b * z.csz + k - z.kb) * kBandRow;
+}
+
+// Row k is formed by row(k, win, pts) with win[kBandMax + t] = level k + t
+// (zero outside 0 .. wlev[f] - 1; a chunk reads kBandMax levels beyond each
+// end) and pts the point fields at k.  Fields are stored as CI (double2 or
+// float2) and held in FP64.  A kernel writes only its point fields' rows or
+// fields it does not read.
 template <int N, class CI = double2>
 struct FieldSet {
     const CI *p[N > 0 ? N : 1];
     int n[N > 0 ? N : 1];  // levels of a window field
 };
 template <int NW, int NP, int PF, class CW, class CP, class Row>
-HC_DEV void z6_stream(size_t plane, size_t col, int nrows, const FieldSet<NW, CW> ws, const FieldSet<NP, CP> ps,
+HC_DEV void z6_stream(size_t plane, size_t col, const ZChunk &z, const FieldSet<NW, CW> ws, const FieldSet<NP, CP> ps,
                       Row &&row)
 {
-    const auto &wlev = ws.n;
     const double2 zero = make_double2(0.0, 0.0);
-    const CW zw_ = czero_t<CW>();
-    const CP zp_ = czero_t<CP>();
-    const int csz = (nrows + (int)gridDim.z - 1) / (int)gridDim.z;
-    const int kb = (int)blockIdx.z * csz, ke = kb + csz < nrows ? kb + csz : nrows;
-    const int ib = kb - kBandMax;
-    // the staging ring holds the stored type: widening to FP64 happens when a
-    // level leaves the ring, so no conversion waits on a load in flight
+    const int kb = z.kb, ke = z.ke;
+    if (kb >= ke) return;
+    auto load_w = [&](int f, int li) __attribute__((always_inline)) {
+        return ws.p[f][(size_t)min(max(li, 0), ws.n[f] - 1) * plane + col];
+    };
+    auto load_p = [&](int p, int k) __attribute__((always_inline)) { return ps.p[p][(size_t)min(k, ke - 1) * plane + col]; };
+    auto level = [&](int f, int li, const CW &v) __attribute__((always_inline)) {
+        return li >= 0 && li < ws.n[f] ? ccast<double2>(v) : zero;
+    };
+    // the ring holds the stored type: widening to FP64 happens when a level
+    // leaves the ring, so no conversion waits on a load in flight
     double2 win[NW][kWin];
-    CW fw[NW][PF];
+    CW fw[NW][PF], first[NW][kWin - 1];
     CP fp[PF][NP > 0 ? NP : 1];
 #pragma unroll
     for (int f = 0; f < NW; ++f)
 #pragma unroll
-        for (int t = 0; t < kWin; ++t) win[f][t] = zero;
+        for (int t = 0; t < kWin - 1; ++t) first[f][t] = load_w(f, kb - kBandMax + t);
 #pragma unroll
     for (int u = 0; u < PF; ++u) {
-        const int li = ib + u, lp = li - kBandMax;
 #pragma unroll
-        for (int f = 0; f < NW; ++f) fw[f][u] = (li >= 0 && li < wlev[f]) ? ws.p[f][(size_t)li * plane + col] : zw_;
+        for (int f = 0; f < NW; ++f) fw[f][u] = load_w(f, kb + u + kBandMax);
 #pragma unroll
-        for (int p = 0; p < NP; ++p) fp[u][p] = (lp >= kb && lp < ke) ? ps.p[p][(size_t)lp * plane + col] : zp_;
+        for (int p = 0; p < NP; ++p) fp[u][p] = load_p(p, kb + u);
     }
-    for (int i0 = ib; i0 < ke + kBandMax; i0 += PF) {
+#pragma unroll
+    for (int f = 0; f < NW; ++f)
+#pragma unroll
+        for (int t = 0; t < kWin - 1; ++t) win[f][t + 1] = level(f, kb - kBandMax + t, first[f][t]);
+    for (int k0 = kb; k0 < ke; k0 += PF) {
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
-            const int i = i0 + u;
+            const int k = k0 + u;
+            if (k >= ke) return;
             double2 pts[NP > 0 ? NP : 1];
 #pragma unroll
             for (int f = 0; f < NW; ++f) {
 #pragma unroll
                 for (int t = 0; t < kWin - 1; ++t) win[f][t] = win[f][t + 1];
-                win[f][kWin - 1] = ccast<double2>(fw[f][u]);
+                win[f][kWin - 1] = level(f, k + kBandMax, fw[f][u]);
             }
 #pragma unroll
             for (int p = 0; p < NP; ++p) pts[p] = ccast<double2>(fp[u][p]);
-            // the loads of iteration i + PF
-            const int li = i + PF, lp = li - kBandMax;
 #pragma unroll
-            for (int f = 0; f < NW; ++f)
-                fw[f][u] = (li >= 0 && li < wlev[f]) ? ws.p[f][(size_t)li * plane + col] : zw_;
+            for (int f = 0; f < NW; ++f) fw[f][u] = load_w(f, k + PF + kBandMax);
 #pragma unroll
-            for (int p = 0; p < NP; ++p) fp[u][p] = (lp >= kb && lp < ke) ? ps.p[p][(size_t)lp * plane + col] : zp_;
-            const int k = i - kBandMax;
-            if (k >= kb && k < ke) row(k, win, pts);
+            for (int p = 0; p < NP; ++p) fp[u][p] = load_p(p, k + PF);
+            row(k, win, pts);
         }
     }
 }
@@ -557,10 +595,6 @@ HC_DEV double2 band_dot(const double *brow, const double2 (&x)[kWin])
         acc.y += b * x[t].y;
     }
     return acc;
-}
-HC_DEV const double *band_row(const StepArgs &A, int band, int k)
-{
-    return A.zband + ((size_t)band * A.nz + k) * kBandRow;
 }
 
 struct ColIdx {
@@ -583,9 +617,12 @@ HC_DEV bool col_idx(const StepArgs &A, ColIdx &c)
 // spectrum dst (get_p_eqn_src / get_div_spec with ZO_D over the interior
 // faces).
 template <class CI>
-__global__ __launch_bounds__(256) void k_z6s_div(StepArgs A, const CI *u, const CI *v, const CI *w, double2 *dst,
+__global__ __launch_bounds__(256, 2) void k_z6s_div(StepArgs A, const CI *u, const CI *v, const CI *w, double2 *dst,
                                                  double scale)
 {
+    extern __shared__ double band_sm[];
+    const ZChunk z = z_chunk(A.nz);
+    stage_bands(A.zband, A.nz, z, {ZB_D}, band_sm);
     ColIdx c;
     if (!col_idx(A, c)) return;
     const int nl = A.nl, ny = A.ny, nz = A.nz;
@@ -593,8 +630,8 @@ __global__ __launch_bounds__(256) void k_z6s_div(StepArgs A, const CI *u, const 
     const double2 sdy = make_double2(A.symy[SY_DRE * ny + c.jm], A.symy[SY_DIM * ny + c.jm]);
     const FieldSet<1, CI> ws = {{w}, {nz - 1}};
     const FieldSet<2, CI> ps = {{u, v}, {0, 0}};
-    z6_stream<1, 2, 8>(c.plane, c.col, nz, ws, ps, [&](int k, const double2 (&win)[1][kWin], const double2 (&p)[2]) __attribute__((always_inline)) {
-        const double2 dz = band_dot(band_row(A, ZB_D, k), win[0]);
+    z6_stream<1, 2, 8>(c.plane, c.col, z, ws, ps, [&](int k, const double2 (&win)[1][kWin], const double2 (&p)[2]) __attribute__((always_inline)) {
+        const double2 dz = band_dot(band_row(band_sm, z, 0, k), win[0]);
         const double2 d = cadd(cadd(cmul(sdx, p[0]), cmul(sdy, p[1])), dz);
         dst[(size_t)k * c.plane + c.col] = make_double2(d.x * scale, d.y * scale);
     });
@@ -607,9 +644,12 @@ __global__ __launch_bounds__(256) void k_z6s_div(StepArgs A, const CI *u, const 
 // substep, cdt = rc dt): the increment is added to c_p in `pinc` and the
 // columns outside the 2/3 rule are zeroed.
 template <class CI>
-__global__ __launch_bounds__(256) void k_z6s_proj(StepArgs A, CI *u, CI *v, CI *w, const double2 *phi, CI *pinc,
+__global__ __launch_bounds__(256, 2) void k_z6s_proj(StepArgs A, CI *u, CI *v, CI *w, const double2 *phi, CI *pinc,
                                                   int mode)
 {
+    extern __shared__ double band_sm[];
+    const ZChunk z = z_chunk(A.nz);
+    stage_bands(A.zband, A.nz, z, {ZB_G, ZB_P}, band_sm);
     ColIdx c;
     if (!col_idx(A, c)) return;
     const int nl = A.nl, ny = A.ny, nz = A.nz;
@@ -623,21 +663,21 @@ __global__ __launch_bounds__(256) void k_z6s_proj(StepArgs A, CI *u, CI *v, CI *
     const FieldSet<1> ws = {{phi}, {nz}};
     // the fourth point field is read only in mode 2 (c_p); u stands in otherwise
     const FieldSet<4, CI> ps = {{u, v, w, mode == 2 ? pinc : u}, {0, 0, 0, 0}};
-    z6_stream<1, 4, 6>(c.plane, c.col, nz, ws, ps, [&](int k, const double2 (&win)[1][kWin], const double2 (&p)[4]) __attribute__((always_inline)) {
+    z6_stream<1, 4, 4>(c.plane, c.col, z, ws, ps, [&](int k, const double2 (&win)[1][kWin], const double2 (&p)[4]) __attribute__((always_inline)) {
         const size_t o = (size_t)k * c.plane + c.col;
         const double2 ph = win[0][kBandMax];
         double2 uu = csub(p[0], cscale(cmul(sgx, ph), cdt));
         double2 vv = csub(p[1], cscale(cmul(sgy, ph), cdt));
         double2 ww = p[2];
         if (k < nz - 1) {
-            const double2 g = band_dot(band_row(A, ZB_G, k), win[0]);
+            const double2 g = band_dot(band_row(band_sm, z, 0, k), win[0]);
             ww = make_double2(ww.x - cdt * g.x, ww.y - cdt * g.y);
         }
         u[o] = kept ? ccast<CI>(uu) : zero;
         v[o] = kept ? ccast<CI>(vv) : zero;
         w[o] = kept ? ccast<CI>(ww) : zero;
         if (mode == 1) return;
-        const double2 pz = band_dot(band_row(A, ZB_P, k), win[0]);
+        const double2 pz = band_dot(band_row(band_sm, z, 1, k), win[0]);
         const double2 inc = make_double2(ph.x - cnu * (slap * ph.x + pz.x), ph.y - cnu * (slap * ph.y + pz.y));
         if (mode == 0) pinc[o] = ccast<CI>(inc);
         else pinc[o] = kept ? ccast<CI>(cadd(p[3], inc)) : zero;
@@ -653,8 +693,11 @@ __global__ __launch_bounds__(256) void k_z6s_proj(StepArgs A, CI *u, CI *v, CI *
 // with X, Y, R the transformed products of the component; f replaces f_old.
 // The (0,0) mode adds the explicit half of the wall data of u.
 template <class CI>
-__global__ __launch_bounds__(256) void k_z6s_rhs_uv(StepArgs A, SpecIO<real_of<CI>> io)
+__global__ __launch_bounds__(256, 2) void k_z6s_rhs_uv(StepArgs A, SpecIO<real_of<CI>> io)
 {
+    extern __shared__ double band_sm[];
+    const ZChunk z = z_chunk(A.nz);
+    stage_bands(A.zband, A.nz, z, {A.ochannel ? ZB_C2_DN : ZB_C2_DD}, band_sm);
     ColIdx c;
     if (!col_idx(A, c)) return;
     const int e = blockIdx.y;
@@ -664,16 +707,16 @@ __global__ __launch_bounds__(256) void k_z6s_rhs_uv(StepArgs A, SpecIO<real_of<C
     const double dif = A.rc * 0.5 * A.dt * A.nu, coe = A.coe, um = A.u_mrf, cdt = A.rc * A.dt;
     const double rb = A.rb * A.dt, ra = A.ra * A.dt, kk = e == 0 ? kx : ky;
     const bool is00 = e == 0 && c.l == 0 && c.jm == 0;
-    const int band = A.ochannel ? ZB_C2_DN : ZB_C2_DD, op = A.ochannel ? ZO_C2_DN : ZO_C2_DD;
+    const int op = A.ochannel ? ZO_C2_DN : ZO_C2_DD;
     // q goes over R_u / R_v (read at the same row by the same thread): c_u,
     // c_v stay intact for the neighbouring z chunks' windows
     CI *cs = e == 0 ? io.cu : io.cv, *fo = e == 0 ? io.cff : io.cgg, *qo = e == 0 ? io.sp[3] : io.sp[4];
     const FieldSet<1, CI> ws = {{cs}, {nz}};
     const FieldSet<5, CI> ps = {{io.sp[e == 0 ? 0 : 1], io.sp[e == 0 ? 1 : 2], io.sp[e == 0 ? 3 : 4], io.cp, fo},
                                 {0, 0, 0, 0, 0}};
-    z6_stream<1, 5, 4>(c.plane, c.col, nz, ws, ps, [&](int k, const double2 (&win)[1][kWin], const double2 (&p)[5]) __attribute__((always_inline)) {
+    z6_stream<1, 5, 3>(c.plane, c.col, z, ws, ps, [&](int k, const double2 (&win)[1][kWin], const double2 (&p)[5]) __attribute__((always_inline)) {
         const double2 x = win[0][kBandMax];
-        const double2 t = band_dot(band_row(A, band, k), win[0]);
+        const double2 t = band_dot(band_row(band_sm, z, 0, k), win[0]);
         double2 q = make_double2(x.x + hxy * x.x + dif * t.x, x.y + hxy * x.y + dif * t.y);
         if (is00) q.x += z6_wall_rhs(A, 0, op, dif, k);
         double2 f = times_i(x, -um * kx);
@@ -688,8 +731,11 @@ __global__ __launch_bounds__(256) void k_z6s_rhs_uv(StepArgs A, SpecIO<real_of<C
     });
 }
 template <class CI>
-__global__ __launch_bounds__(256) void k_z6s_rhs_w(StepArgs A, SpecIO<real_of<CI>> io)
+__global__ __launch_bounds__(256, 2) void k_z6s_rhs_w(StepArgs A, SpecIO<real_of<CI>> io)
 {
+    extern __shared__ double band_sm[];
+    const ZChunk z = z_chunk(A.nz);
+    stage_bands(A.zband, A.nz, z, {ZB_F2, ZB_G}, band_sm);
     ColIdx c;
     if (!col_idx(A, c)) return;
     const int nl = A.nl, ny = A.ny, nz = A.nz;
@@ -699,7 +745,7 @@ __global__ __launch_bounds__(256) void k_z6s_rhs_w(StepArgs A, SpecIO<real_of<CI
     const double rb = A.rb * A.dt, ra = A.ra * A.dt;
     const FieldSet<2, CI> ws = {{io.cw, io.cp}, {nz - 1, nz}};
     const FieldSet<4, CI> ps = {{io.sp[5], io.sp[6], io.sp[7], io.chh}, {0, 0, 0, 0}};
-    z6_stream<2, 4, 4>(c.plane, c.col, nz, ws, ps, [&](int k, const double2 (&win)[2][kWin], const double2 (&p)[4]) __attribute__((always_inline)) {
+    z6_stream<2, 4, 2>(c.plane, c.col, z, ws, ps, [&](int k, const double2 (&win)[2][kWin], const double2 (&p)[4]) __attribute__((always_inline)) {
         const size_t o = (size_t)k * c.plane + c.col;
         const double2 x = win[0][kBandMax];
         double2 f = times_i(x, -um * kx);
@@ -708,8 +754,8 @@ __global__ __launch_bounds__(256) void k_z6s_rhs_w(StepArgs A, SpecIO<real_of<CI
         f = make_double2(f.x + coe * p[2].x, f.y + coe * p[2].y);
         io.chh[o] = ccast<CI>(f);
         if (k == nz - 1) return;  // the top wall face: no equation
-        const double2 t = band_dot(band_row(A, ZB_F2, k), win[0]);
-        const double2 g = band_dot(band_row(A, ZB_G, k), win[1]);
+        const double2 t = band_dot(band_row(band_sm, z, 0, k), win[0]);
+        const double2 g = band_dot(band_row(band_sm, z, 1, k), win[1]);
         double2 q = make_double2(x.x + hxy * x.x + dif * t.x - cdt * g.x, x.y + hxy * x.y + dif * t.y - cdt * g.y);
         q = make_double2(q.x + rb * p[3].x + ra * f.x, q.y + rb * p[3].y + ra * f.y);
         io.sp[7][o] = ccast<CI>(q);  // over R_w, as for u and v
@@ -721,8 +767,11 @@ __global__ __launch_bounds__(256) void k_z6s_rhs_w(StepArgs A, SpecIO<real_of<CI
 // the new s replaces the old one in c_ss; the (0,0) mode adds the explicit
 // half of the wall data.
 template <class CI>
-__global__ __launch_bounds__(256) void k_z6s_rhs_t(StepArgs A, SpecIO<real_of<CI>> io)
+__global__ __launch_bounds__(256, 2) void k_z6s_rhs_t(StepArgs A, SpecIO<real_of<CI>> io)
 {
+    extern __shared__ double band_sm[];
+    const ZChunk z = z_chunk(A.nz);
+    stage_bands(A.zband, A.nz, z, {A.tbc_top ? ZB_C2_DN : ZB_C2_DD}, band_sm);
     ColIdx c;
     if (!col_idx(A, c)) return;
     const int nl = A.nl, ny = A.ny, nz = A.nz;
@@ -731,12 +780,12 @@ __global__ __launch_bounds__(256) void k_z6s_rhs_t(StepArgs A, SpecIO<real_of<CI
     const double dif = A.rc * 0.5 * A.dt * A.alpha, um = A.u_mrf;
     const double rb = A.rb * A.dt, ra = A.ra * A.dt;
     const bool is00 = c.l == 0 && c.jm == 0;
-    const int band = A.tbc_top ? ZB_C2_DN : ZB_C2_DD, op = A.tbc_top ? ZO_C2_DN : ZO_C2_DD;
+    const int op = A.tbc_top ? ZO_C2_DN : ZO_C2_DD;
     const FieldSet<1, CI> ws = {{io.ct}, {nz}};
     const FieldSet<4, CI> ps = {{io.sp[0], io.sp[1], io.sp[2], io.css}, {0, 0, 0, 0}};
-    z6_stream<1, 4, 6>(c.plane, c.col, nz, ws, ps, [&](int k, const double2 (&win)[1][kWin], const double2 (&p)[4]) __attribute__((always_inline)) {
+    z6_stream<1, 4, 4>(c.plane, c.col, z, ws, ps, [&](int k, const double2 (&win)[1][kWin], const double2 (&p)[4]) __attribute__((always_inline)) {
         const double2 x = win[0][kBandMax];
-        const double2 t = band_dot(band_row(A, band, k), win[0]);
+        const double2 t = band_dot(band_row(band_sm, z, 0, k), win[0]);
         double2 d = make_double2(x.x + hxy * x.x + dif * t.x, x.y + hxy * x.y + dif * t.y);
         if (is00) d.x += z6_wall_rhs(A, 3, op, dif, k);
         double2 f = times_i(x, -um * kx);

@@ -15,7 +15,7 @@ void zinterp6(hc_ctx *c, StepArgsT<R> &B)
     R *b[4];
     for (int q = 0; q < 4; ++q) b[q] = reinterpret_cast<R *>(c->zbuf[q]);
     const dim3 grid((unsigned)(((size_t)B.nx * B.ny + 255) / 256), 4, (unsigned)stream_chunks(B.nz));
-    hipLaunchKernelGGL((k_zinterp6<R>), grid, dim3(256), 0, c->stream, I, b[0], b[1], b[2], b[3]);
+    hipLaunchKernelGGL((k_zinterp6<R>), grid, dim3(256), stream_lds(B.nz, 1), c->stream, I, b[0], b[1], b[2], b[3]);
     B.zfu = b[0]; B.zfv = b[1]; B.zcw = b[2]; B.zft = b[3];
 }
 template void zinterp6<double>(hc_ctx *, StepArgsT<double> &);
@@ -26,8 +26,8 @@ template <class R>
 void z6_terms(hc_ctx *c, const StepArgsT<R> &B, int e0)
 {
     const dim3 grid((unsigned)(((size_t)B.nx * B.ny + 255) / 256), e0 == 3 ? 1 : 3, (unsigned)stream_chunks(B.nz));
-    if (c->prm.cds == 1) hipLaunchKernelGGL((k_z6_terms<1, R>), grid, dim3(256), 0, c->stream, B, e0);
-    else hipLaunchKernelGGL((k_z6_terms<2, R>), grid, dim3(256), 0, c->stream, B, e0);
+    if (c->prm.cds == 1) hipLaunchKernelGGL((k_z6_terms<1, R>), grid, dim3(256), stream_lds(B.nz, 2), c->stream, B, e0);
+    else hipLaunchKernelGGL((k_z6_terms<2, R>), grid, dim3(256), stream_lds(B.nz, 2), c->stream, B, e0);
 }
 template void z6_terms<double>(hc_ctx *, const StepArgsT<double> &, int);
 
@@ -90,18 +90,18 @@ void col6_seq(int kind, hipStream_t st, const StepArgs &A, const ColIO<R> &io, i
         B.s[0] = band_sys<CI>(nullptr, nullptr, io.s0, io.s1, A.zscr, 0, 1, 0);
         B.s[1] = band_sys<CI>(nullptr, nullptr, io.s2, nullptr, A.zscr + band_off(A), 1, 0, 0);
         band_launch(st, A, B, 2);
-        hipLaunchKernelGGL((k_z6s_div<CI>), stream_grid(A), dim3(256), 0, st, A, io.s0, io.s1, io.s2, A.zspc, A.idt);
+        hipLaunchKernelGGL((k_z6s_div<CI>), stream_grid(A), dim3(256), stream_lds(A.nz, 1), st, A, io.s0, io.s1, io.s2, A.zspc, A.idt);
         pressure_solve(st, A);
-        hipLaunchKernelGGL((k_z6s_proj<CI>), stream_grid(A), dim3(256), 0, st, A, io.s0, io.s1, io.s2, A.zspc, io.s3, 0);
+        hipLaunchKernelGGL((k_z6s_proj<CI>), stream_grid(A), dim3(256), stream_lds(A.nz, 2), st, A, io.s0, io.s1, io.s2, A.zspc, io.s3, 0);
         break;
     case 1:  // temperature
         B.s[0] = band_sys<CI>(nullptr, nullptr, io.s0, nullptr, A.zscr, 3, 1, 0);
         band_launch(st, A, B, 1);
         break;
     case 2:  // projection onto divergence-free fields (rk_c = 1)
-        hipLaunchKernelGGL((k_z6s_div<CI>), stream_grid(A), dim3(256), 0, st, A, io.s0, io.s1, io.s2, A.zspc, 1.0);
+        hipLaunchKernelGGL((k_z6s_div<CI>), stream_grid(A), dim3(256), stream_lds(A.nz, 1), st, A, io.s0, io.s1, io.s2, A.zspc, 1.0);
         pressure_solve(st, A);
-        hipLaunchKernelGGL((k_z6s_proj<CI>), stream_grid(A), dim3(256), 0, st, A, io.s0, io.s1, io.s2, A.zspc,
+        hipLaunchKernelGGL((k_z6s_proj<CI>), stream_grid(A), dim3(256), stream_lds(A.nz, 2), st, A, io.s0, io.s1, io.s2, A.zspc,
                            (CI *)nullptr, 1);
         break;
     default: {  // one equation: 0 u, 1 v, 2 w, 3 p, 4 t; wall data for u and t, delnull for p
@@ -119,19 +119,19 @@ void spec6_seq(int kind, hipStream_t st, const StepArgs &A, const SpecIO<R> &io)
     using CI = cplx<R>;
     BandArgs<CI> B;
     if (kind == 1) {  // temperature: right-hand side, solve, 2/3 rule
-        hipLaunchKernelGGL((k_z6s_rhs_t<CI>), stream_grid(A), dim3(256), 0, st, A, io);
+        hipLaunchKernelGGL((k_z6s_rhs_t<CI>), stream_grid(A), dim3(256), stream_lds(A.nz, 1), st, A, io);
         B.s[0] = band_sys<CI>(io.sp[2], nullptr, io.ct, nullptr, A.zscr, 3, 1, 1);
         band_launch(st, A, B, 1);
         return;
     }
-    hipLaunchKernelGGL((k_z6s_rhs_uv<CI>), stream_grid(A, 2), dim3(256), 0, st, A, io);
-    hipLaunchKernelGGL((k_z6s_rhs_w<CI>), stream_grid(A), dim3(256), 0, st, A, io);
+    hipLaunchKernelGGL((k_z6s_rhs_uv<CI>), stream_grid(A, 2), dim3(256), stream_lds(A.nz, 1), st, A, io);
+    hipLaunchKernelGGL((k_z6s_rhs_w<CI>), stream_grid(A), dim3(256), stream_lds(A.nz, 2), st, A, io);
     B.s[0] = band_sys<CI>(io.sp[3], io.sp[4], io.cu, io.cv, A.zscr, 0, 1, 0);
     B.s[1] = band_sys<CI>(io.sp[7], nullptr, io.cw, nullptr, A.zscr + band_off(A), 1, 0, 0);
     band_launch(st, A, B, 2);
-    hipLaunchKernelGGL((k_z6s_div<CI>), stream_grid(A), dim3(256), 0, st, A, io.cu, io.cv, io.cw, A.zspc, A.idt);
+    hipLaunchKernelGGL((k_z6s_div<CI>), stream_grid(A), dim3(256), stream_lds(A.nz, 1), st, A, io.cu, io.cv, io.cw, A.zspc, A.idt);
     pressure_solve(st, A);
-    hipLaunchKernelGGL((k_z6s_proj<CI>), stream_grid(A), dim3(256), 0, st, A, io.cu, io.cv, io.cw, A.zspc, io.cp, 2);
+    hipLaunchKernelGGL((k_z6s_proj<CI>), stream_grid(A), dim3(256), stream_lds(A.nz, 2), st, A, io.cu, io.cv, io.cw, A.zspc, io.cp, 2);
 }
 }  // namespace
 

@@ -24,7 +24,8 @@
 // One thread per (i, j) column, field (blockIdx.y: u, v, w, t) and z chunk
 // (blockIdx.z of gridDim.z) streams along z with a window of kIntWin levels,
 // k-kIntHW .. k+kIntHW around the row k being formed, and applies the band
-// rows ZB_IU_* and ZB_IFC (block-uniform values).  The window holds the wall
+// rows ZB_IU_* and ZB_IFC, staged in LDS (FP64 at 256x256x257 423 -> 207 us,
+// 9.2 fields of 135 MB; see z6_stream).  The window holds the wall
 // data of the C convention at levels -1 and nz (u: -u_mrf, and -u_mrf or
 // du/dz = 0 at the top; v: 0; t: tbot, and ttop or the wall gradient) and
 // zero beyond; w is zero outside its interior faces 0..nz-2.  The band rows
@@ -36,19 +37,21 @@ template <class R>
 __global__ __launch_bounds__(256) void k_zinterp6(StepArgsT<R> A, R *fu, R *fv, R *cw, R *ft)
 {
     constexpr int PF = 8;
+    extern __shared__ double band_sm[];
     const int nz = A.nz, f = (int)blockIdx.y;
     const size_t plane = (size_t)A.nx * A.ny;
     const size_t col = blockIdx.x * (size_t)256 + threadIdx.x;
-    if (col >= plane || (f == 3 && !ft)) return;
-    const int csz = (nz + (int)gridDim.z - 1) / (int)gridDim.z;
-    const int kb = (int)blockIdx.z * csz, ke = kb + csz < nz ? kb + csz : nz;
-    const int ib = kb - kIntHW;
+    const ZChunk z = z_chunk(nz);
+    const int band = f == 2 ? ZB_IFC : (f == 3 ? A.tbc_top : A.ochannel) ? ZB_IU_DN : ZB_IU_DD;
+    stage_bands(A.zband, nz, z, {band}, band_sm);
+    if (col >= plane || (f == 3 && !ft) || z.kb >= z.ke) return;
+    const int kb = z.kb, ke = z.ke;
     const R zero = R(0.0);
     // the field's data, its stored levels lo .. nlev-1, wall data at levels
     // -1 and nz, band and output
     const R *src;
     R *dst, wb = zero, wt = zero;
-    int nlev = nz, band = A.ochannel ? ZB_IU_DN : ZB_IU_DD;
+    int nlev = nz;
     if (f == 0) {
         src = A.u; dst = fu;
         wb = R(-A.u_mrf);
@@ -56,43 +59,38 @@ __global__ __launch_bounds__(256) void k_zinterp6(StepArgsT<R> A, R *fu, R *fv, 
     } else if (f == 1) {
         src = A.v; dst = fv;
     } else if (f == 2) {
-        src = A.w; dst = cw; nlev = nz - 1; band = ZB_IFC;
+        src = A.w; dst = cw; nlev = nz - 1;
     } else {
         src = A.t; dst = ft;
         wb = A.tbot;
         wt = A.tbc_top ? R(A.gdz_top * A.lev[LV_IDZT * nz + nz - 1]) : A.ttop;
-        band = A.tbc_top ? ZB_IU_DN : ZB_IU_DD;
     }
     if (f == 2) wb = wt = zero;  // w: zero at both wall faces
-    // level li (block-uniform: the selection branches on scalars)
-    auto load = [&](int li) __attribute__((always_inline)) {
-        return (li >= 0 && li < nlev) ? src[(size_t)li * plane + col] : (li == -1 ? wb : (li == nz ? wt : zero));
+    auto load = [&](int li) __attribute__((always_inline)) { return src[(size_t)min(max(li, 0), nlev - 1) * plane + col]; };
+    auto level = [&](int li, R v) __attribute__((always_inline)) {
+        return li >= 0 && li < nlev ? v : (li == -1 ? wb : (li == nz ? wt : zero));
     };
-    R win[kIntWin];
-    R ring[PF];
+    R win[kIntWin], ring[PF], first[kIntWin - 1];
 #pragma unroll
-    for (int t = 0; t < kIntWin; ++t) win[t] = zero;
+    for (int t = 0; t < kIntWin - 1; ++t) first[t] = load(kb - kIntHW + t);
 #pragma unroll
-    for (int u = 0; u < PF; ++u) ring[u] = load(ib + u);
-    // iteration i: level i enters the window; row k = i - kIntHW is formed
-    for (int i0 = ib; i0 < ke + kIntHW; i0 += PF) {
+    for (int u = 0; u < PF; ++u) ring[u] = load(kb + kIntHW + u);
+#pragma unroll
+    for (int t = 0; t < kIntWin - 1; ++t) win[t + 1] = level(kb - kIntHW + t, first[t]);
+    for (int k0 = kb; k0 < ke; k0 += PF) {
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
-            const int i = i0 + u;
+            const int k = k0 + u;
+            if (k >= ke) return;
 #pragma unroll
             for (int t = 0; t < kIntWin - 1; ++t) win[t] = win[t + 1];
-            win[kIntWin - 1] = ring[u];
-            ring[u] = load(i + PF);
-            const int k = i - kIntHW;
-            if (k >= kb && k < ke) {
-                R acc = zero;
-                if (f != 3 || k < nz - 1) {
-                    const double *b = A.zband + ((size_t)band * nz + k) * kBandRow + kBandMax - kIntHW;
+            win[kIntWin - 1] = level(k + kIntHW, ring[u]);
+            ring[u] = load(k + PF + kIntHW);
+            R acc = zero;
+            const double *b = band_row(band_sm, z, 0, k) + kBandMax - kIntHW;
 #pragma unroll
-                    for (int t = 0; t < kIntWin; ++t) acc += R(b[t]) * win[t];
-                }
-                dst[(size_t)k * plane + col] = acc;
-            }
+            for (int t = 0; t < kIntWin; ++t) acc += R(b[t]) * win[t];
+            dst[(size_t)k * plane + col] = f == 3 && k == nz - 1 ? zero : acc;
         }
     }
 }
@@ -106,7 +104,8 @@ __global__ __launch_bounds__(256) void k_zinterp6(StepArgsT<R> A, R *fu, R *fv, 
 //             rc into hh, qw (levels below the top)
 //   e = 3:    d(tw)/dz, d2t/dz2 into ss, qt
 // One thread per (i, j) column, equation (e0 + blockIdx.y) and z chunk streams
-// along z with windows of kWin levels, as the spectral path's column kernels.
+// along z with windows of kWin levels, as the spectral path's column kernels
+// (192x128x129: 259 us a substep with the band rows read in the loop, 141 so).
 // The fluxes through a face are formed once, where the accessors formed six
 // per point; a wall face carries none.
 // The window of a face quantity holds face kw at level kw; the band rows ZB_D
@@ -115,6 +114,7 @@ __global__ __launch_bounds__(256) void k_zinterp6(StepArgsT<R> A, R *fu, R *fv, 
 template <class R>
 HC_DEV R zwall(const StepArgsT<R> &A, int op, int k, R bot, R top, bool has_top)
 {
+    if (k >= 4 && k < A.nz - 4) return R(0);  // no stencil of these reaches a wall
     const size_t e = (size_t)op * A.nz + k;
     const int s = A.zst[e], jt = A.nz + 1 - s;
     const double *w = A.zwt + e * kZW;
@@ -123,42 +123,62 @@ HC_DEV R zwall(const StepArgsT<R> &A, int op, int k, R bot, R top, bool has_top)
     if (has_top && jt < A.zn2) v += R(w[jt]) * top;
     return v;
 }
-// NR stored values per level (load) become NW window entries (make)
-template <int NR, int NW, class R, class Load, class Make, class Row>
-HC_DEV void zterm_stream(int nrows, Load &&load, Make &&make, Row &&row)
+// NR stored values per level (load, of any level 0 .. nrows) become NW window
+// entries (make); NP values of the row itself (point).  The loads run PF rows
+// ahead, as z6_stream's.
+template <int NR, int NW, int NP, class R, class Load, class Make, class Point, class Row>
+HC_DEV void zterm_stream(const ZChunk &z, int nlev, Load &&load, Make &&make, Point &&point, Row &&row)
 {
-    constexpr int PF = 3;
-    const int csz = (nrows + (int)gridDim.z - 1) / (int)gridDim.z;
-    const int kb = (int)blockIdx.z * csz, ke = min(kb + csz, nrows), ib = kb - kBandMax;
-    R win[NW][kWin], ring[PF][NR];
+    constexpr int PF = 4;
+    const int kb = z.kb, ke = z.ke;
+    R win[NW][kWin], ring[PF][NR], pring[PF][NP];
+    auto lev = [&](int li) { return min(max(li, 0), nlev - 1); };
+    auto enter = [&](int li, const R (&v)[NR]) __attribute__((always_inline)) {
+        R in[NW];
+        make(li, v, in);
+#pragma unroll
+        for (int f = 0; f < NW; ++f) {
+#pragma unroll
+            for (int t = 0; t < kWin - 1; ++t) win[f][t] = win[f][t + 1];
+            win[f][kWin - 1] = in[f];
+        }
+    };
 #pragma unroll
     for (int f = 0; f < NW; ++f)
 #pragma unroll
         for (int t = 0; t < kWin; ++t) win[f][t] = R(0);
+    static_assert((kWin - 1) % 2 == 0);
 #pragma unroll
-    for (int u = 0; u < PF; ++u) load(ib + u, ring[u]);
-    for (int i0 = ib; i0 < ke + kBandMax; i0 += PF) {
+    for (int h = 0; h < 2; ++h) {
+        R first[(kWin - 1) / 2][NR];
+#pragma unroll
+        for (int t = 0; t < (kWin - 1) / 2; ++t) load(lev(kb - kBandMax + h * (kWin - 1) / 2 + t), first[t]);
+#pragma unroll
+        for (int t = 0; t < (kWin - 1) / 2; ++t) enter(kb - kBandMax + h * (kWin - 1) / 2 + t, first[t]);
+    }
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+        load(lev(kb + kBandMax + u), ring[u]);
+        point(min(kb + u, ke - 1), pring[u]);
+    }
+    for (int k0 = kb; k0 < ke; k0 += PF) {
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
-            const int i = i0 + u;
-            R in[NW];
-            make(i, ring[u], in);
+            const int k = k0 + u;
+            if (k >= ke) return;
+            enter(k + kBandMax, ring[u]);
+            R pt[NP];
 #pragma unroll
-            for (int f = 0; f < NW; ++f) {
-#pragma unroll
-                for (int t = 0; t < kWin - 1; ++t) win[f][t] = win[f][t + 1];
-                win[f][kWin - 1] = in[f];
-            }
-            load(i + PF, ring[u]);
-            const int k = i - kBandMax;
-            if (k >= kb && k < ke) row(k, win);
+            for (int p = 0; p < NP; ++p) pt[p] = pring[u][p];
+            load(lev(k + PF + kBandMax), ring[u]);
+            point(min(k + PF, ke - 1), pring[u]);
+            row(k, win, pt);
         }
     }
 }
 template <class R>
-HC_DEV R zdot(const StepArgsT<R> &A, int band, int k, const R (&x)[kWin])
+HC_DEV R zdot(const double *b, const R (&x)[kWin])
 {
-    const double *b = A.zband + ((size_t)band * A.nz + k) * kBandRow;
     R acc = R(0);
 #pragma unroll
     for (int t = 0; t < kWin; ++t) acc += R(b[t]) * x[t];
@@ -170,8 +190,14 @@ __global__ __launch_bounds__(256) void k_z6_terms(StepArgsT<R> A, int e0)
 {
     const int nx = A.nx, ny = A.ny, nz = A.nz, e = e0 + (int)blockIdx.y;
     const size_t plane = (size_t)nx * ny, col = blockIdx.x * (size_t)256 + threadIdx.x;
-    if (col >= plane) return;
+    extern __shared__ double band_sm[];
+    const ZChunk z = z_chunk(e == 2 ? nz - 1 : nz);
+    const bool grad = e == 3 ? A.tbc_top != 0 : A.ochannel != 0;
+    stage_bands(A.zband, nz, z, {e == 2 ? ZB_G : ZB_D, e == 2 ? ZB_F2 : grad ? ZB_C2_DN : ZB_C2_DD}, band_sm);
+    if (col >= plane || z.kb >= z.ke) return;
     const int j = (int)(col / nx), i = (int)(col - (size_t)j * nx);
+    auto none = [](int, R (&p)[1]) { p[0] = R(0); };
+    auto dot = [&](int b, int k, const R (&x)[kWin]) __attribute__((always_inline)) { return zdot(band_row(band_sm, z, b, k), x); };
     if (e < 2) {
         // neighbours of w across x (u) or y (v): the face interpolant whx, why
         const R *f = e == 0 ? A.u : A.v, *zf = e == 0 ? A.zfu : A.zfv;
@@ -181,11 +207,10 @@ __global__ __launch_bounds__(256) void k_z6_terms(StepArgsT<R> A, int e0)
         for (int d = 0; d < 4; ++d)
             o[d] = e == 0 ? (size_t)j * nx + wrapi(i + d - 1, nx) : (size_t)wrapi(j + d - 1, ny) * nx + i;
         const R wall = e == 0 ? R(-A.u_mrf) : R(0);
-        const int op = A.ochannel ? ZO_C2_DN : ZO_C2_DD, band = A.ochannel ? ZB_C2_DN : ZB_C2_DD;
-        zterm_stream<6, 2, R>(nz,
+        const int op = A.ochannel ? ZO_C2_DN : ZO_C2_DD;
+        zterm_stream<6, 2, 1, R>(z, nz,
             [&](int li, R (&v)[6]) __attribute__((always_inline)) {
-                const int lc = min(max(li, 0), nz - 1);
-                const size_t b = (size_t)lc * plane;
+                const size_t b = (size_t)li * plane;
                 v[0] = f[b + col];
                 v[1] = zf[b + col];
 #pragma unroll
@@ -197,17 +222,19 @@ __global__ __launch_bounds__(256) void k_z6_terms(StepArgsT<R> A, int e0)
                                       : (-v[5] + R(9.0) * v[4] + R(9.0) * v[3] - v[2]) / R(16.0);
                 in[1] = li >= 0 && li < nz - 1 ? v[1] * wh : R(0);
             },
-            [&](int k, const R (&win)[2][kWin]) __attribute__((always_inline)) {
+            none,
+            [&](int k, const R (&win)[2][kWin], const R (&)[1]) __attribute__((always_inline)) {
                 const size_t c = (size_t)k * plane + col;
-                conv[c] = zdot(A, ZB_D, k, win[1]);
-                dif[c] = zdot(A, band, k, win[0]) + zwall<R>(A, op, k, wall, wall, A.ochannel == 0);
+                conv[c] = dot(0, k, win[1]);
+                dif[c] = dot(1, k, win[0]) + zwall<R>(A, op, k, wall, wall, A.ochannel == 0);
             });
     } else if (e == 2) {
         R *qw = reinterpret_cast<R *>(A.s2);
         const R cn = R(0.5) * A.dt * A.nu;
-        zterm_stream<3, 3, R>(nz - 1,
+        const R *zt = A.isscalar ? A.zft : A.zcw;
+        zterm_stream<3, 3, 1, R>(z, nz,
             [&](int li, R (&v)[3]) __attribute__((always_inline)) {
-                const size_t b = (size_t)min(max(li, 0), nz - 1) * plane + col;
+                const size_t b = (size_t)li * plane + col;
                 v[0] = A.w[b];
                 v[1] = A.p[b];
                 v[2] = A.zcw[b];
@@ -218,20 +245,22 @@ __global__ __launch_bounds__(256) void k_z6_terms(StepArgsT<R> A, int e0)
                 in[1] = on ? v[1] : R(0);
                 in[2] = on ? sq(v[2]) : R(0);
             },
-            [&](int k, const R (&win)[3][kWin]) __attribute__((always_inline)) {
+            // without temperature a value that is there and is not used
+            [&](int k, R (&p)[1]) __attribute__((always_inline)) { p[0] = zt[(size_t)k * plane + col]; },
+            [&](int k, const R (&win)[3][kWin], const R (&p)[1]) __attribute__((always_inline)) {
                 const size_t c = (size_t)k * plane + col;
-                R con = zdot(A, ZB_G, k, win[2]);
-                if (A.isscalar) con -= A.got * (A.zft[c] - A.t_ref);
+                R con = dot(0, k, win[2]);
+                if (A.isscalar) con -= A.got * (p[0] - A.t_ref);
                 A.hh[c] = con;
-                qw[c] = cn * zdot(A, ZB_F2, k, win[0]) - A.dt * zdot(A, ZB_G, k, win[1]);
+                qw[c] = cn * dot(1, k, win[0]) - A.dt * dot(0, k, win[1]);
             });
     } else {
         R *qt = reinterpret_cast<R *>(A.s0);
         const R top = A.tbc_top ? R(A.gdz_top * A.lev[LV_IDZT * nz + nz - 1]) : A.ttop;
-        const int op = A.tbc_top ? ZO_C2_DN : ZO_C2_DD, band = A.tbc_top ? ZB_C2_DN : ZB_C2_DD;
-        zterm_stream<3, 2, R>(nz,
+        const int op = A.tbc_top ? ZO_C2_DN : ZO_C2_DD;
+        zterm_stream<3, 2, 1, R>(z, nz,
             [&](int li, R (&v)[3]) __attribute__((always_inline)) {
-                const size_t b = (size_t)min(max(li, 0), nz - 1) * plane + col;
+                const size_t b = (size_t)li * plane + col;
                 v[0] = A.t[b];
                 v[1] = A.zft[b];
                 v[2] = A.w[b];
@@ -240,10 +269,11 @@ __global__ __launch_bounds__(256) void k_z6_terms(StepArgsT<R> A, int e0)
                 in[0] = li >= 0 && li < nz ? v[0] : R(0);
                 in[1] = li >= 0 && li < nz - 1 ? v[1] * v[2] : R(0);
             },
-            [&](int k, const R (&win)[2][kWin]) __attribute__((always_inline)) {
+            none,
+            [&](int k, const R (&win)[2][kWin], const R (&)[1]) __attribute__((always_inline)) {
                 const size_t c = (size_t)k * plane + col;
-                A.ss[c] = zdot(A, ZB_D, k, win[1]);
-                qt[c] = zdot(A, band, k, win[0]) + zwall<R>(A, op, k, A.tbot, top, true);
+                A.ss[c] = dot(0, k, win[1]);
+                qt[c] = dot(1, k, win[0]) + zwall<R>(A, op, k, A.tbot, top, true);
             });
     }
 }
