@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void k_yfft_io(YIOArgsT<R> A)
 //   R_v = tmp2/coe - dvwdz - [issk](u dvdx + v dvdy + w dvdz)   (:279-339)
 //   R_w = buoy/coe - dwwdz - [issk](u dwdx + v dwdy + w dwdz)   (:426-496)
 template <int NX, class R, int ZO = 2>
-__global__ __launch_bounds__(1024) void k_spec_mom(StepArgsT<R> A)
+__global__ __launch_bounds__(1024, 8) void k_spec_mom(StepArgsT<R> A)
 {
     using C = cplx<R>;
     constexpr int ROWS = rows_per_block<NX>();
@@ -118,49 +118,75 @@ __global__ __launch_bounds__(1024) void k_spec_mom(StepArgsT<R> A)
         // 6th-order z (zorder = 6): the same products and terms with the
         // face values, z derivatives and z interpolants of the ZOp tables
         PtT<R> g(A, i, j, k);
+        // The columns of the stencils are read in three batches of independent
+        // loads (k_zinterp6 has formed the face values and w at the centres):
+        // u, v, w at three faces twice, in a loop, then w at the centres.  One
+        // load at a time waited out the cache's latency eighteen times over
+        // (FP32 at 256x256x257: 900 us, 690 so); more at once takes more than
+        // the 64 registers that two FP64 blocks per CU leave (54 here, 1.18 ->
+        // 1.14 ms; one block per CU, or 64 with spills, 1.48 ms).  Entries
+        // beyond the width of a stencil or past a wall have zero weight or
+        // value, so their levels are only kept in range.
+        auto at = [&](const R *f, int kk) { return f[((size_t)min(max(kk, 0), A.nz - 1) * A.ny + j) * NX + i]; };
+        // d(u w)/dz, d(v w)/dz and du/dz, dv/dz at this level from the face
+        // values of faces s0-1 .. s0+4, all within -1..nz-1
+        int s0, sg;
+        const double *wd = g.zw(ZO_D, k, s0), *wg = g.zw(ZO_G, min(k, A.nz - 2), sg);
+        R uwz = R(0.0), vwz = R(0.0), duz = R(0.0), dvz = R(0.0);
+#pragma unroll 1
+        for (int q0 = 0; q0 < 6; q0 += 3) {
+            R uf[3], vf[3], wf[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const int kw = s0 + q0 + q - 1;
+                uf[q] = at(A.zfu, kw);
+                vf[q] = at(A.zfv, kw);
+                wf[q] = at(A.w, kw);
+            }
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const int kw = s0 + q0 + q - 1;
+                const R wq = R(wd[q0 + q]), uq = kw < 0 ? -A.u_mrf : uf[q], vq = kw < 0 ? R(0.0) : vf[q];
+                const R ww = (kw < 0 || kw >= A.nz - 1) ? R(0.0) : wf[q];
+                uwz += wq * uq * ww;
+                vwz += wq * vq * ww;
+                duz += wq * uq;
+                dvz += wq * vq;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // d(w w)/dz and dw/dz at this level's face from w at the centres
+        R wwz = R(0.0), dwz = R(0.0), f[6];
+#pragma unroll
+        for (int q = 0; q < 6; ++q) f[q] = at(A.zcw, sg + q);
         const R u = g.U(0, 0, 0), v = g.V(0, 0, 0), w = g.W(0, 0, 0);
+        const R a1 = at(A.zfu, k), a1v = at(A.zfv, k);  // u, v at this level's w face
+        const R wc = at(A.zcw, k);                      // w at this level's centre
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+            wwz += R(wg[q]) * sq(f[q]);
+            dwz += R(wg[q]) * f[q];
+        }
+        __builtin_amdgcn_sched_barrier(0);
         const R coe = A.coe;
         const R dpx = A.dp_opt == 2 ? R(A.scal[0]) : A.dpx;
-        const R a1 = g.uf6(k), a1v = g.vf6(k);  // u, v at this level's w face
+        const R tmp2u = A.dp_opt == 3 ? A.fc * (v - A.vg) : dpx;
+        const R tmp2v = A.dp_opt == 3 ? A.fc * (A.ug - u - A.u_mrf) : R(0.0);
+        R ru = R(1.0) / coe * tmp2u - uwz;
+        R rv = R(1.0) / coe * tmp2v - vwz;
+        R rw = k < A.nz - 1 ? -wwz : R(0.0);
+        if (A.isscalar && k < A.nz - 1) rw += R(1.0) / coe * (A.got * (at(A.zft, k) - A.t_ref));
+        if (A.issk) {
+            auto D = [&](int f) { return sd[(f * ROWS + jj) * NX + i]; };
+            ru -= u * D(0) + v * D(1) + duz * wc;
+            rv -= u * D(2) + v * D(3) + dvz * wc;
+            if (k < A.nz - 1) rw -= a1 * D(4) + a1v * D(5) + w * dwz;
+        }
         out[0] = u * u;
         out[1] = u * v;
         out[2] = v * v;
         out[5] = a1 * w;
         out[6] = a1v * w;
-        const R tmp2u = A.dp_opt == 3 ? A.fc * (v - A.vg) : dpx;
-        const R tmp2v = A.dp_opt == 3 ? A.fc * (A.ug - u - A.u_mrf) : R(0.0);
-        // d(u w)/dz, d(v w)/dz and du/dz, dv/dz at this level from the face values
-        int s0;
-        const double *wd = g.zw(ZO_D, k, s0);
-        R uwz = R(0.0), vwz = R(0.0), duz = R(0.0), dvz = R(0.0);
-#pragma unroll 1
-        for (int q = 0; q < A.zn1; ++q) {  // faces s0-1 .. s0+zn1-2, all within -1..nz-1
-            const int kw = s0 + q - 1;
-            const R uf = g.uf6(kw), vf = g.vf6(kw);
-            const R wf = (kw < 0 || kw >= A.nz - 1) ? R(0.0) : g.W(0, 0, kw - k);
-            uwz += R(wd[q]) * uf * wf;
-            vwz += R(wd[q]) * vf * wf;
-            duz += R(wd[q]) * uf;
-            dvz += R(wd[q]) * vf;
-        }
-        R ru = R(1.0) / coe * tmp2u - uwz;
-        R rv = R(1.0) / coe * tmp2v - vwz;
-        R rw = k < A.nz - 1 ? -g.wwz6() : R(0.0);
-        if (A.isscalar && k < A.nz - 1) rw += R(1.0) / coe * (A.got * (g.thz6(0) - A.t_ref));
-        if (A.issk) {
-            auto D = [&](int f) { return sd[(f * ROWS + jj) * NX + i]; };
-            const R wc = g.whz6(k);  // w at this level's centre
-            ru -= u * D(0) + v * D(1) + duz * wc;
-            rv -= u * D(2) + v * D(3) + dvz * wc;
-            if (k < A.nz - 1) {
-                int sg;
-                const double *wg = g.zw(ZO_G, k, sg);
-                R dwz = R(0.0);
-#pragma unroll 1
-                for (int q = 0; q < A.zn1; ++q) dwz += R(wg[q]) * g.whz6(sg + q);
-                rw -= a1 * D(4) + a1v * D(5) + w * dwz;
-            }
-        }
         out[3] = ru;
         out[4] = rv;
         out[7] = rw;
@@ -248,7 +274,20 @@ __global__ __launch_bounds__(1024) void k_spec_t(StepArgsT<R> A)
         const R a1 = tp * lt + t * (R(1.0) - lt), a2 = tm * lb + t * (R(1.0) - lb);
         out[0] = u * t;
         out[1] = t * v;
-        if constexpr (ZO == 6) out[2] = -g.twz6();
+        if constexpr (ZO == 6) {  // d(t w)/dz from the faces within the walls, in one batch of loads (as k_spec_mom)
+            int s0;
+            const double *wd = g.zw(ZO_D, k, s0);
+            auto at = [&](const R *f, int kk) { return f[((size_t)min(max(kk, 0), A.nz - 1) * A.ny + j) * NX + i]; };
+            R tf[6], wf[6], acc = R(0.0);
+#pragma unroll
+            for (int q = 0; q < 6; ++q) { tf[q] = at(A.zft, s0 + q - 1); wf[q] = at(A.w, s0 + q - 1); }
+#pragma unroll
+            for (int q = 0; q < 6; ++q) {
+                const int kw = s0 + q - 1;
+                acc += (kw < 0 || kw >= A.nz - 1) ? R(0.0) : R(wd[q]) * tf[q] * wf[q];
+            }
+            out[2] = -acc;
+        }
         else out[2] = -((a1 * w - a2 * wm) / A.lev[LV_DZ * A.nz + k]);
     }
 #pragma unroll
