@@ -38,14 +38,14 @@ int adjoint_substep(hc_ctx *c, int t_its)
     io.ou = c->adf[nxt][0]; io.ov = c->adf[nxt][1]; io.ow = c->adf[nxt][2];
     for (int q = 0; q < 3; ++q) io.fb[q] = c->adfb[q];
     for (int q = 0; q < 8; ++q) io.face[q] = c->adface[q];
-    const dim3 gp(2048), bp(256);
+    const dim3 gp(2048), bp(256), gl((unsigned)((c->nx * c->ny + 255) / 256), (unsigned)c->nz);
     hipLaunchKernelGGL(k_adj_fbar, gp, bp, 0, c->stream, A, io);
     if (P.cds == 1) {
-        hipLaunchKernelGGL((k_adj_faces<1>), gp, bp, 0, c->stream, A, io);
-        hipLaunchKernelGGL((k_adj_gather<1>), gp, bp, 0, c->stream, A, io);
+        hipLaunchKernelGGL((k_adj_faces<1>), gl, bp, 0, c->stream, A, io);
+        hipLaunchKernelGGL((k_adj_gather<1>), gl, bp, 0, c->stream, A, io);
     } else {
-        hipLaunchKernelGGL((k_adj_faces<2>), gp, bp, 0, c->stream, A, io);
-        hipLaunchKernelGGL((k_adj_gather<2>), gp, bp, 0, c->stream, A, io);
+        hipLaunchKernelGGL((k_adj_faces<2>), gl, bp, 0, c->stream, A, io);
+        hipLaunchKernelGGL((k_adj_gather<2>), gl, bp, 0, c->stream, A, io);
     }
     c->adcur = nxt;
     HIPCHK(hipGetLastError());
