@@ -591,9 +591,11 @@ def main():
         # the right-hand-side stage's bytes depend on the momentum tile shape
         shapes = getattr(ch, "tuning", None) or {}
         by_shape = tj.get("rhs_by_shape", {})
-        if str(shapes.get("rhs_xt", 0)) in by_shape:
-            traffic["rhs"] = by_shape[str(shapes.get("rhs_xt", 0))]
-        elif "launch_shapes" in tj and shapes.get("rhs_xt", 0) != tj["launch_shapes"].get("rhs_xt", 0):
+        # (0, chosen by size, is the 32x8 tiles at FP64 rows of 96 and more)
+        xt = shapes.get("rhs_xt", 0) or (1 if prm.nx >= 96 and not mixed_main else 0)
+        if str(xt) in by_shape:
+            traffic["rhs"] = by_shape[str(xt)]
+        elif "launch_shapes" in tj and xt != tj["launch_shapes"].get("rhs_xt", 0):
             traffic.pop("rhs", None)
     roofline = None
     if kernels:

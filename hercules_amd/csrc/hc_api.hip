@@ -3,11 +3,12 @@
 // buffers), the FD substep sequence and the small reduction kernels.
 //
 // One substep of the finite-difference RK3 step (time_advancement_fd,
-// src/module_navier_stokes.f90:247-355) is five launches:
-//   k_rhs_mom2    right-hand sides ff,gg,hh and qu,qv,qw, fused with the
-//                 x-direction real-to-complex FFT of the q's (hc_rhs.hip)
+// src/module_navier_stokes.f90:247-355) is five or six launches:
+//   right-hand sides ff,gg,hh and qu,qv,qw and the x-direction real-to-complex
+//                 FFT of the q's: k_rhs_mom_march and k_x_r2c (hc_march.h), or
+//                 k_rhs_mom2 for short rows and FP32 (hc_rhs.hip)
 //   k_yfft<-1>    y-direction FFT of the three q spectra (hc_xfer.hip)
-//   k_column_mom  per (l,m) column: Helmholtz solves for u*, v*, w*, the
+//   k_column_mom  (k_column_mom_mixed with FP32 spectra) per (l,m) column: Helmholtz solves for u*, v*, w*, the
 //                 divergence source, the pressure Poisson solve, the
 //                 projection and the pressure increment, all in spectral
 //                 space (exact equivalents of get_p_eqn_src, calculate_uvw

@@ -241,10 +241,12 @@ int hc_get_scalar(hc_ctx *ctx, int id, double *value);
  * context from its current state for each candidate launch shape of the
  * finite-difference kernels (RHS tile-order group, y-transform columns per
  * block, inverse-x points per block, column block order, momentum tile
- * shape: 0 whole x rows with the x transform fused, 1-4 tiles of 32x8, 64x8,
- * 32x16, 64x4 points and a separate in-place x transform; coordinate
- * descent, steps_per_trial steps per trial) and keeps the fastest.  Every
- * candidate gives bit-identical results.  The state and step counters are
+ * shape: 0 chosen by size, 1-4 tiles of 32x8, 64x8, 32x16, 64x4 points that
+ * march up the levels, with a separate in-place x transform; by size: 32x8
+ * for FP64 rows of 96 and more, otherwise whole x rows with the x transform
+ * fused; coordinate descent, steps_per_trial steps per trial) and keeps the
+ * fastest.  Every candidate gives bit-identical results but for the last knob
+ * where it changes between tiles and whole rows (round-off).  The state and step counters are
  * restored; the spectral path (cds = 3) keeps its fixed shapes. */
 int hc_autotune(hc_ctx *ctx, int steps_per_trial);
 /* Set one of those launch shapes directly (knob 0..4 in the order above;
