@@ -185,8 +185,9 @@ HC_DEV void col_drain(CI *__restrict__ dst, const CI *sub, int nz, size_t plane,
     }
 }
 
-// Table tab at the r-th level of this lane (r < m.cnt).  For parts the tables are kept in lane order, one line of 512 bytes per load; by level,
-// a load of 64 lanes touches 20 lines and more.
+// Table tab at the r-th level of this lane (r < m.cnt).  For parts the tables
+// are kept in lane order, one run of 512 bytes per load; by level, a load of
+// 64 lanes touches 20 lines and more.
 template <int L, class M>
 HC_DEV double col_lev(const StepArgs &A, const M &m, int tab, int r)
 {

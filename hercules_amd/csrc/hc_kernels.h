@@ -341,36 +341,6 @@ struct Interp {
             if (j < zn(false)) acc += Re(w[j]) * tdat(s + j);
         return acc;
     }
-    // u, v at the face of w level kw = -1..nz-1 (both walls included), for
-    // the advective z terms of the spectral path
-    HC_DEV auto uf6(int kw) const
-    {
-        const D &q = d();
-        using Re = typename D::Real;
-        if (kw < 0) return Re(-q.A.u_mrf);
-        if (q.A.zfu) return Re(q.A.zfu[q.at(0, 0, kw)]);
-        int s;
-        const double *w = zw(q.A.ochannel ? ZO_I_DN : ZO_I_DD, kw, s);
-        Re acc = Re(0.0);
-#pragma unroll
-        for (int j = 0; j < 6; ++j)
-            if (j < zn(false)) acc += Re(w[j]) * udat(0, 0, s + j);
-        return acc;
-    }
-    HC_DEV auto vf6(int kw) const
-    {
-        const D &q = d();
-        using Re = typename D::Real;
-        if (kw < 0) return Re(0.0);
-        if (q.A.zfv) return Re(q.A.zfv[q.at(0, 0, kw)]);
-        int s;
-        const double *w = zw(q.A.ochannel ? ZO_I_DN : ZO_I_DD, kw, s);
-        Re acc = Re(0.0);
-#pragma unroll
-        for (int j = 0; j < 6; ++j)
-            if (j < zn(false)) acc += Re(w[j]) * vdat(0, 0, s + j);
-        return acc;
-    }
     template <int ZO> HC_DEV auto uhzO(int di, int dj, int dk) const
     {
         // through the accessor, which may override the interpolant (PtD)
