@@ -17,8 +17,8 @@
 // incoming state S through the first point with |d| > S, which is one of the
 // run's records (strict prefix maxima of |d|, about ln n of them), to the d
 // where that point's chain of pointers ends.  Three launches:
-//   k_div_units   d of 4096 consecutive points (scan order is memory order)
-//                 in LDS, 64 chunks of 64.  Per chunk and point, the end of
+//   k_div_units   d of 2048 consecutive points (scan order is memory order)
+//                 in LDS, 32 chunks of 64.  Per chunk and point, the end of
 //                 its chain within the chunk (next-greater search over a
 //                 table of shuffled maxima, then pointer doubling).  One lane
 //                 per record then walks the chunks to the end of the unit:
@@ -28,7 +28,7 @@
 //                 div_hist_max in order.
 // A unit with more than kRec records (long monotone |d|) or a group of such
 // units is walked by k_div_final point by point instead.  At 128x128x129 the
-// three take 107 + 36 + 21 us; one wavefront that visited every taken point
+// three take 62 + 36 + 18 us; one wavefront that visited every taken point
 // (a state that a negative d resets takes ~10% of all points) took 2350 us
 // after a 28 us pass for the row maxima.
 #include "hc_host.h"
@@ -37,8 +37,9 @@
 
 namespace {
 constexpr int kScrLen = 32;
-constexpr int kChunk = 64;                 // points of a chunk, chunks of a batch, units of a group
-constexpr int kBatch = kChunk * kChunk;    // points held in LDS at a time
+constexpr int kChunk = 64;                 // points of a chunk, units of a group
+constexpr int kChunks = 32;                // chunks of a batch
+constexpr int kBatch = kChunks * kChunk;   // points held in LDS at a time
 constexpr int kRec = 32;                   // records kept per unit / group
 // a unit's or group's summary: sum |d|, max |d|, NaN flag, number of records
 // (-1: more than kRec, or a member had), records, final states
@@ -101,11 +102,13 @@ HC_DEV void write_summary(const Walk &w, double *o, double sum, int nan, int lan
 }
 
 // Bound by the walk's LDS latency and the shuffles of the chunk tables, not
-// by HBM: 4096 points keep 70 KB of LDS, two blocks per CU.
+// by HBM: 2048 points keep 35 KB of LDS, four blocks per CU that hide each
+// other's walks (128x128x129: 62 us; 107 with 4096 points, two blocks per CU,
+// where four of the 516 blocks ran by themselves).
 template <int CDS, class R>
 __global__ __launch_bounds__(256) void k_div_units(StepArgsT<R> F, StepArgs D, unsigned N, int nb, double *units)
 {
-    __shared__ double dd[kBatch], pm[kBatch], cmax[kChunk], rs[4];
+    __shared__ double dd[kBatch], pm[kBatch], cmax[kChunks], rs[4];
     __shared__ unsigned char ex[kBatch];
     __shared__ int rn[4];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -116,7 +119,7 @@ __global__ __launch_bounds__(256) void k_div_units(StepArgsT<R> F, StepArgs D, u
     for (int bt = 0; bt < nb; ++bt) {
         const size_t base = ((size_t)blockIdx.x * nb + bt) * kBatch;
         if (base >= N) break;
-        for (int c = wv; c < kChunk; c += 4) {
+        for (int c = wv; c < kChunks; c += 4) {
             const size_t q = base + (size_t)c * kChunk + lane;
             double d = 0.0, a = ninf;
             if (q < N) {
@@ -161,7 +164,7 @@ __global__ __launch_bounds__(256) void k_div_units(StepArgsT<R> F, StepArgs D, u
         }
         __syncthreads();
         if (wv == 0) {
-            for (int c = 0; c < kChunk; ++c) {
+            for (int c = 0; c < kChunks; ++c) {
                 const double cm = cmax[c];
                 const int at = c * kChunk;
                 if (lane < w.nrec && cm > w.S) w.S = dd[at + ex[at + first_above(pm + at, kChunk, w.S)]];
@@ -331,7 +334,7 @@ __global__ void k_scr_set(double *f, double v)
 // Partials of one screen: the units' and groups' summaries
 struct ScreenBufs {
     double *units, *groups, *state, *rec;
-    int nb;  // batches of 4096 points per unit
+    int nb;  // batches of 2048 points per unit
 };
 inline int screen_units(const hc_ctx *c, int nb)
 {
@@ -434,7 +437,7 @@ extern "C" int hc_screen_div_error_noalloc(hc_ctx *c, int isfinal, double *div_a
     // the size of grid that is taken: ny nz rows and 3 values for 16 rows of a
     // level within the scratch
     const size_t need = 8 + (size_t)c->ny * c->nz + 3 * (size_t)((c->ny + 15) / 16) * c->nz;
-    // units of as many batches as make their summaries fit: 1 to 8 (a grid of
+    // units of as many batches as make their summaries fit: 1 to 16 (a grid of
     // this size has nx <= 512, so under 2^28 points)
     int nb = 1, nu = screen_units(c, 1);
     while (nb < 64 && 8 + (size_t)(nu + screen_groups(nu)) * kSum > kScratchDoubles) {

@@ -118,7 +118,7 @@ def _planted(kind, shape, dz, rng):
 def test_scan_equals_the_point_by_point_rule(kind, shape):
     """div_max and div_hist_max bit for bit against the rule applied to one
     point after another (u = v = 0, so d = (w(k) - w(k-1)) / dz(k)), runs
-    shorter and longer than the 4096 points of a unit, and more records than
+    shorter and longer than the 2048 points of a unit, and more records than
     a unit keeps; div_avg to the rounding of a sum of positive terms."""
     nz, ny, nx = shape
     ch = Channel(cases.closed_channel(nx=nx, ny=ny, nz=nz))
