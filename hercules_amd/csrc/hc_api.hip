@@ -764,7 +764,7 @@ extern "C" int hc_create(const hc_params *prm, hc_ctx **out)
         hipError_t ae = hipSuccess;
         if (ae == hipSuccess) ae = columns_set_lds(L, (int)kColLds);
         if (ae == hipSuccess) ae = spec_set_lds(L, (int)kColLds);
-        if (ae == hipSuccess) ae = z6_set_lds(L, (int)kColLds);
+        if (ae == hipSuccess && P.zorder != 2) ae = z6_set_lds(L, (int)kColLds);
         c->big_lds = ae == hipSuccess;
         (void)hipGetLastError();
     }
@@ -779,16 +779,19 @@ extern "C" int hc_create(const hc_params *prm, hc_ctx **out)
     build_symbols(P, c->nx, c->nl, c->dx, P.lx, sx);
     build_symbols(P, c->ny, c->ny, c->dy, P.ly, sy);
     auto tnl = twiddles(c->nl), tnx = twiddles(c->nx), tny = twiddles(c->ny);
-    if (!e) e = dalloc(c, (void **)&c->lev, c->h_lev.size() * sizeof(double));
-    // the level tables as the column kernels read them: lane 16 (s mod 4) + s / 4
-    // holds levels s L .. s L + L - 1 (hc_device.h)
-    std::vector<double> hp((size_t)LV_COUNT * L * 64, 0.0);
+    // the level tables, and behind them (from a line on) the tables as the
+    // column kernels read them: lane 16 (s mod 4) + s / 4 holds levels
+    // s L .. s L + L - 1 (hc_device.h)
+    std::vector<double> hl(c->h_lev);
+    const size_t parts0 = (hl.size() + 15) / 16 * 16;
+    hl.resize(parts0 + (size_t)LV_COUNT * L * 64, 0.0);
     for (int tab = 0; tab < LV_COUNT; ++tab)
         for (int k = 0; k < P.nz; ++k) {
             const int s = k / L, lane = 16 * (s % 4) + s / 4;
-            hp[((size_t)tab * L + k % L) * 64 + lane] = c->h_lev[(size_t)tab * P.nz + k];
+            hl[parts0 + ((size_t)tab * L + k % L) * 64 + lane] = c->h_lev[(size_t)tab * P.nz + k];
         }
-    if (!e) e = dalloc(c, (void **)&c->levp, hp.size() * sizeof(double));
+    if (!e) e = dalloc(c, (void **)&c->lev, hl.size() * sizeof(double));
+    if (!e) c->levp = c->lev + parts0;
     if (!e) e = dalloc(c, (void **)&c->symx, sx.size() * sizeof(double));
     if (!e) e = dalloc(c, (void **)&c->symy, sy.size() * sizeof(double));
     if (!e) e = dalloc(c, (void **)&c->tw_nl, tnl.size() * sizeof(double2));
@@ -853,8 +856,7 @@ extern "C" int hc_create(const hc_params *prm, hc_ctx **out)
         hs[kk] = P.cdamp * 0.5 * (1.0 - std::cos(kPi * zd));
     }
     double scal0[8] = {P.dp_opt == 1 ? 1.0 : 0.0, 0, 0, 0, 0, 0, 0, 0};
-    hipError_t r = hipMemcpyAsync(c->lev, c->h_lev.data(), c->h_lev.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
-    if (r == hipSuccess) r = hipMemcpyAsync(c->levp, hp.data(), hp.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
+    hipError_t r = hipMemcpyAsync(c->lev, hl.data(), hl.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
     if (r == hipSuccess) r = hipMemcpyAsync(c->symx, sx.data(), sx.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
     if (r == hipSuccess) r = hipMemcpyAsync(c->symy, sy.data(), sy.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
     if (r == hipSuccess) r = hipMemcpyAsync(c->tw_nl, tnl.data(), tnl.size() * sizeof(double2), hipMemcpyHostToDevice, c->stream);

@@ -84,7 +84,7 @@ struct hc_ctx {
     int fcur, scur;
     double2 *s[4];
     double *lev, *symx, *symy, *scal, *part, *stage;
-    double *levp = nullptr;  // lev in the order the column kernels read it: [table][r][lane] for level r of a lane's Lcol
+    double *levp = nullptr;  // behind lev, in the order the column kernels read it: [table][r][lane] for level r of a lane's Lcol
     // 6th-order z operators (zorder = 6): stencil starts and weights, and
     // the interpolants the right-hand-side kernels read (k_zinterp6)
     int *zst = nullptr;
