@@ -1943,9 +1943,7 @@ extern "C" int hc_autotune(hc_ctx *c, int steps_per_trial)
         return 0;
     };
     // candidates per knob
-    const int ty = P.nx == 16 ? 16 : P.nx == 32 ? 32 : P.nx == 64 ? 16 : P.nx == 128 ? 8 : P.nx == 192 ? 4 :
-                   P.nx == 256 ? 4 : 1;
-    const int nty = c->ny / ty;
+    const int nty = c->ny / rhs_tile_rows(c->nx);
     std::vector<int> groups = {0};
     if (P.nx <= 256)
         for (int g : {1, 2, 4, 8, 16, 32})

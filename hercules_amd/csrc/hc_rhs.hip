@@ -644,6 +644,10 @@ int rhs_momentum(hc_ctx *c, const StepArgs &A, StepArgsT<R> &B)
             cplx<R> *dst[3] = {B.s0, B.s1, B.s2};
             err = launch_r2c_n<R>(c, 3, src, dst, 0, ksplit);
         } else {
+            // a group must hold whole tiles: hc_set_tuning takes values that do not
+            // divide the y tiles of rows of 48 and 96, which would leave tiles
+            // out and run past the last one
+            if (B.rgroup > 0 && (c->ny / rhs_tile_rows(c->nx)) % B.rgroup) B.rgroup = 0;
 #define HC_RHS(NX_)                                                                                     \
     if constexpr (NX_ <= 256) {                                                                          \
         constexpr int TY_ = rhs2_ty<NX_>();                                                              \

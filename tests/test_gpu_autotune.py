@@ -82,3 +82,18 @@ def test_bad_launch_shapes_are_rejected():
         with pytest.raises(HerculesError, match="status 1"):
             ch.set_tuning(**shape)
     ch.close()
+
+
+@pytest.mark.parametrize("kw,groups", [(dict(nx=48, ny=48, nz=17), (2, 4, 16)),
+                                       (dict(nx=48, ny=96, nz=9, cds=1), (32, 3)),
+                                       (dict(nx=96, ny=96, nz=17, precision=1), (16, 32, 4)),
+                                       (dict(nx=96, ny=16, nz=17, precision=1), (4, 16))])
+def test_tile_groups_that_do_not_divide_the_tiles(kw, groups):
+    """Rows of 48 and 96: the y tiles hold 16 and 8 rows, and a tile-order
+    group that does not divide their number leaves the order as it is."""
+    prm, st = small_case("closed", **kw)
+    ref, _ = _run(prm, st, 1)
+    for g in groups:
+        got, _ = _run(prm, st, 1, shape=dict(rgroup=g))
+        for k in ref:
+            assert np.array_equal(got[k], ref[k]), (kw, g, k)
