@@ -1259,13 +1259,11 @@ struct LdT : Interp<LdT<NX, TY, R>> {
 // (src/module_io.f90:103-128): x and y differences of order cds, the z
 // difference (w(k) - w(k-1))/dz(k) with w = 0 below the first level; with
 // zorder = 6 the z derivative is the face-to-centre operator ZO_D.  F holds
-// the fields in their stored precision R, D the FP64 metrics; the spectral
-// path (CDS = 3) reads the divergence formed beforehand from F.aux.
+// the fields in their stored precision R, D the FP64 metrics.
 template <int CDS, class R>
 HC_DEV double div_at(const StepArgsT<R> &F, const StepArgs &D, int i, int j, int k)
 {
     PtT<R> P{F, i, j, k};
-    if (CDS == 3) return (double)F.aux[P.at(0, 0, k)];
     auto U = [&](int di) -> double { return (double)P.U(di, 0, 0); };
     auto V = [&](int dj) -> double { return (double)P.V(0, dj, 0); };
     double dudx, dvdy;

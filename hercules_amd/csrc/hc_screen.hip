@@ -26,6 +26,9 @@
 //   k_div_groups  the same walk over the records of 64 units
 //   k_div_final   one wavefront applies the groups to div_max and
 //                 div_hist_max in order.
+// The spectral path's states are plain maxima of |d|, which need no order:
+//   k_div_max     sum, largest |d| and NaN flag of a block's share of the points
+//   k_div_max_final  the blocks' to div_avg, div_max and div_hist_max
 // A unit with more than kRec records (long monotone |d|) or a group of such
 // units is walked by k_div_final point by point instead.  At 128x128x129 the
 // three take 62 + 36 + 18 us; one wavefront that visited every taken point
@@ -33,6 +36,7 @@
 // after a 28 us pass for the row maxima.
 #include "hc_host.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace {
@@ -50,8 +54,7 @@ __global__ void k_scr_zero(double *f, int n)
     if ((int)threadIdx.x < n) f[threadIdx.x] = 0.0;
 }
 
-// signed divergence of point q (scan order) as the states keep it
-// (screen_div_error_spec stores |d|, src/module_spectral.f90:931-946) and the
+// signed divergence of point q (scan order) as the states keep it and the
 // magnitude it is compared by; a NaN is never taken
 template <int CDS, class R>
 HC_DEV void point_div(const StepArgsT<R> &F, const StepArgs &D, unsigned q, double &d, double &a)
@@ -60,7 +63,6 @@ HC_DEV void point_div(const StepArgsT<R> &F, const StepArgs &D, unsigned q, doub
     const unsigned k = row / (unsigned)D.ny, j = row - k * (unsigned)D.ny;
     d = div_at<CDS, R>(F, D, (int)i, (int)j, (int)k);
     a = fabs(d);
-    if (CDS == 3) d = a;
 }
 
 // One lane's walk state: lane r < nrec follows record r.
@@ -326,6 +328,86 @@ __global__ __launch_bounds__(64) void k_div_final(StepArgsT<R> F, StepArgs D, un
     }
 }
 
+// The largest |d| of the spectral path (screen_div_error_spec stores |d|,
+// src/module_spectral.f90:931-946), whose divergence lies in F.aux: a NaN is
+// never taken.  Bound by HBM: four reads of every point, four points of a
+// thread in flight (256x256x257: 119 us, 4.5 TB/s; a whole screen of that grid
+// 351 us, 501 with the units and records of the signed states, and 71 against
+// 151 at 128x128x129).
+constexpr int kMaxBlocks = 2048;  // eight blocks of four wavefronts per CU
+template <class R>
+__global__ __launch_bounds__(256) void k_div_max(StepArgsT<R> F, unsigned N, double *part)
+{
+    __shared__ double rs[4], rm[4];
+    __shared__ int rn[4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    double s = 0.0, m = -HUGE_VAL;
+    int nan = 0;
+    constexpr int U = 4;
+    for (size_t q0 = (size_t)blockIdx.x * 256 * U + threadIdx.x; q0 < N; q0 += (size_t)gridDim.x * 256 * U) {
+        R d[U], u[U], v[U], w[U];
+#pragma unroll
+        for (int e = 0; e < U; ++e) {
+            const size_t q = min(q0 + 256 * e, (size_t)N - 1);
+            d[e] = F.aux[q]; u[e] = F.u[q]; v[e] = F.v[q]; w[e] = F.w[q];
+        }
+#pragma unroll
+        for (int e = 0; e < U; ++e) {
+            if (q0 + 256 * e >= N) continue;
+            const double a = fabs((double)d[e]);
+            s += a;
+            if (a > m) m = a;
+            if (u[e] != u[e] || v[e] != v[e] || w[e] != w[e]) nan = 1;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o, 64);
+        m = fmax(m, __shfl_xor(m, o, 64));
+        nan |= __shfl_xor(nan, o, 64);
+    }
+    if (lane == 0) { rs[wv] = s; rm[wv] = m; rn[wv] = nan; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double *o = part + 3 * (size_t)blockIdx.x;
+        o[0] = (rs[0] + rs[1]) + (rs[2] + rs[3]);
+        o[1] = fmax(fmax(rm[0], rm[1]), fmax(rm[2], rm[3]));
+        o[2] = (double)(rn[0] | rn[1] | rn[2] | rn[3]);
+    }
+}
+
+// state and rec as k_div_final's
+__global__ __launch_bounds__(256) void k_div_max_final(const double *part, int nblk, double np, double *state,
+                                                       double *rec, int fin)
+{
+    __shared__ double rs[4], rm[4];
+    __shared__ int rn[4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    double s = 0.0, m = -HUGE_VAL;
+    int nan = 0;
+    for (int b = threadIdx.x; b < nblk; b += 256) {
+        s += part[3 * (size_t)b];
+        m = fmax(m, part[3 * (size_t)b + 1]);
+        nan |= part[3 * (size_t)b + 2] != 0.0;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o, 64);
+        m = fmax(m, __shfl_xor(m, o, 64));
+        nan |= __shfl_xor(nan, o, 64);
+    }
+    if (lane == 0) { rs[wv] = s; rm[wv] = m; rn[wv] = nan; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        nan = rn[0] | rn[1] | rn[2] | rn[3];
+        m = fmax(fmax(rm[0], rm[1]), fmax(rm[2], rm[3]));
+        const double hist = state[0], h = fin && !nan && m > hist ? m : hist;
+        rec[0] = ((rs[0] + rs[1]) + (rs[2] + rs[3])) / np;
+        rec[1] = !nan && m > 0.0 ? m : 0.0;
+        rec[2] = h;
+        rec[3] = nan;
+        state[0] = h;
+    }
+}
+
 __global__ void k_scr_set(double *f, double v)
 {
     if (threadIdx.x == 0) f[0] = v;
@@ -354,6 +436,17 @@ void launch_screen(hc_ctx *c, const StepArgsT<R> &F, const StepArgs &D, const Sc
                        B.state, B.rec, fin);
 }
 
+// the spectral path: three values per block, fewer than a unit's summary each
+template <class R>
+void launch_screen_max(hc_ctx *c, const StepArgsT<R> &F, const ScreenBufs &B, int fin)
+{
+    const unsigned N = (unsigned)c->nx * (unsigned)c->ny * (unsigned)c->nz;
+    const int nblk = (int)std::min((N + 1023) / 1024, (unsigned)kMaxBlocks);
+    hipLaunchKernelGGL((k_div_max<R>), dim3(nblk), dim3(256), 0, c->stream, F, N, B.units);
+    hipLaunchKernelGGL(k_div_max_final, dim3(1), dim3(256), 0, c->stream, B.units, nblk,
+                       (double)c->nx * c->ny * c->nz, B.state, B.rec, fin);
+}
+
 // Queue a screen of the context's current fields with the partials in B.
 int queue_screen(hc_ctx *c, const ScreenBufs &B, int fin)
 {
@@ -365,12 +458,12 @@ int queue_screen(hc_ctx *c, const ScreenBufs &B, int fin)
         F.aux = c->m32.ptmp;
         if (c->prm.cds == 1) launch_screen<1, float>(c, F, A, B, fin);
         else if (c->prm.cds == 2) launch_screen<2, float>(c, F, A, B, fin);
-        else launch_screen<3, float>(c, F, A, B, fin);
+        else launch_screen_max<float>(c, F, B, fin);
     } else {
         A.aux = c->ptmp;
         if (c->prm.cds == 1) launch_screen<1, double>(c, A, A, B, fin);
         else if (c->prm.cds == 2) launch_screen<2, double>(c, A, A, B, fin);
-        else launch_screen<3, double>(c, A, A, B, fin);
+        else launch_screen_max<double>(c, A, B, fin);
     }
     HIPCHK(hipGetLastError());
     return 0;

@@ -148,3 +148,97 @@ def test_scan_equals_the_point_by_point_rule(kind, shape):
         assert ch.L.hc_screen_div_error_noalloc(ch.h, fin, C.byref(a1), C.byref(m1), C.byref(h2)) == 0
         assert m1.value == mx and h2.value == hist
     ch.close()
+
+
+def _spectral_divergence(ch):
+    """get_div_spec in numpy: Fourier derivatives without the Nyquist
+    wavenumber, (w(k) - w(k-1)) / dz(k) in z."""
+    p = ch.prm
+    u, v, w = (ch.get_field(k).astype(np.float64) for k in ("u", "v", "w"))
+    kx = 2 * np.pi / p.lx * np.arange(p.nx // 2 + 1)
+    ky = 2 * np.pi / p.ly * np.fft.fftfreq(p.ny, 1.0 / p.ny)
+    kx[-1] = ky[p.ny // 2] = 0.0
+    dudx = np.fft.irfft(1j * kx * np.fft.rfft(u, axis=2), n=p.nx, axis=2)
+    dvdy = np.fft.ifft(1j * ky[:, None] * np.fft.fft(v, axis=1), axis=1).real
+    return dudx + dvdy + (w - np.concatenate([np.zeros_like(w[:1]), w[:-1]], 0)) / ch.mesh()[1][:, None, None]
+
+
+@pytest.mark.parametrize("shape", [(16, 16, 3), (48, 16, 20), (64, 32, 33), (96, 96, 49)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_spectral_screen_is_the_plain_maximum(shape, precision):
+    """cds = 3: |d| is stored (src/module_spectral.f90:931-946), so the states
+    are plain maxima; sizes of less than a block, of a ragged last one and of
+    several points per thread.  FP64 to the rounding of the transforms, FP32
+    spectra to 2^-24 times their ten levels of butterflies."""
+    nx, ny, nz = shape
+    prm = cases.closed_channel(nx=nx, ny=ny, nz=nz, cds=3, issk=1, precision=precision)
+    st = random_state(prm, 3 + nx)
+    ch = Channel(prm)
+    for k, v in st.items():
+        ch.set_field(k, v)
+    ch.init()
+    st = {k: ch.get_field(k) for k in ("u", "v", "w")}
+    d = np.abs(_spectral_divergence(ch))
+    tol = 1e-5 if precision else 1e-12
+    hist = 0.0
+    for scale, fin in ((1.0, 1), (-0.5, 1), (4.0, 0), (2.0, 1)):
+        for k, v in st.items():
+            ch.set_field(k, scale * v)
+        m = abs(scale) * d.max()
+        hist = max(hist, m) if fin else hist
+        got = ch.screen_div_error_ref(fin)
+        assert got[0] == pytest.approx(abs(scale) * d.mean(), rel=tol)
+        assert got[1] == pytest.approx(m, rel=tol) and got[2] == pytest.approx(hist, rel=tol)
+    bad = st["v"].copy()
+    bad[-1, -1, -1] = np.nan
+    ch.set_field("v", bad)
+    with pytest.raises(HerculesError) as ei:
+        ch.screen_div_error_ref(1)
+    assert ei.value.code == 4
+    ch.close()
+
+
+@pytest.mark.parametrize("cds", [1, 2])
+def test_screen_of_fp32_fields_equals_fp64_fields_of_the_same_values(cds):
+    """The mixed variant forms the divergence of its FP32 fields in FP64."""
+    out = []
+    for precision in (0, 1):
+        prm = cases.closed_channel(nx=48, ny=32, nz=33, cds=cds, precision=precision)
+        st = random_state(prm, 5)
+        ch = Channel(prm)
+        for k, v in st.items():
+            ch.set_field(k, v.astype(np.float32).astype(np.float64))
+        out.append([ch.screen_div_error_ref(f) for f in (1, 0)])
+        ch.close()
+    for a, b in zip(*out):
+        assert a[0] == pytest.approx(b[0], rel=1e-12) and a[1:] == b[1:]
+
+
+def test_units_of_several_batches_equal_units_of_one():
+    """256x256x257: the allocation-free entry forms units of two batches, the
+    other of one; a rising start (units with more records than are kept, walked
+    point by point) and random signs after it."""
+    import ctypes as C
+    prm = cases.closed_channel(nx=256, ny=256, nz=257)
+    ch = Channel(prm)
+    rng = np.random.default_rng(1)
+    d = rng.standard_normal(prm.nx * prm.ny * prm.nz)
+    d[:20000] = np.arange(1, 20001) / 10000.0
+    d[30000:40000] = -np.arange(1, 10001) / 3000.0
+    dz = ch.mesh()[1]
+    w = np.cumsum(d.reshape(prm.nz, prm.ny, prm.nx) * dz[:, None, None], axis=0)
+    ch.set_field("w", w)
+    h = C.c_double(0.0)
+    for fin in (1, 0, 1):
+        avg, mx, hist = ch.screen_div_error_ref(fin)
+        a, m = C.c_double(), C.c_double()
+        assert ch.L.hc_screen_div_error_noalloc(ch.h, fin, C.byref(a), C.byref(m), C.byref(h)) == 0
+        assert m.value == mx and h.value == hist
+        assert a.value == pytest.approx(avg, rel=1e-12)
+    d = ((w - np.concatenate([np.zeros_like(w[:1]), w[:-1]], 0)) / dz[:, None, None]).reshape(-1)
+    ref = 0.0
+    for x in d.tolist():
+        if abs(x) > ref:
+            ref = x
+    assert mx == ref
+    ch.close()
