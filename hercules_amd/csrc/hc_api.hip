@@ -762,8 +762,8 @@ extern "C" int hc_create(const hc_params *prm, hc_ctx **out)
     {
         // allow the multi-field column tiles (up to kColLds of dynamic LDS)
         hipError_t ae = hipSuccess;
-        if (ae == hipSuccess) ae = columns_set_lds(L, (int)kColLds);
-        if (ae == hipSuccess) ae = spec_set_lds(L, (int)kColLds);
+        if (ae == hipSuccess) ae = columns_set_lds(L, P.precision == HC_MIXED, (int)kColLds);
+        if (ae == hipSuccess) ae = spec_set_lds(L, P.precision == HC_MIXED, (int)kColLds);
         if (ae == hipSuccess && P.zorder != 2) ae = z6_set_lds(L, (int)kColLds);
         c->big_lds = ae == hipSuccess;
         (void)hipGetLastError();

@@ -278,6 +278,13 @@ __global__ __launch_bounds__(64 * kColWaves) void k_column_t(StepArgs A, ColIO<R
     col_store<L>(io.s0, tile, A.nz, plane, col0, m, d[0]);
 }
 
+// How the two kernels below spread a column of FP64 spectra.  Beyond 896 levels
+// both keep a, b, c and two vectors of 16 levels per lane in scratch, and lanes
+// that share the levels evenly touch less of it than parts of 16 (900 levels,
+// 128x128: pressure solve 469 against 500 us, projection 4.51 against 4.60 ms).
+template <int L, class RIO>
+constexpr bool solve_by_parts() { return sizeof(RIO) == 8 && L < 16; }
+
 // Projection of (u, v, w) spectra in s0, s1, s2 onto discretely
 // divergence-free fields with the pressure operator at rk_c = 1:
 // phi = L^{-1} div u, u -= G phi (the operators of get_p_eqn_src,
@@ -292,7 +299,7 @@ __global__ __launch_bounds__(64 * kColWaves) void k_column_project(StepArgs A, C
     const ColPos pos = col_pos(io, A.ny);
     if (pos.skip) return;
     const int l = pos.bx * kColWaves + (threadIdx.x >> 6), jm = pos.jm;
-    const auto m = col_map<L, sizeof(RIO) == 8>(A.nz);
+    const auto m = col_map<L, solve_by_parts<L, RIO>()>(A.nz);
     const bool is00 = (l == 0 && jm == 0);
     const size_t plane = (size_t)A.ny * A.nl, col0 = (size_t)jm * A.nl + (size_t)pos.bx * kColWaves;
     CC u[1][L], v[1][L], w[1][L], ph[1][L];
@@ -325,7 +332,7 @@ __global__ __launch_bounds__(64 * kColWaves) void k_column_solve(StepArgs A, Col
     const ColPos pos = col_pos(io, A.ny);
     if (pos.skip) return;
     const int l = pos.bx * kColWaves + (threadIdx.x >> 6), jm = pos.jm;
-    const auto m = col_map<L, sizeof(RIO) == 8>(A.nz);
+    const auto m = col_map<L, solve_by_parts<L, RIO>()>(A.nz);
     const bool is00 = (l == 0 && jm == 0);
     const size_t plane = (size_t)A.ny * A.nl, col0 = (size_t)jm * A.nl + (size_t)pos.bx * kColWaves;
     cplx<RC> d[1][L];
@@ -398,12 +405,12 @@ int launch_columns(hc_ctx *c, int kind, StepArgs A, const View<R> &V, int nfield
             io.sel = 1;
             const dim3 glo(c->lo_l, 2 * c->lo_m + 1);
 #define HC_CK(L_) col_kernel<L_, float, double>(kind, glo, lds, c->stream, A, io, eq);
-            HC_DISPATCH_L(c->Lcol, HC_CK)
+            HC_DISPATCH_L_MIXED(c->Lcol, HC_CK)
 #undef HC_CK
         }
         io.sel = c->lo_l > 0 ? 2 : 0;
 #define HC_CK(L_) col_kernel<L_, float, float>(kind, gfull, lds, c->stream, A, io, eq);
-        HC_DISPATCH_L(c->Lcol, HC_CK)
+        HC_DISPATCH_L_MIXED(c->Lcol, HC_CK)
 #undef HC_CK
     }
     return 0;
@@ -412,26 +419,28 @@ int launch_columns(hc_ctx *c, int kind, StepArgs A, const View<R> &V, int nfield
 template int launch_columns<double>(hc_ctx *, int, StepArgs, const View<double> &, int, int);
 template int launch_columns<float>(hc_ctx *, int, StepArgs, const View<float> &, int, int);
 
-hipError_t columns_set_lds(int L, int bytes)
+hipError_t columns_set_lds(int L, bool mixed, int bytes)
 {
     hipError_t e = hipSuccess;
 #define HC_A1(K_)                                                                                                   \
     if (e == hipSuccess)                                                                                            \
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(&K_), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-#define HC_A(L_)                            \
-    HC_A1((k_column_mom<L_>))               \
-    HC_A1((k_column_mom_mixed<L_, float>))  \
-    HC_A1((k_column_mom_mixed<L_, double>))
+#define HC_A(L_) HC_A1((k_column_mom<L_>))
+#define HC_AM(L_) HC_A1((k_column_mom_mixed<L_, float>)) HC_A1((k_column_mom_mixed<L_, double>))
     switch (L) {
-    case 2: HC_A(2) break;
-    case 3: HC_A(3) break;
-    case 4: HC_A(4) break;
-    case 5: HC_A(5) break;
-    case 7: HC_A(7) break;
-    case 8: HC_A(8) break;
-    case 16: HC_A(16) break;
+    HC_CASES_L(HC_A)
+    case 7: HC_A(7); break;
+    case 10: HC_A(10); break;
+    case 12: HC_A(12); break;
+    case 14: HC_A(14); break;
     default: return hipErrorInvalidValue;
     }
+    if (mixed)
+        switch (L) {
+        HC_CASES_L(HC_AM)
+        default: return hipErrorInvalidValue;
+        }
+#undef HC_AM
 #undef HC_A
 #undef HC_A1
     return e;

@@ -194,17 +194,22 @@ inline int rhs_tile_rows(int nx)
     return nx == 16 ? 16 : nx == 32 ? 32 : nx == 48 ? 16 : nx == 64 ? 16 : nx == 96 ? 8 : nx == 128 ? 8 : nx <= 256 ? 4 : 1;
 }
 
-// levels per lane of the column kernels (7 for FP64 spectra only)
+// levels per lane of the column kernels: the smallest of those they are built
+// for that holds nz.  FP64 spectra fill lane after lane with L levels, so too
+// large an L leaves lanes idle and the others with more in scratch (128x128x600
+// at 16 levels, 38 lanes, against 10: pressure solve 349 -> 178 us, FD step 5.02
+// -> 3.32 ms; 128x128x840 at 16 against 14: 443 -> 353 us); FP32 spectra spread
+// the levels over all lanes and keep their coarser steps.
+constexpr int kColL[] = {2, 3, 4, 5, 7, 8, 10, 12, 14, 16}, kColLMixed[] = {2, 3, 4, 5, 8, 16};
 inline int col_levels(int nz, bool mixed)
 {
-    int L = (nz + 63) / 64;
-    if (L <= 2) return 2;
-    if (L <= 3) return 3;
-    if (L <= 4) return 4;
-    if (L <= 5) return 5;
-    if (L <= 7 && !mixed) return 7;
-    if (L <= 8) return 8;
-    if (L <= 16) return 16;
+    if (mixed) {
+        for (int L : kColLMixed)
+            if (nz <= 64 * L) return L;
+    } else {
+        for (int L : kColL)
+            if (nz <= 64 * L) return L;
+    }
     return -1;
 }
 
@@ -290,15 +295,26 @@ inline StepArgsT<double> rows_args<double>(const StepArgs &A, const View<double>
     case 512: MACRO(512); break;                                                          \
     default: return set_err(HC_ERR_UNSUPPORTED, "unsupported transform length %d", n);   \
     }
-#define HC_DISPATCH_L(L_, MACRO)                                                         \
-    switch (L_) {                                                                         \
+// kColL and kColLMixed
+#define HC_CASES_L(MACRO)                                                                 \
     case 2: MACRO(2); break;                                                              \
     case 3: MACRO(3); break;                                                              \
     case 4: MACRO(4); break;                                                              \
     case 5: MACRO(5); break;                                                              \
-    case 7: MACRO(7); break;                                                              \
     case 8: MACRO(8); break;                                                              \
-    case 16: MACRO(16); break;                                                            \
+    case 16: MACRO(16); break;
+#define HC_DISPATCH_L(L_, MACRO)                                                         \
+    switch (L_) {                                                                         \
+    HC_CASES_L(MACRO)                                                                     \
+    case 7: MACRO(7); break;                                                              \
+    case 10: MACRO(10); break;                                                            \
+    case 12: MACRO(12); break;                                                            \
+    case 14: MACRO(14); break;                                                            \
+    default: return set_err(HC_ERR_UNSUPPORTED, "unsupported nz");                       \
+    }
+#define HC_DISPATCH_L_MIXED(L_, MACRO)                                                   \
+    switch (L_) {                                                                         \
+    HC_CASES_L(MACRO)                                                                     \
     default: return set_err(HC_ERR_UNSUPPORTED, "unsupported nz");                       \
     }
 
@@ -344,7 +360,7 @@ template <class R> int mean_interp(hc_ctx *c, StepArgsT<R> &B);
 // Column passes over the spectra s[0..3] of V (hc_columns.hip): kind 0
 // k_column_mom, 1 k_column_t, 2 k_column_project, 3 k_column_solve (eq).
 template <class R> int launch_columns(hc_ctx *c, int kind, StepArgs A, const View<R> &V, int nfields, int eq = 0);
-hipError_t columns_set_lds(int L, int bytes);
+hipError_t columns_set_lds(int L, bool mixed, int bytes);
 
 // Spectral path (hc_spec.hip, hc_spec_col.hip)
 int spec_init(hc_ctx *c);
@@ -360,7 +376,7 @@ int spec_divergence(hc_ctx *c);
 int spec_products(hc_ctx *c, const StepArgs &A, int which);
 int spec_forward64(hc_ctx *c, const double *phys, double2 *spec);
 int spec_damp_one(hc_ctx *c, double2 *f);
-hipError_t spec_set_lds(int L, int bytes);
+hipError_t spec_set_lds(int L, bool mixed, int bytes);
 
 // 6th- and 4th-order z operators (hc_z6.hip): the interpolant pre-pass of
 // the right-hand side, and the column passes (kind as in launch_columns /

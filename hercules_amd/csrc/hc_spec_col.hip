@@ -40,12 +40,12 @@ int launch_spec_columns(hc_ctx *c, int kind, StepArgs A, const View<R> &V)
             io.sel = 1;
             const dim3 glo(c->lo_l, 2 * c->lo_m + 1);
 #define HC_CK(L_) spec_col_kernel<L_, float, double>(kind, glo, lds, c->stream, A, io);
-            HC_DISPATCH_L(c->Lcol, HC_CK)
+            HC_DISPATCH_L_MIXED(c->Lcol, HC_CK)
 #undef HC_CK
         }
         io.sel = c->lo_l > 0 ? 2 : 0;
 #define HC_CK(L_) spec_col_kernel<L_, float, float>(kind, gfull, lds, c->stream, A, io);
-        HC_DISPATCH_L(c->Lcol, HC_CK)
+        HC_DISPATCH_L_MIXED(c->Lcol, HC_CK)
 #undef HC_CK
     }
     return 0;
@@ -54,26 +54,28 @@ int launch_spec_columns(hc_ctx *c, int kind, StepArgs A, const View<R> &V)
 template int launch_spec_columns<double>(hc_ctx *, int, StepArgs, const View<double> &);
 template int launch_spec_columns<float>(hc_ctx *, int, StepArgs, const View<float> &);
 
-hipError_t spec_set_lds(int L, int bytes)
+hipError_t spec_set_lds(int L, bool mixed, int bytes)
 {
     hipError_t e = hipSuccess;
 #define HC_A1(K_)                                                                                                   \
     if (e == hipSuccess)                                                                                            \
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(&K_), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-#define HC_A(L_)                                \
-    HC_A1((k_column_spec<L_, double, double>))  \
-    HC_A1((k_column_spec<L_, float, float>))    \
-    HC_A1((k_column_spec<L_, float, double>))
+#define HC_A(L_) HC_A1((k_column_spec<L_, double, double>))
+#define HC_AM(L_) HC_A1((k_column_spec<L_, float, float>)) HC_A1((k_column_spec<L_, float, double>))
     switch (L) {
-    case 2: HC_A(2) break;
-    case 3: HC_A(3) break;
-    case 4: HC_A(4) break;
-    case 5: HC_A(5) break;
-    case 7: HC_A(7) break;
-    case 8: HC_A(8) break;
-    case 16: HC_A(16) break;
+    HC_CASES_L(HC_A)
+    case 7: HC_A(7); break;
+    case 10: HC_A(10); break;
+    case 12: HC_A(12); break;
+    case 14: HC_A(14); break;
     default: return hipErrorInvalidValue;
     }
+    if (mixed)
+        switch (L) {
+        HC_CASES_L(HC_AM)
+        default: return hipErrorInvalidValue;
+        }
+#undef HC_AM
 #undef HC_A
 #undef HC_A1
     return e;

@@ -246,3 +246,35 @@ def test_gradient_matches_torch_autograd_reference(kind, kw):
         print(f"   d loss / d {k}: rel L2 {err:.2e}")
         assert err < 1e-9, (k, err)
     ch.close()
+
+
+@pytest.mark.parametrize("nz", [129, 193, 257, 321, 448, 449, 513, 641, 769, 897])
+def test_tall_columns_adjoint_is_the_transposed_jacobian(nz):
+    """k_adj_column at every number of levels per lane.  The central difference
+    carries the forward substep's rounding of p over eps, round-off times the
+    condition of its (0,0) Neumann system."""
+    prm = _params("closed", nx=16, ny=16, nz=nz, wall_rows=1, zstretch=0.5, dt=2e-4)
+    x = _state(prm, seed=3)
+    rng = np.random.default_rng(nz)
+    shape = (prm.nz, prm.ny, prm.nx)
+    ch = Channel(prm)
+    d = {k: rng.standard_normal(shape) for k in OUT}
+    lam = {k: rng.standard_normal(shape) for k in OUT}
+    d["w"][-1] = 0.0
+    lam["w"][-1] = 0.0
+    eps = 1e-4
+    outs = []
+    for sgn in (1.0, -1.0):
+        _set(ch, {k: x[k] + sgn * eps * d[k] for k in OUT})
+        ch.substep(2)
+        outs.append({k: ch.get_field(k) for k in OUT})
+    fd = sum(float(np.vdot(outs[0][k] - outs[1][k], lam[k])) for k in OUT) / (2 * eps)
+    _set(ch, x)
+    for k in OUT:
+        ch.set_adjoint(k, lam[k])
+    ch.adjoint_substep(2)
+    ad = sum(float(np.vdot(d[k], ch.get_adjoint(k))) for k in OUT)
+    kappa = 4.0 / ch.mesh()[1].min() ** 2 / (np.pi / prm.lz) ** 2
+    print(f"nz {nz}: fd {fd:.12e} adjoint {ad:.12e} rel {abs(fd - ad) / abs(ad):.2e}")
+    assert abs(fd - ad) <= max(1e-9, 10 * 2.3e-16 / eps * kappa) * abs(ad)
+    ch.close()

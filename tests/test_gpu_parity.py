@@ -271,3 +271,77 @@ def test_column_levels_match_oracle(nz, kw):
         print(f"nz {nz} {kw} {n}: rel L2 {err:.3e}")
         assert err < max(1e-10, 10 * 2.3e-16 * kappa if n == "p" else 0.0), (n, err)
     ch.close()
+
+
+def _kappa(ch):
+    """condition of the (0,0) Neumann system: 4/dz_min^2 over (pi/lz)^2"""
+    return 4.0 / ch.mesh()[1].min() ** 2 / (np.pi / ch.prm.lz) ** 2
+
+
+# the first or last number of levels of every count per lane from 7 on
+TALL = [321, 448, 449, 512, 513, 640, 641, 768, 769, 896, 897, 1024]
+
+
+@pytest.mark.parametrize("nz", TALL)
+@pytest.mark.parametrize("eq", ["u", "w", "p", "t"])
+def test_tall_columns_solve_matches_oracle(nz, eq):
+    """k_column_solve; tolerances as for the shapes above, p to round-off times
+    the condition beyond that."""
+    prm = cases.closed_channel(nx=16, ny=16, nz=nz, wall_rows=1)
+    src = np.random.default_rng(nz).standard_normal((nz, 16, 16))
+    if eq == "p":
+        src -= src.mean(axis=(1, 2), keepdims=True)
+    ref = make_oracle(prm, {}).solve(eq, 8.0 / 15.0, src)
+    with Channel(prm) as ch:
+        got = ch.poisson_solver_fft(eq, 8.0 / 15.0, src)
+        kappa = _kappa(ch)
+    err = rel_l2(got, ref)
+    print(f"solve {eq} nz {nz}: rel L2 {err:.3e}")
+    if eq == "p":
+        assert err < max(1e-9, 10 * 2.3e-16 * kappa)
+        assert poisson_residual(prm, 8.0 / 15.0, got, src) < 1e-14
+    else:
+        assert err < 1e-13
+
+
+@pytest.mark.parametrize("nz", TALL)
+def test_tall_columns_project(nz):
+    """k_column_project: the divergence left is the pressure solve's residual,
+    below 1e-14 of |L| |phi| + |div| as in the solves above, and the second
+    projection removes no more than such a divergence holds (a field of
+    divergence r differs from its projection by at most lz/pi |r|)."""
+    prm, st = small_case("closed", nx=16, ny=16, nz=nz, wall_rows=1)
+    d0, _ = divergence(st["u"], st["v"], st["w"], prm)
+    with Channel(prm) as ch:
+        for k in ("u", "v", "w"):
+            ch.set_field(k, st[k])
+        phi = ch.poisson_solver_fft("p", 1.0, d0)
+        ch.project()
+        once = [ch.get_field(k) for k in ("u", "v", "w")]
+        ch.project()
+        twice = [ch.get_field(k) for k in ("u", "v", "w")]
+        lnorm = 4.0 / ch.mesh()[1].min() ** 2 + 6.0 * (prm.nx / prm.lx) ** 2 + 6.0 * (prm.ny / prm.ly) ** 2
+    d = divergence(*once, prm)[0]
+    scale = lnorm * np.abs(phi).max() + np.abs(d0).max()
+    print(f"project nz {nz}: {np.abs(d).max() / scale:.3e}")
+    assert np.abs(d).max() < 1e-14 * scale
+    bound = prm.lz / np.pi * 1e-14 * scale
+    assert bound < 1e-3 * max(np.abs(a).max() for a in once)  # the check has a meaning
+    for a, b in zip(once, twice):
+        assert np.abs(b - a).max() < bound
+
+
+@pytest.mark.parametrize("nz", [513, 640, 641, 768, 769, 896, 897])
+def test_tall_columns_steps_match_oracle(nz):
+    """k_column_mom and k_column_t; p is left to the solves above (its error is
+    the condition's, and three substeps add theirs)."""
+    prm, st = small_case("open_t", nx=16, ny=16, nz=nz, wall_rows=1, dt=2e-4)
+    o = make_oracle(prm, st)
+    ch = _channel(prm, st)
+    o.steps(1)
+    ch.steps(1)
+    for n in ["u", "v", "w", "t"]:
+        err = rel_l2(ch.get_field(n), o.get(n))
+        print(f"nz {nz} {n}: rel L2 {err:.3e}")
+        assert err < 1e-10, (n, err)
+    ch.close()

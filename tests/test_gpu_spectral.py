@@ -104,3 +104,19 @@ def test_spectral_damping_matches_oracle(kind, kw):
         print(f"spectral damped {kind} {n}: rel L2 {err:.3e}")
         assert err < 1e-10, (n, err)
     ch.close()
+
+
+@pytest.mark.parametrize("nz", [193, 320, 321, 448, 449, 513, 640, 641, 769, 896, 897, 1024])
+def test_spectral_tall_columns_match_oracle(nz):
+    """k_column_spec and k_column_spec_t at the ends of the numbers of levels
+    per lane (p, whose error is the condition of its (0,0) system, is left to
+    the solves)."""
+    prm, st = small_case("open_t", nx=16, ny=16, nz=nz, cds=3, issk=1, wall_rows=1, dt=2e-4)
+    o, ch = _pair(prm, st)
+    o.steps(1)
+    ch.steps(1)
+    for n in ("u", "v", "w", "t"):
+        err = rel_l2(ch.get_field(n), o.get(n))
+        print(f"spectral nz {nz} {n}: rel L2 {err:.3e}")
+        assert err < 1e-10, (n, err)
+    ch.close()
