@@ -6,8 +6,10 @@
 // Columns per block of k_column_mom: four, so that two blocks share a CU (a
 // block's loads and stores then overlap the other's solves); the two halves
 // of a 128-byte line belong to neighbouring blocks of one XCD.  Two beyond
-// 512 levels, whose tiles would not fit.
+// 512 levels, whose tiles would not fit, and from 342 levels on where the
+// runtime has refused more than 64 KB of dynamic LDS.
 template <int L> constexpr int mom_waves() { return L > 8 ? 2 : 4; }
+constexpr size_t kLdsDefault = 64 * 1024;  // dynamic LDS of any kernel
 
 // One fused column pass of the substep: Helmholtz solves of u*, v*, w*, the
 // divergence source, the pressure Poisson solve, the projection and the
@@ -20,12 +22,12 @@ template <int L> constexpr int mom_waves() { return L > 8 ? 2 : 4; }
 // 256x256x257 FP64 (0.94 GB, 2.8 TB/s; with every field in registers, 247
 // VGPRs and one block of eight columns per CU, 473 us),
 // 47 us at 128x128x129 (91), 3.0 ms at 512x512x385 (6.2, spilling).
-template <int L>
-__global__ __launch_bounds__(64 * mom_waves<L>(), 2) void k_column_mom(StepArgs A, ColIO<double> io)
+template <int L, int W = mom_waves<L>()>
+__global__ __launch_bounds__(64 * W, 2) void k_column_mom(StepArgs A, ColIO<double> io)
 {
     using RC = double;
     using CC = double2;
-    constexpr int W = mom_waves<L>(), T = 64 * W;
+    constexpr int T = 64 * W;
     extern __shared__ double2 tile_raw[];
     CC *tile = tile_raw;
     const ColPos pos = col_pos<W>(io, A.ny);
@@ -354,10 +356,23 @@ __global__ __launch_bounds__(64 * kColWaves) void k_column_solve(StepArgs A, Col
     col_store<L>(io.s0, tile, A.nz, plane, col0, m, d[0]);
 }
 
+// k_column_mom with W columns per block in at most lim bytes of LDS: the fourth
+// tile unless it does not fit or more blocks share a CU with three (the
+// registers hold four blocks up to 3 levels per lane, three up to 5)
+template <int L, int W>
+static void mom_kernel(dim3 g, size_t lim, hipStream_t st, const StepArgs &A, const ColIO<double> &io)
+{
+    const size_t one = col_sub<W>(A.nz) * sizeof(double2), regs = L <= 3 ? 4 : L <= 5 ? 3 : 2;
+    StepArgs M = A;
+    M.ntile = 4 * one > lim || std::min(regs, kColLds / (3 * one)) > std::min(regs, kColLds / (4 * one)) ? 3 : 4;
+    hipLaunchKernelGGL((k_column_mom<L, W>), dim3(g.x * (kColWaves / W), g.y), dim3(64 * W), M.ntile * one, st, M, io);
+}
+
 // Column kernels: kind 0 k_column_mom, 1 k_column_t, 2 k_column_project,
 // 3 k_column_solve (equation eq).
 template <int L, class RIO, class RC>
-static void col_kernel(int kind, dim3 g, size_t lds, hipStream_t st, const StepArgs &A, const ColIO<RIO> &io, int eq)
+static void col_kernel(int kind, dim3 g, size_t lds, bool big, hipStream_t st, const StepArgs &A, const ColIO<RIO> &io,
+                       int eq)
 {
     const dim3 b(64 * kColWaves);
     switch (kind) {
@@ -365,13 +380,14 @@ static void col_kernel(int kind, dim3 g, size_t lds, hipStream_t st, const StepA
         if constexpr (sizeof(RIO) == 4) {
             hipLaunchKernelGGL((k_column_mom_mixed<L, RC>), g, b, lds, st, A, io);
         } else {
-            // the fourth tile unless more blocks share a CU with three (the
-            // registers hold four blocks up to 3 levels per lane, three up to 5)
             constexpr int W = mom_waves<L>();
-            const size_t one = col_sub<W>(A.nz) * sizeof(double2), regs = L <= 3 ? 4 : L <= 5 ? 3 : 2;
-            StepArgs M = A;
-            M.ntile = std::min(regs, kColLds / (3 * one)) > std::min(regs, kColLds / (4 * one)) ? 3 : 4;
-            hipLaunchKernelGGL((k_column_mom<L>), dim3(g.x * (kColWaves / W), g.y), dim3(64 * W), M.ntile * one, st, M, io);
+            const size_t lim = big ? kColLds : kLdsDefault;
+            if constexpr (L == 7 || L == 8)
+                if (3 * col_sub<W>(A.nz) * sizeof(double2) > lim) {
+                    mom_kernel<L, 2>(g, lim, st, A, io);
+                    break;
+                }
+            mom_kernel<L, W>(g, lim, st, A, io);
         }
         break;
     case 1: hipLaunchKernelGGL((k_column_t<L, RIO, RC>), g, b, lds, st, A, io); break;
@@ -397,19 +413,19 @@ int launch_columns(hc_ctx *c, int kind, StepArgs A, const View<R> &V, int nfield
     const dim3 gfull((c->nl + kColWaves - 1) / kColWaves, c->ny);
     if constexpr (std::is_same<R, double>::value) {
         io.sel = 0;
-#define HC_CK(L_) col_kernel<L_, double, double>(kind, gfull, lds, c->stream, A, io, eq);
+#define HC_CK(L_) col_kernel<L_, double, double>(kind, gfull, lds, c->big_lds, c->stream, A, io, eq);
         HC_DISPATCH_L(c->Lcol, HC_CK)
 #undef HC_CK
     } else {
         if (c->lo_l > 0) {
             io.sel = 1;
             const dim3 glo(c->lo_l, 2 * c->lo_m + 1);
-#define HC_CK(L_) col_kernel<L_, float, double>(kind, glo, lds, c->stream, A, io, eq);
+#define HC_CK(L_) col_kernel<L_, float, double>(kind, glo, lds, c->big_lds, c->stream, A, io, eq);
             HC_DISPATCH_L_MIXED(c->Lcol, HC_CK)
 #undef HC_CK
         }
         io.sel = c->lo_l > 0 ? 2 : 0;
-#define HC_CK(L_) col_kernel<L_, float, float>(kind, gfull, lds, c->stream, A, io, eq);
+#define HC_CK(L_) col_kernel<L_, float, float>(kind, gfull, lds, c->big_lds, c->stream, A, io, eq);
         HC_DISPATCH_L_MIXED(c->Lcol, HC_CK)
 #undef HC_CK
     }
