@@ -1878,7 +1878,8 @@ extern "C" int hc_wall_shear_gradient(hc_ctx *c, int nsteps, int ckpt_every, dou
 // Launch shapes that leave every result bit-identical (each tile, transform
 // row or column is computed the same way whatever the block shape): the RHS
 // tile-order group, the y-transform columns per block, the inverse-x points
-// per block and the column-kernel block order.  Coordinate descent over the
+// per block and the column-kernel block order; and the momentum tile shape,
+// where tiles and whole rows agree to round-off.  Coordinate descent over the
 // knobs, each trial timing whole steps from the same saved state with HIP
 // events; a candidate replaces the current choice when it is more than 1%
 // faster.  The state and step counters are restored afterwards.
@@ -1944,8 +1945,11 @@ extern "C" int hc_autotune(hc_ctx *c, int steps_per_trial)
     };
     // candidates per knob
     const int nty = c->ny / rhs_tile_rows(c->nx);
+    // (the order of tiles only where a kernel reads it: whole rows, the sponge)
+    const int by_size = rhs_shape_by_size(P.nx, c->mixed);
+    const bool hiz = P.zorder == 4 || P.zorder == 6;
     std::vector<int> groups = {0};
-    if (P.nx <= 256)
+    if (P.nx <= 256 && !hiz && (by_size == 0 || P.isdamp == 1))
         for (int g : {1, 2, 4, 8, 16, 32})
             if (nty % g == 0 && g <= nty) groups.push_back(g);
     std::vector<int> ytiles = {0, kYTile};
@@ -1953,7 +1957,7 @@ extern "C" int hc_autotune(hc_ctx *c, int steps_per_trial)
     std::vector<int> xts = {0};
     if (P.zorder == 2)
         for (int sh = 1; sh <= 4; ++sh)
-            if (rhs_xt_fits(sh, c->nx, c->ny)) xts.push_back(sh);
+            if (sh != by_size && rhs_xt_fits(sh, c->nx, c->ny)) xts.push_back(sh);
     int *knob[5] = {&c->tune.rgroup, &c->tune.ytile, &c->tune.c2r_pts, &c->tune.col_remap, &c->tune.rhs_xt};
     std::vector<int> cand[5] = {groups, ytiles, {1024, 512, 2048}, {0, 1}, xts};
     float best = 0.0f;

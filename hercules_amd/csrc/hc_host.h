@@ -318,6 +318,10 @@ inline StepArgsT<double> rows_args<double>(const StepArgs &A, const View<double>
     default: return set_err(HC_ERR_UNSUPPORTED, "unsupported nz");                       \
     }
 
+// Momentum tile shape that the knob's 0 stands for (the measurements are at
+// march_shape): 32x8 for FP64 rows of 96 and more, else whole rows (0)
+inline int rhs_shape_by_size(int nx, bool mixed) { return !mixed && nx >= 96 ? 1 : 0; }
+
 inline int rows_for(int nx) { return nx >= kRowPoints ? 1 : kRowPoints / nx; }
 
 // LDS of the column kernels: `nfields` sub-tiles of nz x kColWaves complex

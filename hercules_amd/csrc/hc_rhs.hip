@@ -440,7 +440,7 @@ template <class R>
 static int march_shape(const hc_ctx *c)
 {
     if (rhs_xt_fits(c->tune.rhs_xt, c->nx, c->ny)) return c->tune.rhs_xt;
-    return sizeof(R) == 8 && c->nx >= 96 ? 1 : 0;
+    return rhs_shape_by_size(c->nx, sizeof(R) == 4);
 }
 // Levels of one block's run.  A run costs two levels' loads more than it
 // forms, so about 12 levels and more; but at least three blocks per CU (what
@@ -649,7 +649,7 @@ int rhs_momentum(hc_ctx *c, const StepArgs &A, StepArgsT<R> &B)
             // out and run past the last one
             if (B.rgroup > 0 && (c->ny / rhs_tile_rows(c->nx)) % B.rgroup) B.rgroup = 0;
 #define HC_RHS(NX_)                                                                                     \
-    if constexpr (NX_ <= 256) {                                                                          \
+    if constexpr (NX_ < 96 || (NX_ <= 256 && sizeof(R) == 4)) {                                          \
         constexpr int TY_ = rhs2_ty<NX_>();                                                              \
         dim3 g1((unsigned)(c->ny / TY_ * ksplit));                                                       \
         constexpr int T_ = rhs2_threads<NX_>();                                                          \

@@ -97,3 +97,15 @@ def test_tile_groups_that_do_not_divide_the_tiles(kw, groups):
         got, _ = _run(prm, st, 1, shape=dict(rgroup=g))
         for k in ref:
             assert np.array_equal(got[k], ref[k]), (kw, g, k)
+
+
+@pytest.mark.parametrize("kw", [dict(nx=96, ny=16, nz=9), dict(nx=128, ny=32, nz=17),
+                                dict(nx=64, ny=16, nz=17, zorder=6), dict(nx=128, ny=16, nz=17, zorder=4, precision=1)])
+def test_tuning_leaves_knobs_that_no_kernel_reads(kw):
+    """Marching tiles and the high-order z kernels have no tile-order group,
+    and the tile shape that 0 stands for is not tried under its own number."""
+    prm, st = small_case("closed", **kw)
+    for _ in range(3):
+        _, chosen = _run(prm, st, 1, tune=True)
+        assert chosen["rgroup"] == 0, chosen
+        assert chosen["rhs_xt"] in ((0,) if kw.get("zorder") else (0, 2, 3, 4)), chosen

@@ -345,3 +345,20 @@ def test_tall_columns_steps_match_oracle(nz):
         print(f"nz {nz} {n}: rel L2 {err:.3e}")
         assert err < 1e-10, (n, err)
     ch.close()
+
+
+@pytest.mark.parametrize("shapes", [dict(), dict(rgroup=1), dict(rgroup=32)])
+def test_whole_rows_over_many_tiles_match_oracle(shapes):
+    """64x512x25: right-hand sides of whole rows fused with the x transform (the
+    FP64 rows that do not march), 32 y tiles per level in every tile order."""
+    prm, st = small_case("closed", nx=64, ny=512, nz=25)
+    o = make_oracle(prm, st)
+    ch = _channel(prm, st)
+    ch.set_tuning(**shapes)
+    o.steps(1)
+    ch.steps(1)
+    for n in ["u", "v", "w", "p"]:
+        err = rel_l2(ch.get_field(n), o.get(n))
+        print(f"{shapes} {n}: rel L2 {err:.3e}")
+        assert err < 1e-10, (n, err)
+    ch.close()
