@@ -31,7 +31,7 @@
 template <class CI>
 struct BandSys {
     const CI *in[2];  // right-hand sides (k, j, l)
-    CI *f[2];         // solutions (may be in[]); hold the eliminated right-hand sides in between
+    CI *f[2];         // solutions (may be in[])
     double *scr;    // segment starts: PI (PI + 1 + 2 nr) doubles per segment and column
     int nr;         // right-hand sides sharing the matrix: 1 or 2
     int eq;         // 0 u/v, 1 w, 2 p, 3 t

@@ -16,7 +16,7 @@ constexpr size_t kLdsDefault = 64 * 1024;  // dynamic LDS of any kernel
 // pressure increment (FP64).  A column lives in its block's LDS tiles (u, v,
 // w; the increment in a fourth if A.ntile says so, else in u's after that is
 // stored) and only the fields being solved for are in registers, which keeps
-// up to 8 levels per lane below the 256 VGPRs of two waves per SIMD (160 VGPRs
+// up to 8 levels per lane below the 256 VGPRs of two waves per SIMD (156 VGPRs
 // at 5 levels: three blocks of four waves).  Bound by HBM and, less, VALU
 // issue (2060 instructions per column at 5 levels): 335 us per substep at
 // 256x256x257 FP64 (0.94 GB, 2.8 TB/s; with every field in registers, 247

@@ -527,8 +527,9 @@ extern "C" int hc_screen_div_error_noalloc(hc_ctx *c, int isfinal, double *div_a
 {
     if (!c || !div_hist_max) return set_err(HC_ERR_ARG, "null argument");
     if (isfinal != 0 && isfinal != 1) return set_err(HC_ERR_ARG, "isfinal must be 0 or 1");
-    // the size of grid that is taken: ny nz rows and 3 values for 16 rows of a
-    // level within the scratch
+    // the grids that are taken: the limit is that of row maxima and block sums
+    // (ny nz rows and 3 values for 16 rows of a level), which the summaries of
+    // units no longer need and which stays so that no answer changes
     const size_t need = 8 + (size_t)c->ny * c->nz + 3 * (size_t)((c->ny + 15) / 16) * c->nz;
     // units of as many batches as make their summaries fit: 1 to 16 (a grid of
     // this size has nx <= 512, so under 2^28 points)
