@@ -331,7 +331,7 @@ __global__ __launch_bounds__(64) void k_div_final(StepArgsT<R> F, StepArgs D, un
 // The largest |d| of the spectral path (screen_div_error_spec stores |d|,
 // src/module_spectral.f90:931-946), whose divergence lies in F.aux: a NaN is
 // never taken.  Bound by HBM: four reads of every point, four points of a
-// thread in flight (256x256x257: 119 us, 4.5 TB/s; a whole screen of that grid
+// thread in flight (256x256x257: 122 us, 4.4 TB/s; a whole screen of that grid
 // 351 us, 501 with the units and records of the signed states, and 71 against
 // 151 at 128x128x129).
 constexpr int kMaxBlocks = 2048;  // eight blocks of four wavefronts per CU
